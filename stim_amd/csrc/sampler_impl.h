@@ -150,7 +150,9 @@ struct mfs_sampler {
     // the launch in progress (set only while a call returns errors).
     DevBuf d_site_mech, d_err, d_err_tmp;
     // Outcome records of the specialised scan kernel (built with the symptom table when it applies).
-    DevBuf d_orecs, d_orec_base, d_orec_sites, d_orec_ovf;
+    DevBuf d_orecs, d_orec_base, d_orec_sites, d_orec_ovf, d_direct;
+    bool sym_direct = false;     // every site has a direct entry
+    uint32_t direct_null = 0;
     uint64_t orec_blocks = 0, orec_records = 0;
     bool sym_fast = false;
     int sym_variant = 0;         // 0: specialised scan kernel where it applies; 1: generic scan kernel
@@ -867,8 +869,10 @@ struct mfs_sampler {
             site0[c] = nsites;
             nsites += plan.classes[c].nsites;
         }
-        if (nsites >= (1ull << 31)) return;
+        if (nsites >= (1ull << 30)) return;
         std::vector<uint2> sites(std::max<uint64_t>(nsites, 1), make_uint2(0, 0));
+        std::vector<uint4> direct(sites.size(), make_uint4(0, 0, 0, 0));
+        bool all_direct = nsites < (1ull << 27);   // 32-bit byte offsets of 16-byte entries
         std::vector<uint2> orec;
         std::vector<uint32_t> oovf;
         std::vector<uint32_t> acc;
@@ -881,6 +885,7 @@ struct mfs_sampler {
             const uint32_t nout = cl.nout & 0xFFFFu;
             site_syms.resize(nout);
             for (uint64_t st = 0; st < cl.nsites; st++) {
+                if (all_direct) all_direct = direct_entry(cl, st, offs, ents, direct[site0[c] + st]);
                 uint32_t lo = D;
                 for (uint32_t code = 1; code <= nout; code++) {
                     acc.clear();
@@ -962,9 +967,42 @@ struct mfs_sampler {
         upload(d_orec_base, base, "outcome record site bases");
         upload(d_orec_sites, sites, "outcome record sites");
         upload(d_orec_ovf, oovf, "outcome record overflow lists");
+        sym_direct = all_direct;
+        if (sym_direct) {
+            direct_null = (uint32_t)direct.size();
+            for (uint32_t l = 0; l < 64; l++) {
+                const uint32_t d = D ? 32 * l % D : 0;
+                direct.push_back(make_uint4(d | (d << 14) | (1u << 28), d | (d << 14), d | (d << 14), 0));
+            }
+            upload(d_direct, direct, "direct site entries");
+        }
         orec_blocks = blocks.size();
         orec_records = orec.size();
         sym_fast = true;
+    }
+
+    // Direct entry of site st of a class (layout in symptom.h); false when its basis columns reach more
+    // detectors than the entry holds.
+    bool direct_entry(const SymClass &cl, uint64_t st, const std::vector<uint32_t> &offs,
+                      const std::vector<uint32_t> &ents, uint4 &out) const {
+        uint32_t d[SYM_DIRECT_DETECTORS] = {}, nd = 0, w = 0;
+        for (uint32_t j = 0; j < cl.basis; j++) {
+            const uint64_t col = cl.col0 + st * cl.basis + j;
+            for (uint32_t t = offs[col]; t < offs[col + 1]; t++) {
+                uint32_t bit;
+                if (ents[t] >= prog.num_detectors) {
+                    bit = SYM_DIRECT_DETECTORS + (ents[t] - prog.num_detectors);
+                } else {
+                    for (bit = 0; bit < nd && d[bit] != ents[t]; bit++) {}
+                    if (bit == SYM_DIRECT_DETECTORS) return false;
+                    if (bit == nd) d[nd++] = ents[t];
+                }
+                w ^= 1u << (8 * j + bit);
+            }
+        }
+        for (uint32_t k = nd; k < SYM_DIRECT_DETECTORS; k++) d[k] = d[0];
+        out = make_uint4(d[0] | (d[1] << 14) | ((cl.nout & 0xFFFFu) << 28), d[2] | (d[3] << 14), d[4] | (d[5] << 14), w);
+        return true;
     }
 
     // Builds the symptom tables of a detector error model (reference DemSampler,
@@ -1174,6 +1212,7 @@ struct mfs_sampler {
         P.orec_base = nullptr;
         P.orec_sites = nullptr;
         P.orec_ovf = nullptr;
+        P.direct = nullptr;
         P.err_words = err_words_cur;
         P.err_stride_words = err_stride_cur;
         P.site_mech = dem_mode ? d_site_mech.as<uint32_t>() : nullptr;
@@ -1241,6 +1280,8 @@ struct mfs_sampler {
             P.orec_base = d_orec_base.as<uint32_t>();
             P.orec_sites = d_orec_sites.as<uint2>();
             P.orec_ovf = d_orec_ovf.as<uint32_t>();
+            P.direct = sym_direct ? d_direct.as<uint4>() : nullptr;
+            P.direct_null = direct_null;
         }
         return r;
     }

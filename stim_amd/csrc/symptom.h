@@ -148,7 +148,15 @@ struct SymDevParams {
     const uint32_t *orec_base;
     const uint2 *orec_sites;
     const uint32_t *orec_ovf;      // overflow lists: count, then entries (detector b + m, observable D + k)
+    // Direct site entries of the specialised scan kernel, indexed as orec_sites (null when some site
+    // reaches more than SYM_DIRECT_DETECTORS detectors: its hits then read orec_sites and orecs).
+    const uint4 *direct;
+    uint32_t direct_null;          // first of 64 null entries (no flips; their fields name words spread over a row)
 };
+// Direct site entry (16 bytes): x = d0 | d1 << 14 | nout << 28, y = d2 | d3 << 14, z = d4 | d5 << 14 with the
+// detectors that the site's basis columns reach (unused fields repeat d0, or are 0), w = byte j: bit e < 6
+// set when basis column j flips detector d_e, bits 6 and 7 when it flips observable 0 and 1.
+constexpr uint32_t SYM_DIRECT_DETECTORS = 6;
 // Outcome record (8 bytes): x = e0 | e1 << 14 | valid << 28, y = e2 | e3 << 14 | obs1 << 28 | obs0 << 29;
 // entries are relative to the site's base detector, valid has bit e set for each of the n = 0..4
 // entries in use (bits 0 .. n - 1), unused entries are 0. A symptom with more than four detectors has

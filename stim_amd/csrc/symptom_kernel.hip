@@ -281,29 +281,47 @@ constexpr uint32_t SCAN_M_MAX = 8;
 // Gaps are clamped at 2^31, above any group's position count N (at most 2^31 - 1), so a clamped gap
 // always passes the end of the group and g + 1 cannot overflow.
 __device__ __forceinline__ uint32_t gap32(uint32_t r, float inv_log2_1mp) {
-    const float u = ((float)(r >> 8) + 1.0f) * (1.0f / 16777216.0f);
-    const float g = __log2f(u) * inv_log2_1mp;
-    return g < 2147483648.0f ? (uint32_t)g : 0x80000000u;
+    // (r >> 8) + 1 is at most 2^24, so the fused form is the exact product ((r >> 8) + 1) * 2^-24.
+    const float u = fmaf((float)(r >> 8), 1.0f / 16777216.0f, 1.0f / 16777216.0f);
+    return (uint32_t)fminf(__log2f(u) * inv_log2_1mp, 2147483648.0f);
 }
 
 __device__ __forceinline__ uint32_t sat_add(uint32_t a, uint32_t b) {
-    const uint32_t c = a + b;
-    return c < a ? 0xFFFFFFFFu : c;
+    return __builtin_elementwise_add_sat(a, b);   // one v_add_u32 with clamp
 }
 
-// Saturating prefix sum over the 256 lanes of the workgroup (saturating addition of non-negative
-// values is associative, so any sum that reaches 2^32 - 1 stays there). Returns (exclusive, total).
+// One step of a wave's prefix sum: adds the value that the DPP control word CTRL moves in (row_shr within 16-lane
+// rows, then row_bcast of a row's last lane into the rows of mask ROWS); lanes that receive nothing add 0.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t scan_step(uint32_t x) {
+    return sat_add(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xF, false));
+}
+
+// Inclusive saturating prefix sum over the wave's 64 lanes (saturating addition of non-negative values is
+// associative, so any sum that reaches 2^32 - 1 stays there): 12 VALU instructions and no LDS round trips, where
+// six shuffles took 24 and waited for LDS six times.
+__device__ __forceinline__ uint32_t wave_inclusive(uint32_t x) {
+    x = scan_step<0x111, 0xF>(x);   // row_shr:1, 2, 4, 8
+    x = scan_step<0x112, 0xF>(x);
+    x = scan_step<0x114, 0xF>(x);
+    x = scan_step<0x118, 0xF>(x);
+    x = scan_step<0x142, 0xA>(x);   // row_bcast:15 into rows 1 and 3
+    return scan_step<0x143, 0xC>(x);   // row_bcast:31 into rows 2 and 3
+}
+
+// The value of the lane before (wave_shr:1); 0 for lane 0.
+__device__ __forceinline__ uint32_t lane_before(uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x138, 0xF, 0xF, false);
+}
+
+// Saturating prefix sum over the 256 lanes of the workgroup. Returns (exclusive, total). scratch: NT / 64 words
+// that no wave still reads from a scan before the last one (callers alternate between two sets, so one barrier
+// per scan is enough).
 __device__ __forceinline__ uint2 block_scan(uint32_t v, uint32_t *scratch) {
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    uint32_t x = v;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t y = __shfl_up(x, d, 64);
-        if (lane >= (uint32_t)d) x = sat_add(x, y);
-    }
-    if (lane == 63) scratch[wave] = x;
-    uint32_t ex = __shfl_up(x, 1, 64);
-    if (lane == 0) ex = 0;
+    const uint32_t wave = threadIdx.x >> 6;
+    const uint32_t x = wave_inclusive(v);
+    if ((threadIdx.x & 63) == 63) scratch[wave] = x;
+    const uint32_t ex = lane_before(x);
     __syncthreads();
     uint32_t before = 0, total = 0;
 #pragma unroll
@@ -312,7 +330,6 @@ __device__ __forceinline__ uint2 block_scan(uint32_t v, uint32_t *scratch) {
         if (w < wave) before = sat_add(before, t);
         total = sat_add(total, t);
     }
-    __syncthreads();
     return make_uint2(sat_add(before, ex), total);
 }
 
@@ -455,17 +472,8 @@ __device__ __forceinline__ void record_error(const SymDevParams &P, uint64_t row
 
 // Saturating prefix sum over the 64 lanes of a wave. Returns (exclusive, total).
 __device__ __forceinline__ uint2 wave_scan(uint32_t v) {
-    const uint32_t lane = threadIdx.x & 63;
-    uint32_t x = v;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t y = __shfl_up(x, d, 64);
-        if (lane >= (uint32_t)d) x = sat_add(x, y);
-    }
-    const uint32_t total = __shfl(x, 63, 64);
-    uint32_t ex = __shfl_up(x, 1, 64);
-    if (lane == 0) ex = 0;
-    return make_uint2(ex, total);
+    const uint32_t x = wave_inclusive(v);
+    return make_uint2(lane_before(x), (uint32_t)__builtin_amdgcn_readlane((int)x, 63));
 }
 
 // Position where draw-space coordinate a falls in a group that starts at draw-space coordinate c and
@@ -608,8 +616,9 @@ __device__ __forceinline__ void scan_tile(const SymDevParams &P, uint32_t btile,
     const uint32_t det_words = (S * P.det_row_bytes + 15) / 16 * 4;
     const uint32_t obs_words = (S * P.obs_row_bytes + 15) / 16 * 4;
     Images im{lds, lds + det_words};
-    uint32_t *const scratch = lds + det_words + obs_words;  // 8 words
+    uint32_t *const scratch = lds + det_words + obs_words;  // 8 words: two sets of NT / 64, by round parity
     uint32_t *const otab_lds = scratch + 8;
+    uint32_t scans = 0;
     const bool otab_in_lds = P.otab_words <= SYM_OTAB_LDS_WORDS;
     const uint32_t *otab = otab_in_lds ? otab_lds : P.otab;
     const uint32_t tid = threadIdx.x;
@@ -658,7 +667,7 @@ __device__ __forceinline__ void scan_tile(const SymDevParams &P, uint32_t btile,
             for (uint32_t k = 0; k < SCAN_M_MAX; k++) {
                 if (k < m) sum = sat_add(sum, g[k] + 1);
             }
-            const uint2 sc = block_scan(sum, scratch);
+            const uint2 sc = block_scan(sum, scratch + 4 * (scans++ & 1));
             // Positions stay at most N < 2^31: the start and every gap are clamped at N.
             uint32_t pos = sat_add(base, sc.x);
             pos = pos < N ? pos : N;
@@ -715,69 +724,179 @@ __device__ __forceinline__ void scan_tile(const SymDevParams &P, uint32_t btile,
                    P.obs.ptr + s0 * P.obs.stride, P.obs.stride);
 }
 
-// Applies up to K hits of one lane (the specialised scan kernel's pass 2 and 3): loads the K hits'
-// site entries together, then their K outcome records together (entries past the round's hits name
-// the group's first site and are skipped), so that the compiler can wait for each load in turn; then
-// flips each hit's detector bits without branching per entry (an absent entry XORs 0 into its word)
-// and its observable flags. site[k] = the hit's site entry index, oc[k] = its outcome draw: the code is
-// mulhi(oc, nout) + 1 with the site's nout from its entry, as the generic kernel computes it.
+// Applies a lane's K hits (the specialised scan kernel's pass 2 and 3) from outcome blocks: loads the hits' site
+// entries together, then their outcome records together, so that the compiler can wait for each load in turn;
+// then flips each hit's detector bits. site[k] = the hit's site entry index, oc[k] = its outcome draw: the code is
+// mulhi(oc, nout) + 1 with the site's nout from its entry, as the generic kernel computes it. A lane without a
+// k-th hit reads the group's first site and XORs 0 into a word of some shot (shot[k]: spread over the lanes, since
+// atomics on one word serialise: all of them on shot 0's words cost 4%); an absent entry XORs 0 too. Nothing
+// branches but the rare hits that flip an observable or more than four detectors, once per K hits.
 template <bool OBS, uint32_t K>
 __device__ __forceinline__ void apply_outcomes(const SymDevParams &P, const Sink &sink, const uint32_t *site,
-                                               const uint32_t *oc, const uint32_t *shot, uint32_t S) {
+                                               const uint32_t *oc, const uint32_t *shot, const bool *hit) {
     uint2 se[K], rec[K];
 #pragma unroll
     for (uint32_t k = 0; k < K; k++) se[k] = P.orec_sites[site[k]];
 #pragma unroll
     for (uint32_t k = 0; k < K; k++) rec[k] = P.orecs[(se[k].x & 0x0FFFFFFFu) + __umulhi(oc[k], se[k].x >> 28)];
+    uint32_t rare = 0;
 #pragma unroll
     for (uint32_t k = 0; k < K; k++) {
-        if (shot[k] < S) {
-            // Shot and row-bit counts fit 24 bits (S <= 8192, rows below 64 KB); the site's base
-            // detector is below D, so every entry's bit lies in the shot's row.
-            const uint32_t dbase = __umul24(shot[k], sink.det_bits) + sink.det_col0 + se[k].y;
-            const uint2 r = rec[k];
-            // An overflow record holds its list offset where entries 2 and 3 would be (and no valid
-            // bits): read those entries, and its observable flags, as 0 so that every address stays
-            // inside the tile's image.
-            const uint32_t ry = (r.y & SYM_OREC_OVERFLOW) ? 0u : r.y;
-            const uint32_t f[4] = {r.x & 0x3FFFu, (r.x >> 14) & 0x3FFFu, ry & 0x3FFFu, (ry >> 14) & 0x3FFFu};
+        // Shot and row-bit counts fit 24 bits (S <= 8192, rows below 64 KB); the site's base detector is
+        // below D, so every entry's bit lies in the shot's row.
+        const uint32_t dbase = __umul24(shot[k], sink.det_bits) + sink.det_col0 + se[k].y;
+        const uint32_t x = hit[k] ? rec[k].x : 0u, y = hit[k] ? rec[k].y : 0u;
+        // An overflow record holds its list offset where entries 2 and 3 would be (and no valid bits): read
+        // those entries as 0 so that every address stays inside the tile's image.
+        const uint32_t ry = (y & SYM_OREC_OVERFLOW) ? 0u : y;
+        lds_xor_bit(dbase + (x & 0x3FFFu), (x >> 28) & 1u);
+        lds_xor_bit(dbase + ((x >> 14) & 0x3FFFu), (x >> 29) & 1u);
+        lds_xor_bit(dbase + (ry & 0x3FFFu), (x >> 30) & 1u);
+        lds_xor_bit(dbase + ((ry >> 14) & 0x3FFFu), x >> 31);
+        rec[k].y = y;
+        rare |= y;
+    }
+    if (rare >> 28) {
 #pragma unroll
-            for (uint32_t e = 0; e < 4; e++) lds_xor_bit(dbase + f[e], (r.x >> (28 + e)) & 1u);
-            if (OBS && ((ry >> 28) & 3u)) {
-                const uint32_t obase = sink.obs_base + __umul24(shot[k], sink.obs_bits) + sink.obs_col0;
-                if ((ry >> 29) & 1u) xor_bit(sink, obase);
-                if ((ry >> 28) & 1u) xor_bit(sink, obase + 1);
-            }
-            if (r.y & SYM_OREC_OVERFLOW) {
-                const uint32_t obase = sink.obs_base + __umul24(shot[k], sink.obs_bits) + sink.obs_col0;
+        for (uint32_t k = 0; k < K; k++) {
+            const uint32_t y = rec[k].y;
+            if (!(y >> 28)) continue;
+            const uint32_t obase = sink.obs_base + __umul24(shot[k], sink.obs_bits) + sink.obs_col0;
+            if (y & SYM_OREC_OVERFLOW) {
                 // More than four detectors: the list (detector m, observable D + k).
-                const uint32_t *list = P.orec_ovf + (r.y & ~SYM_OREC_OVERFLOW);
+                const uint32_t dbase = __umul24(shot[k], sink.det_bits) + sink.det_col0 + se[k].y;
+                const uint32_t *list = P.orec_ovf + (y & ~SYM_OREC_OVERFLOW);
                 const uint32_t cnt = list[0];
                 for (uint32_t e = 0; e < cnt; e++) {
                     const uint32_t v = list[1 + e];
                     if (v < sink.D) xor_bit(sink, dbase + v);
                     else if (OBS) xor_bit(sink, obase + (v - sink.D));
                 }
+            } else if (OBS) {
+                if ((y >> 29) & 1u) xor_bit(sink, obase);
+                if ((y >> 28) & 1u) xor_bit(sink, obase + 1);
             }
         }
     }
 }
 
+// The same from direct site entries (symptom.h): one 16-byte load per hit names the site's (at most six) detectors
+// and holds, per basis column, a byte of which of them and of the two observables the column flips; the
+// outcome's mask is the XOR of the bytes its code selects. at[k] = the entry's byte offset; a lane without a k-th
+// hit reads one of the 64 null entries, which flip nothing. What bounds the kernel is the gathers, then VALU
+// issue: a wave's 64 scattered loads from an L2-resident table take about 145 cycles of its CU's L1 whatever
+// their width (64 128-byte lines at 56 B per cycle), and a d=25 tile applies 1,745 hits, so the second dependent
+// load per hit that outcome blocks need (site entry, then record) costs more than the XORs into two more words:
+// 2^20 shots at d=25 take 0.547 ms with direct entries, 0.593 ms with outcome blocks (1.11e8 128-byte lines from L2
+// for 1.14e8 hits; 839 VALU instructions per wave; with its row stores the L1 is busy about nine tenths of the time).
+template <bool OBS, uint32_t K>
+__device__ __forceinline__ void apply_direct(const SymDevParams &P, const Sink &sink, const uint32_t *at,
+                                             const uint32_t *oc, const uint32_t *shot) {
+    uint4 se[K];
+#pragma unroll
+    for (uint32_t k = 0; k < K; k++)
+        se[k] = *reinterpret_cast<const uint4 *>(reinterpret_cast<const char *>(P.direct) + at[k]);
+    uint32_t mask[K], rare = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < K; k++) {
+        const uint32_t code = __umulhi(oc[k], se[k].x >> 28) + 1;
+        // Bit j of the code to byte j (0 or 255), the selected bytes XORed together.
+        const uint32_t bits = __umul24(code, 0x204081u) & 0x01010101u;
+        uint32_t t = se[k].w & ((bits << 8) - bits);
+        t ^= t >> 16;
+        t ^= t >> 8;
+        mask[k] = t;
+        rare |= t;
+        const uint32_t dbase = __umul24(shot[k], sink.det_bits) + sink.det_col0;
+        const uint32_t f[6] = {se[k].x & 0x3FFFu, (se[k].x >> 14) & 0x3FFFu, se[k].y & 0x3FFFu,
+                               (se[k].y >> 14) & 0x3FFFu, se[k].z & 0x3FFFu, (se[k].z >> 14) & 0x3FFFu};
+#pragma unroll
+        for (uint32_t e = 0; e < 6; e++) lds_xor_bit(dbase + f[e], (t >> e) & 1u);
+    }
+    // Observables 0 and 1: nearly every wave has a hit that flips observable 0, few lanes do.
+    if (OBS && (rare & 64u)) {
+#pragma unroll
+        for (uint32_t k = 0; k < K; k++)
+            if (mask[k] & 64u) xor_bit(sink, sink.obs_base + __umul24(shot[k], sink.obs_bits) + sink.obs_col0);
+    }
+    if (OBS && (rare & 128u)) {
+#pragma unroll
+        for (uint32_t k = 0; k < K; k++)
+            if (mask[k] & 128u) xor_bit(sink, sink.obs_base + __umul24(shot[k], sink.obs_bits) + sink.obs_col0 + 1);
+    }
+}
+
+// One round of the specialised scan: m gaps per lane, m = M or M - 1 (M fixed at compile time, so that a round is
+// straight-line code: the Philox calls, gaps and positions of all draws are independent work for the scheduler,
+// where a test of the count before every draw kept each in a block of its own). Returns the total of the
+// workgroup's gaps.
+template <bool OBS, bool DIRECT, uint32_t M>
+__device__ __forceinline__ uint32_t fast_round(const SymDevParams &P, const Sink &sink, const SymGroup &G, uint32_t N,
+                                               uint32_t m, uint32_t b0, uint32_t base, uint32_t draw0,
+                                               uint32_t lane_word, uint32_t tile, uint32_t tag, uint32_t k0,
+                                               uint32_t k1, uint32_t *scratch) {
+    const uint32_t S = P.shots_per_tile, lg = P.tile_log2;
+    uint32_t g[M + (M & 1)], oc[M + (M & 1)];
+#pragma unroll
+    for (uint32_t k = 0; 2 * k < M; k++) {
+        const uint4 r = philox10(make_uint4(draw0 + k, lane_word, tile, tag), k0, k1);
+        g[2 * k] = gap32(r.x, G.inv_log);
+        oc[2 * k] = r.y;
+        g[2 * k + 1] = gap32(r.z, G.inv_log);
+        oc[2 * k + 1] = r.w;
+    }
+    // Every draw takes its gap and one position.
+    uint32_t sum = m == M ? g[M - 1] : 0u;
+#pragma unroll
+    for (uint32_t k = 0; k + 1 < M; k++) sum = sat_add(sum, g[k]);
+    const uint2 sc = block_scan(sat_add(sum, m), scratch);
+    // Positions stay at most N: with N < 2^31 - 1 and gaps of at most 2^31, no sum below overflows.
+    uint32_t pos = min(sat_add(base, sc.x), N);
+    // Pass 1: site entry and shot of every hit (no hit: an entry and a shot that are read and applied as 0, spread
+    // over the lanes, since atomics on one word serialise).
+    if (DIRECT) {
+        const uint32_t null_at = (P.direct_null + (threadIdx.x & 63)) << 4;
+        uint32_t at[M], shot[M];
+#pragma unroll
+        for (uint32_t k = 0; k < M; k++) {
+            pos = min(pos + g[k], N);
+            const bool hit = pos < N && (k + 1 < M || m == M);
+            at[k] = hit ? (b0 + (pos >> lg)) << 4 : null_at;
+            shot[k] = pos & (S - 1);
+            pos += 1;
+        }
+        apply_direct<OBS, M>(P, sink, at, oc, shot);
+    } else {
+        uint32_t idx[M], shot[M];
+        bool hit[M];
+#pragma unroll
+        for (uint32_t k = 0; k < M; k++) {
+            pos = min(pos + g[k], N);
+            hit[k] = pos < N && (k + 1 < M || m == M);
+            idx[k] = b0 + (hit[k] ? pos >> lg : 0u);
+            shot[k] = (hit[k] ? pos : threadIdx.x) & (S - 1);
+            pos += 1;
+        }
+        apply_outcomes<OBS, M>(P, sink, idx, oc, shot, hit);
+    }
+    return sc.y;
+}
+
 // Specialised scan tile for models whose groups are plain (compact records, no thinning) and whose
 // members draw outcomes uniformly over codes 1..nout: the QEC memory circuits. It draws exactly the
 // hits scan_tile draws (same counters, gaps, positions and outcome codes), so its rows are
-// bit-identical; it differs in how a hit is applied. Each (site, outcome) has one 8-byte outcome
-// record holding the outcome's whole symptom (entries that cancel between the outcome's basis columns
-// already removed), so a hit reads one record and flips at most four detector bits plus observable
-// flags, instead of testing four basis records of two entries each. Each round first forms every
-// hit's record index and shot, then issues all record loads together (a lane past the end of the
-// group reads the group's first record and applies nothing), then applies the hits.
-template <bool OBS>
+// bit-identical; it differs in how a hit is applied. DIRECT (every site reaches at most six detectors, as in
+// memory circuits without longer checks): one 16-byte entry per site (apply_direct). Otherwise each
+// (site, outcome) has one 8-byte outcome record holding the outcome's whole symptom (entries that cancel
+// between the outcome's basis columns already removed; apply_outcomes). Each round first forms every hit's
+// entry and shot, then issues all entry loads together, then applies the hits.
+template <bool OBS, bool DIRECT>
 __device__ __forceinline__ void scan_tile_fast(const SymDevParams &P, uint32_t btile, uint32_t *lds) {
     const uint32_t S = P.shots_per_tile;
     const uint32_t det_words = (S * P.det_row_bytes + 15) / 16 * 4;
     const uint32_t obs_words = (S * P.obs_row_bytes + 15) / 16 * 4;
-    uint32_t *const scratch = lds + det_words + obs_words;  // 8 words
+    uint32_t *const scratch = lds + det_words + obs_words;  // 8 words: two sets of NT / 64, by round parity
+    uint32_t scans = 0;
     const uint32_t tid = threadIdx.x;
     {
         uint4 *const v = reinterpret_cast<uint4 *>(lds);
@@ -801,51 +920,21 @@ __device__ __forceinline__ void scan_tile_fast(const SymDevParams &P, uint32_t b
         const uint32_t b0 = P.orec_base[4 * gi];
         uint32_t base = 0;
         for (uint32_t round = 0; base < N; round++) {
-            uint32_t g[SCAN_M_MAX], oc[SCAN_M_MAX];
-            uint32_t sum = 0;
-#pragma unroll
-            for (uint32_t k = 0; k < SCAN_M_MAX / 2; k++) {
-                if (2 * k < m) {
-                    const uint4 r = philox10(make_uint4(round * (SCAN_M_MAX / 2) + k, lane_word, tile, TAG_SCAN | gi), k0, k1);
-                    g[2 * k] = gap32(r.x, G.inv_log);
-                    oc[2 * k] = r.y;
-                    g[2 * k + 1] = gap32(r.z, G.inv_log);
-                    oc[2 * k + 1] = r.w;
-                } else {
-                    g[2 * k] = g[2 * k + 1] = 0;
-                    oc[2 * k] = oc[2 * k + 1] = 0;
-                }
-            }
-#pragma unroll
-            for (uint32_t k = 0; k < SCAN_M_MAX; k++) {
-                if (k < m) sum = sat_add(sum, g[k] + 1);
-            }
-            const uint2 sc = block_scan(sum, scratch);
-            uint32_t pos = sat_add(base, sc.x);
-            pos = pos < N ? pos : N;
-            // Pass 1: site entry and shot of every hit (shot S marks no hit; its entry is the group's
-            // first site's, which is read and not applied).
-            uint32_t idx[SCAN_M_MAX], shot[SCAN_M_MAX];
-#pragma unroll
-            for (uint32_t k = 0; k < SCAN_M_MAX; k++) {
-                idx[k] = b0;
-                shot[k] = S;
-                if (k < m) {
-                    pos += g[k] < N ? g[k] : N;
-                    pos = pos < N ? pos : N;
-                    if (pos < N) {
-                        idx[k] = b0 + (pos >> lg);
-                        shot[k] = pos & (S - 1);
-                    }
-                    pos += 1;
-                }
-            }
-            // Pass 2 and 3: record loads in flight together, then the flips (m is uniform).
-            static_assert(SCAN_M_MAX == 8, "two apply widths");
-            if (m > 4) apply_outcomes<OBS, 8>(P, sink, idx, oc, shot, S);
-            else apply_outcomes<OBS, 4>(P, sink, idx, oc, shot, S);
-            base = sat_add(base, sc.y);
-            base = base < N ? base : N;
+            const uint32_t draw0 = round * (SCAN_M_MAX / 2);
+            uint32_t total = 0;
+            static_assert(SCAN_M_MAX == 8, "widths of the rounds");
+            // Five widths: odd counts above 1 run with the next even one, which draws no more Philox blocks.
+#define STIM_AMD_ROUND(M) \
+    total = fast_round<OBS, DIRECT, M>(P, sink, G, N, m, b0, base, draw0, lane_word, tile, TAG_SCAN | gi, k0, k1, \
+                                       scratch + 4 * (scans & 1))
+            if (m > 6) STIM_AMD_ROUND(8);
+            else if (m > 4) STIM_AMD_ROUND(6);
+            else if (m > 2) STIM_AMD_ROUND(4);
+            else if (m > 1) STIM_AMD_ROUND(2);
+            else STIM_AMD_ROUND(1);
+#undef STIM_AMD_ROUND
+            scans++;
+            base = min(sat_add(base, total), N);
         }
     }
     __syncthreads();
@@ -872,20 +961,23 @@ __global__ __launch_bounds__(NT, 6) void sym_scan_waves_kernel(SymDevParams P) {
     scan_tile_waves(P, blockIdx.x, lds);
 }
 
-// The specialised form holds a round's record loads in registers (16 more VGPRs); at d=25 its
-// 31 KB tile image allows 5 workgroups per CU, so it asks for 5 waves per SIMD.
-template <bool OBS>
+// The specialised form holds a round's entry loads in registers; at d=25 its 31 KB tile image allows 5
+// workgroups per CU, so it asks for 5 waves per SIMD (96 VGPRs).
+template <bool OBS, bool DIRECT>
 __global__ __launch_bounds__(NT, 5) void sym_scan_fast_kernel(SymDevParams P) {
     extern __shared__ __align__(16) uint32_t lds[];
-    scan_tile_fast<OBS>(P, blockIdx.x, lds);
+    scan_tile_fast<OBS, DIRECT>(P, blockIdx.x, lds);
 }
 
 // A batch job's tile: the specialised scan for jobs whose sampler has outcome records (the job's
 // plain launch runs that kernel too; rows are identical either way), the generic scan otherwise.
 __device__ __forceinline__ void batch_tile(const SymDevParams &P, uint32_t btile, uint32_t *lds) {
-    if (P.orecs) {
-        if (P.obs_mode != 0) scan_tile_fast<true>(P, btile, lds);
-        else scan_tile_fast<false>(P, btile, lds);
+    if (P.direct) {
+        if (P.obs_mode != 0) scan_tile_fast<true, true>(P, btile, lds);
+        else scan_tile_fast<false, true>(P, btile, lds);
+    } else if (P.orecs) {
+        if (P.obs_mode != 0) scan_tile_fast<true, false>(P, btile, lds);
+        else scan_tile_fast<false, false>(P, btile, lds);
     } else if (P.wave_split) {
         scan_tile_waves(P, btile, lds);
     } else {
@@ -1093,17 +1185,21 @@ hipError_t launch_sym_sample(const SymDevParams &P, uint32_t tiles, size_t lds, 
 hipError_t launch_sym_scan(const SymDevParams &P, uint32_t tiles, size_t lds, hipStream_t stream, bool fast) {
     if (!tiles) return hipSuccess;
     if (fast) {
+#define STIM_AMD_LAUNCH(OBS, DIRECT)                                                                        \
+    {                                                                                                       \
+        static size_t reserved_fast = 0;                                                                    \
+        const hipError_t e = reserve_lds((const void *)sym_scan_fast_kernel<OBS, DIRECT>, lds, reserved_fast); \
+        if (e != hipSuccess) return e;                                                                      \
+        hipLaunchKernelGGL((sym_scan_fast_kernel<OBS, DIRECT>), dim3(tiles), dim3(NT), lds, stream, P);     \
+    }
         if (P.obs_mode != 0) {
-            static size_t reserved_obs = 0;
-            const hipError_t e = reserve_lds((const void *)sym_scan_fast_kernel<true>, lds, reserved_obs);
-            if (e != hipSuccess) return e;
-            hipLaunchKernelGGL(sym_scan_fast_kernel<true>, dim3(tiles), dim3(NT), lds, stream, P);
+            if (P.direct) STIM_AMD_LAUNCH(true, true)
+            else STIM_AMD_LAUNCH(true, false)
         } else {
-            static size_t reserved_plain = 0;
-            const hipError_t e = reserve_lds((const void *)sym_scan_fast_kernel<false>, lds, reserved_plain);
-            if (e != hipSuccess) return e;
-            hipLaunchKernelGGL(sym_scan_fast_kernel<false>, dim3(tiles), dim3(NT), lds, stream, P);
+            if (P.direct) STIM_AMD_LAUNCH(false, true)
+            else STIM_AMD_LAUNCH(false, false)
         }
+#undef STIM_AMD_LAUNCH
         return hipGetLastError();
     }
     if (P.wave_split) {

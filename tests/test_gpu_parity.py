@@ -478,6 +478,32 @@ def test_specialised_scan_kernel_equals_generic(golden, name):
             assert (ra[0] if isinstance(ra, tuple) else ra).any()
 
 
+@pytest.mark.parametrize('shots', [1, 63, 8191, 3 * 8192 + 1])
+def test_specialised_scan_widths_equal_generic(shots):
+    """Every draw count of a round (1 to 8 gaps per lane, and several rounds of 8) and ragged last tiles:
+    the specialised kernel's rows, from direct site entries, equal the generic kernel's bit for bit."""
+    from stim_amd import gen
+
+    def samplers(p):
+        text = gen.generate('surface_code:rotated_memory_z', distance=3, rounds=3, after_clifford_depolarization=p,
+                            after_reset_flip_probability=p, before_measure_flip_probability=p)
+        return [_sampler(text, seed=5, engine='symptom') for _ in range(2)]
+
+    info = samplers(1e-3)[0].engine_info()
+    assert info['outcome_records']
+    positions = info['sites'] * info['tile_shots']
+    # A round of m gaps per lane covers mu + 3 sqrt(mu) + 4 in ((m - 1) * 256, m * 256]; the last p takes several.
+    mus = [((256 * m - 128 - 4 + 2.25) ** 0.5 - 1.5) ** 2 for m in range(1, 9)]
+    widths = [int((mu + 3 * mu ** 0.5 + 4) / 256) + 1 for mu in mus]
+    assert widths == list(range(1, 9))
+    for mu in mus + [20000.0]:
+        a, b = samplers(mu / positions)
+        b.set_scan_variant('generic')
+        for x, y in zip(a.sample(shots, bit_packed=True, separate_observables=True),
+                        b.sample(shots, bit_packed=True, separate_observables=True)):
+            np.testing.assert_array_equal(x, y, err_msg=f'{mu} hits per tile')
+
+
 def test_outcome_blocks_repeat_across_rounds(golden):
     """The specialised kernel stores each distinct block of a site's outcome records (relative to the
     site's lowest detector) once: the d=25, 25-round memory circuit's 108,674 sites and 979,874
