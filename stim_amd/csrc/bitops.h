@@ -94,6 +94,53 @@ __device__ __forceinline__ uint32_t transpose32(uint32_t x, uint32_t lane) {
     return x;
 }
 
+// One level of a 32x32 bit transpose held by one lane: rows i and i + J exchange their off-diagonal blocks.
+__device__ __forceinline__ uint32_t bit_select_const(uint32_t keep, uint32_t a, uint32_t b) {
+    uint32_t r;
+    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "s"(keep), "v"(a), "v"(b));
+    return r;
+}
+
+template <int J>
+__device__ __forceinline__ void transpose_rows_level(uint32_t (&x)[32]) {
+    constexpr uint32_t m = J == 4 ? 0x0F0F0F0Fu : J == 2 ? 0x33333333u : 0x55555555u;
+#pragma unroll
+    for (int i = 0; i < 32; i++) {
+        if (i & J) continue;
+        const uint32_t a = x[i], b = x[i + J];
+        if constexpr (J == 16) {
+            x[i] = __builtin_amdgcn_perm(b, a, 0x05040100u);
+            x[i + J] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+        } else if constexpr (J == 8) {
+            x[i] = __builtin_amdgcn_perm(b, a, 0x06020400u);
+            x[i + J] = __builtin_amdgcn_perm(b, a, 0x07030501u);
+        } else {
+            x[i] = bit_select_const(m, a, b << J);
+            x[i + J] = bit_select_const(m, a >> J, b);
+        }
+    }
+}
+
+// 32x32 bit transpose of 32 rows held by one lane: bit k of x[s] on input becomes bit s of x[k]. 8 VALU
+// instructions per word (byte moves for the two outer levels, shift and bit select for the inner ones) and no
+// cross-lane move, where transpose32 takes 15 and two LDS swizzles; a wave then loads and stores rows with
+// consecutive lanes on consecutive words.
+__device__ __forceinline__ void transpose_rows(uint32_t (&x)[32]) {
+    transpose_rows_level<16>(x);
+    transpose_rows_level<8>(x);
+    transpose_rows_level<4>(x);
+    transpose_rows_level<2>(x);
+    transpose_rows_level<1>(x);
+}
+
+// Tile of workgroup `block` in a grid of n: workgroups go to the 8 XCDs in turn, so tile = block would put
+// neighbouring tiles, which share the 128-byte lines at their edges, on different L2s. Here each XCD
+// gets one contiguous range of tiles (a permutation of 0 .. n - 1 for every n).
+__device__ __forceinline__ uint32_t xcd_tile(uint32_t block, uint32_t n) {
+    const uint32_t x = block & 7u, q = n >> 3, r = n & 7u;
+    return x * q + (x < r ? x : r) + (block >> 3);
+}
+
 // Streams up to 4 bytes of x to p with the widest aligned stores (non-temporal: output rows are
 // written once and must not evict the program from L2).
 __device__ __forceinline__ void store_bytes(uint8_t *p, uint32_t x, uint32_t nbytes) {

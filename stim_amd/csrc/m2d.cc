@@ -12,7 +12,7 @@
 #include "tableau.h"
 
 namespace sa {
-hipError_t launch_m2d(const M2dParams &P, hipStream_t stream);
+hipError_t launch_m2d(M2dParams P, hipStream_t stream);
 size_t m2d_lds_bytes(uint32_t blocks, uint32_t sweep_blocks);
 hipError_t launch_m2d_win(const M2dParams &P, const M2dWindow &Wn, hipStream_t stream);
 size_t m2d_win_lds_bytes(uint32_t ring_words, uint32_t nchunks);
@@ -186,6 +186,12 @@ struct mfs_m2d {
     uint32_t K = 0;   // sweep bits the circuit reads
     std::vector<uint2> cols;
     std::vector<uint32_t> ovf;
+    // Tables of the whole-record kernel (m2d.h).
+    std::vector<uint32_t> terms;
+    std::vector<uint2> block_info;
+    std::vector<uint4> spill;
+    uint32_t spill_slots = 0, slow = 0;
+    DevBuf d_terms, d_block_info, d_spill;
     DevBuf d_cols, d_ovf, d_in, d_out, d_obs, d_tmp, d_sweep;
     // Windowed kernel (no sweep bits), one plan per output layout: 0 = observables appended, 1 =
     // observables separate, 2 = detectors only, 3 = observables appended and separate. kernel_mode:
@@ -232,7 +238,57 @@ struct mfs_m2d {
         P.sweep_stride = 0;
         P.sweep_row_bytes = (uint32_t)sweep_row();
         P.sweep_blocks = sweep_blocks();
+        P.terms = const_cast<DevBuf &>(d_terms).as<uint32_t>();
+        P.block_info = const_cast<DevBuf &>(d_block_info).as<uint2>();
+        P.spill = const_cast<DevBuf &>(d_spill).as<uint4>();
+        P.spill_chunks = (uint32_t)spill.size();
+        P.spill_slots = spill_slots;
+        P.total_blocks = (D + O + 31) / 32;
+        P.slow = slow;
         return P;
+    }
+
+    size_t tile_lds() const { return (size_t)m2d_subtile_words(blocks(), sweep_blocks(), spill_slots) * 4; }
+
+    // Builds the whole-record kernel's tables from the columns' terms (LDS word indices) and inversions. Columns of
+    // more than four terms get a slot each while a tile's words and slots fit in LDS.
+    void build_tables(const std::vector<std::vector<uint32_t>> &col_terms, const std::vector<uint8_t> &invert) {
+        const uint32_t zero = m2d_zero_word(blocks(), sweep_blocks()), cols = D + O;
+        const uint32_t tb = (cols + 31) / 32;
+        for (const auto &ts : col_terms) spill_slots += ts.size() > 4;
+        if (tile_lds() > MAX_LDS) {
+            slow = spill_slots ? 1 : 0;
+            spill_slots = 0;
+        }
+        const uint32_t z = m2d_padded(zero), none = z | (z << 16);
+        terms.assign((size_t)64 * std::max(tb, 1u), none);
+        block_info.assign(std::max(tb, 1u), make_uint2(0, 0));
+        uint32_t slot = 0;
+        for (uint32_t j = 0; j < cols; j++) {
+            const auto &ts = col_terms[j];
+            const uint32_t b = j / 32;
+            uint32_t w[4] = {z, z, z, z};
+            bool listed = false;
+            if (ts.size() <= 4) {
+                for (size_t i = 0; i < ts.size(); i++) w[i] = m2d_padded(ts[i]);
+                if (ts.size() > 2) block_info[b].y = 1;
+            } else if (slow) {
+                listed = true;
+            } else {
+                // The first three terms inline, the others summed into the slot.
+                for (size_t i = 0; i < 3; i++) w[i] = m2d_padded(ts[i]);
+                w[3] = m2d_padded(zero + 4 + slot++);
+                block_info[b].y = 1;
+                for (size_t i = 3; i < ts.size(); i += 4) {
+                    uint32_t u[4];
+                    for (size_t k = 0; k < 4; k++) u[k] = i + k < ts.size() ? m2d_padded(ts[i + k]) : z;
+                    spill.push_back(make_uint4(u[0] | (u[1] << 16), u[2] | (u[3] << 16), w[3], 0));
+                }
+            }
+            terms[(size_t)(j % 32) * tb + b] = listed ? 0xFFFFFFFFu : w[0] | (w[1] << 16);
+            terms[(size_t)(32 + j % 32) * tb + b] = w[2] | (w[3] << 16);
+            if (invert[j]) block_info[b].x |= 1u << (j % 32);
+        }
     }
 
     // Windowed layout usable for a launch, or -1.
@@ -348,6 +404,7 @@ int mfs_m2d_compile(const char *stim_text, size_t len, int skip_reference_sample
                 }
             }
         }
+        if (c->whole_fits()) c->build_tables(col_terms, invert);
         const uint32_t zero_word = m2d_zero_word(c->blocks(), c->sweep_blocks());
         for (size_t j = 0; j < col_terms.size(); j++) {
             const auto &ts = col_terms[j];
@@ -372,6 +429,9 @@ int mfs_m2d_compile(const char *stim_text, size_t len, int skip_reference_sample
         check(hipStreamCreate(&c->stream), "stream");
         mfs_sampler::upload(c->d_cols, c->cols, "m2d columns");
         mfs_sampler::upload(c->d_ovf, c->ovf, "m2d overflow terms");
+        mfs_sampler::upload(c->d_terms, c->terms, "m2d terms");
+        mfs_sampler::upload(c->d_block_info, c->block_info, "m2d blocks");
+        mfs_sampler::upload(c->d_spill, c->spill, "m2d spilled columns");
         for (int l = 0; l < 4; l++) {
             if (c->win[l].ring_words) mfs_sampler::upload(c->d_chunk_end[l], c->win[l].chunk_end, "m2d window");
         }

@@ -1,20 +1,17 @@
-// Measurement-to-detection-event kernel for gfx950 (MI355X).
+// Measurement-to-detection-event kernels for gfx950 (MI355X).
 //
-// One workgroup converts a tile of 32 shots. Its measurement rows are loaded (16-byte loads, several
-// in flight per lane) and transposed 32x32 bits at a time across half-waves into measurement-major
-// words in LDS (word m = measurement m of the tile's 32 shots). Each output column is then the XOR
-// of its measurements' words, inverted when its reference parity is 1 (semantics in m2d.h), and the
-// column words are transposed back into shot-major rows, staged in LDS a chunk of columns at a time
-// and copied to the rows with coalesced stores. HBM traffic is the minimum: each shot's measurement
-// row is read once and its output rows written once.
-//
-// Work is laid out so that lane-dependent branches are rare: loads and LDS stores whose lanes fall
-// past the tile's shots or the row's end go to clamped addresses or padding that no output reads.
+// m2d_kernel converts tiles of 32 shots: 32-column blocks of the measurement rows are loaded one per lane, turned
+// into measurement-major words in LDS (word m = measurement m of the tile's 32 shots) by a transpose in
+// registers; each output column is the XOR of its measurements' words, inverted when its reference parity is 1
+// (semantics in m2d.h), and the column words are transposed back, again one block per lane, and stored. HBM
+// traffic is the minimum: each shot's measurement row is read once and its output rows written once.
 //
 // Also here: the windowed conversion kernel (a ring of recent measurement words per tile, for records
 // longer than LDS holds; m2d.h) and the measurement sampler's expansion kernel (detection events to
 // measurement records; expand.h).
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "bitops.h"
 #include "launch_util.h"
@@ -24,48 +21,7 @@ using namespace sa;
 
 namespace {
 
-constexpr int NT = 1024;
-constexpr uint32_t HALVES = NT / 32;
-constexpr uint32_t UNROLL = 4;                       // 16-byte loads in flight per lane
-constexpr uint32_t CHUNK_BLOCKS = 64;                // output columns staged per pass: 64 blocks of 32
-constexpr uint32_t CHUNK_BYTES = CHUNK_BLOCKS * 4;   // staged bytes per shot row
-constexpr uint32_t PITCH = CHUNK_BYTES + 4;          // LDS bytes per staged row: the pad spreads the
-                                                     // 32 rows of one column block over 32 banks
-
-// Bytes [4b, 4b + 4) of a row, zero past the row's end.
-__device__ __forceinline__ uint32_t load_word_bytes(const uint8_t *row, uint32_t row_bytes, uint32_t b) {
-    uint32_t x = 0;
-#pragma unroll
-    for (uint32_t k = 0; k < 4; k++) {
-        const uint32_t i = 4 * b + k;
-        if (i < row_bytes) x |= (uint32_t)row[i] << (8 * k);
-    }
-    return x;
-}
-
-// Word i of the tile's words, read at its LDS byte address (the words start at LDS address `base`,
-// 0 in these kernels, so no base is added per read).
-typedef __attribute__((address_space(3))) const uint32_t lds_cu32;
-__device__ __forceinline__ uint32_t lds_word(uint32_t base, uint32_t i) {
-    return *(lds_cu32 *)(uintptr_t)(base + 4 * i);
-}
-
-__device__ __forceinline__ uint32_t column_word(const M2dParams &P, uint32_t base, uint2 r) {
-    uint32_t v;
-    if (((r.x >> 28) & 3u) == 3u) {
-        v = 0;
-        const uint32_t n = r.x & M2D_INDEX_MASK;
-        const uint4 *q = reinterpret_cast<const uint4 *>(P.ovf + r.y);
-        for (uint32_t t = 0; t < n; t += 4) {
-            const uint4 a = q[t / 4];
-            v ^= lds_word(base, a.x) ^ lds_word(base, a.y) ^ lds_word(base, a.z) ^ lds_word(base, a.w);
-        }
-    } else {
-        // Unused index fields name the zero word, so both words are XORed unconditionally.
-        v = lds_word(base, r.x & M2D_INDEX_MASK) ^ lds_word(base, r.y);
-    }
-    return v ^ (0u - (r.x >> 31));
-}
+constexpr int M2D_NT = 512;   // whole-record conversion and expansion: lanes per workgroup
 
 // Copies staged rows [0, valid) (pitch P bytes in LDS) to bytes [off, off + nbytes) of shot rows s0 + r
 // as 4-byte stores at any byte alignment (the HSA runtime enables unaligned global access; the
@@ -73,6 +29,7 @@ __device__ __forceinline__ uint32_t column_word(const M2dParams &P, uint32_t bas
 // so one store instruction writes 256 contiguous bytes of a row; the wave's rows step by NTHREADS /
 // 64. A tail of 1 to 3 bytes at the end of a row is written byte by byte.
 typedef uint32_t unaligned_u32 __attribute__((aligned(1)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 template <uint32_t NTHREADS, uint32_t P>
 __device__ __forceinline__ void flush_words(const uint8_t *img, uint8_t *dst, uint64_t stride, uint32_t off,
                                             uint32_t nbytes, uint64_t s0, uint32_t valid) {
@@ -94,123 +51,224 @@ __device__ __forceinline__ void flush_words(const uint8_t *img, uint8_t *dst, ui
     }
 }
 
-// Produces columns [c0, c0 + ncols) of the tile (ncols >= 1), transposed, into shot rows dst (bit 0 =
-// column c0), CHUNK_BLOCKS column blocks at a time: lane l of a half-wave gets shot l's 4 bytes of a
-// 32-column block and puts them in the chunk's LDS image (PITCH bytes per shot); the chunk is then
-// copied to the rows with 4-byte stores at any alignment (flush_words). Image slots of lanes past
-// the tile's shots or blocks past the last are written but never copied; columns past the last
-// read as zero, so the padding bits of each row's last byte are 0.
-__device__ __forceinline__ void emit_columns(const M2dParams &P, const uint32_t *words, uint8_t *img, uint8_t *dst,
-                                             uint64_t stride, uint32_t ncols, uint32_t c0, uint32_t half,
-                                             uint32_t lane, uint64_t s0, uint32_t valid) {
-    constexpr uint32_t CB = CHUNK_BLOCKS / HALVES;
-    const uint32_t nb = (ncols + 31) / 32, pitch = (ncols + 7) / 8;
-    uint32_t *const slot = reinterpret_cast<uint32_t *>(img + lane * PITCH);
-    const uint32_t base = (uint32_t)(uintptr_t)(lds_cu32 *)words;
-    for (uint32_t cb0 = 0; cb0 < nb; cb0 += CHUNK_BLOCKS) {
-        // Every lane of a half-wave runs the same iterations (the transpose moves data within the half).
-        uint2 r[CB];
+// Row words of one lane: x[s] = bytes [4b, 4b + 4) of row s of a subtile (row_bytes - 4 .. row_bytes, shifted
+// down, where the row ends first and `exact` forbids reading past it), for the subtile's rows up to `valid`;
+// later rows repeat the last valid one (their bits belong to shots that are never written). Row s is at
+// base + s * stride + off with `base` and `stride` the same for the whole workgroup, so a row costs a scalar
+// add. Any alignment (the HSA runtime runs with unaligned global access on); a wave's lanes read consecutive
+// words of a row.
+__device__ __forceinline__ void load_rows(uint32_t (&x)[32], const uint8_t *base, uint64_t stride, uint32_t off,
+                                          uint32_t row_bytes, uint32_t b, bool exact, uint32_t valid) {
+    if (exact && row_bytes < 4) {
 #pragma unroll
-        for (uint32_t u = 0; u < CB; u++) {
-            const uint32_t c = (cb0 + half * CB + u) * 32 + lane;
-            const uint2 rec = P.cols[c0 + (c < ncols ? c : ncols - 1)];
-            r[u] = c < ncols ? rec : make_uint2(0, 0);
+        for (uint32_t s = 0; s < 32; s++) {
+            const uint8_t *r = base + (s < valid ? s : valid - 1) * stride + off;
+            uint32_t v = 0;
+            for (uint32_t k = 0; k < row_bytes; k++) v |= (uint32_t)r[k] << (8 * k);
+            x[s] = v;
         }
+        return;
+    }
+    const uint32_t at = exact && 4 * b + 4 > row_bytes ? row_bytes - 4 : 4 * b;
+    if (valid == 32) {
 #pragma unroll
-        for (uint32_t u = 0; u < CB; u++) {
-            slot[half * CB + u] = transpose32(column_word(P, base, r[u]), lane);
-        }
-        __syncthreads();
-        const uint32_t off = 4 * cb0;
-        const uint32_t nbytes = pitch - off < CHUNK_BYTES ? pitch - off : CHUNK_BYTES;
-        flush_words<NT, PITCH>(img, dst, stride, off, nbytes, s0, valid);
-        __syncthreads();
+        for (uint32_t s = 0; s < 32; s++)
+            x[s] = *reinterpret_cast<const unaligned_u32 *>(base + s * stride + (off + at));
+    } else {
+#pragma unroll
+        for (uint32_t s = 0; s < 32; s++)
+            x[s] = *reinterpret_cast<const unaligned_u32 *>(base + (s < valid ? s : valid - 1) * stride + (off + at));
+    }
+    if (exact) {
+        const uint32_t sh = 8 * (4 * b - at);
+#pragma unroll
+        for (uint32_t s = 0; s < 32; s++) x[s] >>= sh;
     }
 }
 
-__global__ __launch_bounds__(NT) void m2d_kernel(M2dParams P) {
-    extern __shared__ __align__(16) uint32_t words[];
-    const uint32_t tid = threadIdx.x, half = tid >> 5, lane = tid & 31;
-    const uint64_t s0 = (uint64_t)blockIdx.x * 32;
-    const uint64_t left = P.shots - s0;
-    const uint32_t valid = left < 32 ? (uint32_t)left : 32u;
-    const bool have = lane < valid;
-    // Lanes past the tile's shots read the tile's first row; their words are never used.
-    const uint8_t *row = P.in + (s0 + (have ? lane : 0)) * P.in_stride;
-    const uint32_t nblk = P.blocks;
-    const uint32_t zero = m2d_zero_word(nblk, P.sweep_blocks);
-    if (tid < 4) words[zero + tid] = 0;
-    if (P.sweep_blocks) {
-        // Sweep-bit words: each lane reads its shot's 4 bytes of a 32-bit block (zero without sweep
-        // data), transposed like the measurement words.
-        const uint8_t *srow = P.sweep ? P.sweep + (s0 + (have ? lane : 0)) * P.sweep_stride : nullptr;
-        const uint32_t sw0 = m2d_sweep_word(nblk);
-        for (uint32_t b = half; b < P.sweep_blocks; b += HALVES) {
-            const uint32_t x = (have && srow) ? load_word_bytes(srow, P.sweep_row_bytes, b) : 0u;
-            words[sw0 + b * 32 + lane] = transpose32(x, lane);
+// Stores a lane's words of a subtile's rows: bytes [4b, 4b + 4) of the row_bytes bytes of row s from x[s];
+// addresses as in load_rows. A row's last word of 1 to 3 bytes goes out as the row's last four bytes, the missing
+// ones from the lane before (which holds the word before and writes the same bytes), or byte by byte where that
+// lane belongs to another wave.
+__device__ __forceinline__ void store_rows(uint32_t (&x)[32], uint8_t *base, uint64_t stride, uint32_t off,
+                                           uint32_t b, uint32_t row_bytes, uint32_t valid) {
+    const uint32_t left = row_bytes - 4 * b;
+    uint32_t at = off + 4 * b;
+    bool single = false;
+    if (__any(left < 4)) {
+        single = left < 4 && (b == 0 || (threadIdx.x & 63) == 0);
+        const bool join = left < 4 && !single;
+#pragma unroll
+        for (uint32_t s = 0; s < 32; s++) {
+            const uint32_t before = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x[s], 0x138, 0xF, 0xF, false);
+            const uint32_t last = __builtin_amdgcn_alignbyte(x[s], before, left & 3u);
+            x[s] = join ? last : x[s];
         }
+        if (join) at = off + row_bytes - 4;
     }
-
-    if (P.in_vec) {
-        // Groups of 4 blocks (16 bytes of each row); UNROLL groups per iteration. Loads past the last
-        // group re-read it; the word region holds whole groups.
-        const uint32_t ngrp = (nblk + 3) / 4;
-        for (uint32_t g0 = half * UNROLL; g0 < ngrp; g0 += HALVES * UNROLL) {
-            uint4 v[UNROLL];
+    if (!single) {
+        if (valid == 32) {
 #pragma unroll
-            for (uint32_t u = 0; u < UNROLL; u++) {
-                const uint32_t g = g0 + u < ngrp ? g0 + u : ngrp - 1;
-                v[u] = *reinterpret_cast<const uint4 *>(row + 16 * (uint64_t)g);
-            }
+            for (uint32_t s = 0; s < 32; s++) *reinterpret_cast<unaligned_u32 *>(base + s * stride + at) = x[s];
+        } else {
 #pragma unroll
-            for (uint32_t u = 0; u < UNROLL; u++) {
-                if (g0 + u < ngrp) {
-                    const uint32_t xs[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-#pragma unroll
-                    for (uint32_t k = 0; k < 4; k++) words[(4 * (g0 + u) + k) * 32 + lane] = transpose32(xs[k], lane);
-                }
-            }
+            for (uint32_t s = 0; s < 32; s++)
+                if (s < valid) *reinterpret_cast<unaligned_u32 *>(base + s * stride + at) = x[s];
         }
     } else {
-        for (uint32_t b = half; b < nblk; b += HALVES) {
-            const uint32_t x = transpose32(have ? load_word_bytes(row, P.in_row_bytes, b) : 0u, lane);
-            words[b * 32 + lane] = x;
+#pragma unroll
+        for (uint32_t s = 0; s < 32; s++) {
+            if (s >= valid) continue;
+            uint8_t *const p = base + s * stride + at;
+            p[0] = (uint8_t)x[s];
+            if (left > 1) p[1] = (uint8_t)(x[s] >> 8);
+            if (left > 2) p[2] = (uint8_t)(x[s] >> 16);
+        }
+    }
+}
+
+// XOR of a column's words (first and second plane entries a, b; column `col` when listed).
+// (a word's LDS address, base + 4 * index, is one multiply-add of a 16-bit half of the entry).
+__device__ __forceinline__ uint32_t terms_word(const uint32_t *w, uint32_t a) {
+    typedef __attribute__((address_space(3))) const uint32_t lds_cu32;
+    const uint32_t base = (uint32_t)(uintptr_t)(lds_cu32 *)w;
+    uint32_t lo, hi;
+    asm("v_mad_u32_u16 %0, %1, 4, %2" : "=v"(lo) : "v"(a), "v"(base));
+    asm("v_mad_u32_u16 %0, %1, 4, %2 op_sel:[1,0,0,0]" : "=v"(hi) : "v"(a), "v"(base));
+    return *(lds_cu32 *)(uintptr_t)lo ^ *(lds_cu32 *)(uintptr_t)hi;
+}
+__device__ __forceinline__ uint32_t listed_word(const M2dParams &P, const uint32_t *w, uint32_t col) {
+    const uint2 rec = P.cols[col];
+    const uint32_t n = rec.x & M2D_INDEX_MASK;
+    const uint4 *q = reinterpret_cast<const uint4 *>(P.ovf + rec.y);
+    uint32_t v = 0;
+    for (uint32_t u = 0; u < n; u += 4) {
+        const uint4 a = q[u / 4];
+        v ^= w[m2d_padded(a.x)] ^ w[m2d_padded(a.y)] ^ w[m2d_padded(a.z)] ^ w[m2d_padded(a.w)];
+    }
+    return v;
+}
+
+// Separate observable rows (a few columns) of a workgroup's shots: one lane per shot and byte.
+template <bool SLOW>
+__device__ __forceinline__ void store_observables(const M2dParams &P, const uint32_t *words, uint32_t subw, uint64_t s0,
+                                                  uint32_t shots) {
+    const uint32_t obytes = (P.n_obs + 7) / 8;
+    for (uint32_t i = threadIdx.x; i < shots * obytes; i += M2D_NT) {
+        const uint32_t shot = i / obytes, j = i - shot * obytes;
+        const uint32_t *const w = words + (shot / 32) * subw;
+        uint32_t v = 0;
+        for (uint32_t k = 0; k < 8 && 8 * j + k < P.n_obs; k++) {
+            const uint32_t col = P.num_det + 8 * j + k, b = col / 32, r = col % 32;
+            const uint2 info = P.block_info[b];
+            const uint32_t a = P.terms[(size_t)r * P.total_blocks + b];
+            uint32_t x;
+            if (SLOW && a == 0xFFFFFFFFu) x = listed_word(P, w, col);
+            else x = terms_word(w, a) ^ (info.y ? terms_word(w, P.terms[(size_t)(32 + r) * P.total_blocks + b]) : 0u);
+            v |= (((x >> (shot % 32)) ^ (info.x >> r)) & 1u) << k;
+        }
+        P.obs[(s0 + shot) * P.obs_stride + j] = (uint8_t)v;
+    }
+}
+
+// Whole-record conversion. A workgroup takes P.group subtiles of 32 shots; its work items are 32-column blocks of
+// a subtile, one lane each. A lane loads its block's word of all 32 rows (32 loads in flight, a wave's lanes on
+// consecutive words of the same row), transposes them in registers and puts the 32 measurement words into LDS;
+// after a barrier it XORs 32 output columns together from LDS, transposes those and stores each row's word, a
+// wave again on consecutive words of a row. Nothing is staged and, but for the columns of more than four terms
+// (summed into slots between two more barriers), one barrier per workgroup is all.
+// What bounds it: HBM and, for output rows of odd width, their stores (1,951-byte rows written 4 bytes a lane
+// take 0.47 ms per 2^20 where 1,948-byte rows take 0.34; with non-temporal stores 0.77). Blocks on lanes
+// rather than rows on lanes (32x32 transposes across half-waves, output staged in LDS 64 blocks at a time) take
+// 0.96 instead of 1.53 ms per 2^20 shots at d=25 (4.3 TB/s); without its loads and stores the kernel takes 0.52.
+// Resident workgroups that prefetch the next tile's rows spill and wait for their stores: 2.1 ms.
+template <bool SLOW>
+__global__ __launch_bounds__(M2D_NT, 4) void m2d_kernel(M2dParams P) {
+    extern __shared__ __align__(16) uint32_t words[];
+    const uint32_t tid = threadIdx.x, G = P.group;
+    const uint64_t s0 = (uint64_t)xcd_tile(blockIdx.x, gridDim.x) * 32 * G;
+    const uint64_t left = P.shots - s0;
+    const uint32_t shots = left < 32 * G ? (uint32_t)left : 32 * G;
+    const uint32_t subs = (shots + 31) / 32;
+    const uint32_t subw = m2d_subtile_words(P.blocks, P.sweep_blocks, P.spill_slots);
+    const uint32_t zero = m2d_padded(m2d_zero_word(P.blocks, P.sweep_blocks));
+    for (uint32_t i = tid; i < subs; i += M2D_NT) words[i * subw + zero] = 0;
+    for (uint32_t i = tid; i < subs * P.spill_slots; i += M2D_NT) {
+        const uint32_t t = i / P.spill_slots;
+        words[t * subw + m2d_padded(m2d_zero_word(P.blocks, P.sweep_blocks) + 4 + (i - t * P.spill_slots))] = 0;
+    }
+
+    // Rows whose stride covers whole words are read past their last byte (never past the buffer's
+    // shots * stride bytes); the bits there belong to no measurement.
+    for (uint32_t i = tid; i < subs * P.blocks; i += M2D_NT) {
+        const uint32_t t = i / P.blocks, b = i - t * P.blocks;
+        uint32_t x[32];
+        load_rows(x, P.in + s0 * P.in_stride, P.in_stride, 32 * t * (uint32_t)P.in_stride, P.in_row_bytes, b, !P.in_vec,
+                  min(shots - 32 * t, 32u));
+        transpose_rows(x);
+        uint32_t *const w = words + t * subw + 33 * b;
+#pragma unroll
+        for (uint32_t k = 0; k < 32; k++) w[k] = x[k];
+    }
+    if (P.sweep_blocks) {
+        const uint32_t sw0 = m2d_padded(m2d_sweep_word(P.blocks));
+        for (uint32_t i = tid; i < subs * P.sweep_blocks; i += M2D_NT) {
+            const uint32_t t = i / P.sweep_blocks, b = i - t * P.sweep_blocks;
+            uint32_t x[32];
+#pragma unroll
+            for (uint32_t s = 0; s < 32; s++) x[s] = 0;
+            // Without sweep data every sweep bit is 0.
+            if (P.sweep)
+                load_rows(x, P.sweep + s0 * P.sweep_stride, P.sweep_stride, 32 * t * (uint32_t)P.sweep_stride,
+                          P.sweep_row_bytes, b, true, min(shots - 32 * t, 32u));
+            transpose_rows(x);
+            uint32_t *const w = words + t * subw + sw0 + 33 * b;
+#pragma unroll
+            for (uint32_t k = 0; k < 32; k++) w[k] = x[k];
         }
     }
     __syncthreads();
-
-    uint8_t *const img = reinterpret_cast<uint8_t *>(words + zero + 4);
-    if (P.n_out) emit_columns(P, words, img, P.out, P.out_stride, P.n_out, 0, half, lane, s0, valid);
-    if (P.n_obs) emit_columns(P, words, img, P.obs, P.obs_stride, P.n_obs, P.num_det, half, lane, s0, valid);
-}
-
-// The expansion's output: column m of the rows is measurement word m, inverted where the reference
-// sample is 1. Column inversion flips bit m of every shot's row, which after the transpose is one XOR
-// of the block's 32 inversion bits (inv[b], the same for every lane) into each lane's output word, so
-// no column records are read. Words past the last measurement are zero, as are their inversion bits.
-__device__ __forceinline__ void emit_identity(const uint32_t *words, const uint32_t *inv, uint8_t *img, uint8_t *dst,
-                                              uint64_t stride, uint32_t ncols, uint32_t half, uint32_t lane,
-                                              uint64_t s0, uint32_t valid) {
-    constexpr uint32_t CB = CHUNK_BLOCKS / HALVES;
-    const uint32_t nb = (ncols + 31) / 32, pitch = (ncols + 7) / 8;
-    uint32_t *const slot = reinterpret_cast<uint32_t *>(img + lane * PITCH);
-    for (uint32_t cb0 = 0; cb0 < nb; cb0 += CHUNK_BLOCKS) {
-        uint32_t w[CB], iv[CB];
-#pragma unroll
-        for (uint32_t u = 0; u < CB; u++) {
-            const uint32_t b = cb0 + half * CB + u;
-            const uint32_t bc = b < nb ? b : nb - 1;
-            w[u] = words[bc * 32 + lane];
-            iv[u] = inv[bc];
+    if (P.spill_chunks) {
+        for (uint32_t i = tid; i < subs * P.spill_chunks; i += M2D_NT) {
+            const uint32_t t = i / P.spill_chunks;
+            const uint4 c = P.spill[i - t * P.spill_chunks];
+            uint32_t *const w = words + t * subw;
+            atomicXor(&w[c.z], terms_word(w, c.x) ^ terms_word(w, c.y));
         }
-#pragma unroll
-        for (uint32_t u = 0; u < CB; u++) slot[half * CB + u] = transpose32(w[u], lane) ^ iv[u];
-        __syncthreads();
-        const uint32_t off = 4 * cb0;
-        const uint32_t nbytes = pitch - off < CHUNK_BYTES ? pitch - off : CHUNK_BYTES;
-        flush_words<NT, PITCH>(img, dst, stride, off, nbytes, s0, valid);
         __syncthreads();
     }
+
+    const uint32_t nb = (P.n_out + 31) / 32, TB = P.total_blocks;
+    for (uint32_t i = tid; i < subs * nb; i += M2D_NT) {
+        const uint32_t t = i / nb, b = i - t * nb;
+        const uint32_t *const w = words + t * subw;
+        const uint2 info = P.block_info[b];
+        uint32_t x[32];
+#pragma unroll
+        for (uint32_t k = 0; k < 32; k++) x[k] = (P.terms + (size_t)k * TB)[b];
+        if (SLOW) {
+#pragma unroll
+            for (uint32_t k = 0; k < 32; k++)
+                x[k] = x[k] != 0xFFFFFFFFu ? terms_word(w, x[k]) : listed_word(P, w, 32 * b + k);
+        } else {
+#pragma unroll
+            for (uint32_t k = 0; k < 32; k++) x[k] = terms_word(w, x[k]);
+        }
+        if (info.y) {
+            // Some column of the block has a third or fourth term.
+#pragma unroll
+            for (uint32_t k = 0; k < 32; k++) x[k] ^= terms_word(w, (P.terms + (size_t)(32 + k) * TB)[b]);
+        }
+        transpose_rows(x);
+        // Inverting a column flips its bit in every shot's row; columns past the last are 0.
+        const uint32_t live = P.n_out - 32 * b;
+        const uint32_t keep = live < 32 ? (1u << live) - 1 : 0xFFFFFFFFu;
+#pragma unroll
+        for (uint32_t s = 0; s < 32; s++) x[s] = (x[s] ^ info.x) & keep;
+        store_rows(x, P.out + s0 * P.out_stride, P.out_stride, 32 * t * (uint32_t)P.out_stride, b, (P.n_out + 7) / 8,
+                   min(shots - 32 * t, 32u));
+    }
+    store_observables<SLOW>(P, words, subw, s0, shots);
 }
 
 // Random words of the free results: Philox4x32-10 keyed by the sampler's expansion key, counter (group of
@@ -218,143 +276,211 @@ __device__ __forceinline__ void emit_identity(const uint32_t *words, const uint3
 constexpr uint32_t TAG_EXPAND = 7u << 28;
 
 // One substitution record (layout in expand.h): words r.x .. r.w, q.x .. q.w.
-__device__ __forceinline__ void expand_record(const ExpandDev &E, uint32_t *words, uint4 r, uint4 q) {
+__device__ __forceinline__ void expand_record(uint32_t *words, uint4 r, uint4 q) {
     uint32_t k = r.x & 0xFFFFu;
     const uint32_t n = r.x >> 16;
-    uint32_t v = words[k];
     if (n == 1) {
         // A chain: each later result XORs the one before it, kept in v. Its results are distinct
         // (stride w > 0) and only this record writes them, so the words it reads are the values
-        // before the chain: they are read 8 at a time ahead of the writes, which turns the chain's
-        // dependent LDS round trips into one per 8 steps.
-        v ^= words[r.y];
-        words[k] = v;
+        // before the chain: they are read 8 at a time ahead of the writes (the last batch repeats its last
+        // result), which turns the chain's dependent LDS round trips into one per 8 (24 at a time: no faster).
+        uint32_t v = words[m2d_padded(k)] ^ words[m2d_padded(r.y)];
+        words[m2d_padded(k)] = v;
         uint32_t j = 1;
         for (; j + 8 <= r.z; j += 8) {
-            uint32_t t[8];
+            uint32_t t[8], at[8];
 #pragma unroll
-            for (uint32_t u = 0; u < 8; u++) t[u] = words[k + (u + 1) * r.w];
+            for (uint32_t u = 0; u < 8; u++) {
+                k += r.w;
+                at[u] = m2d_padded(k);
+                t[u] = words[at[u]];
+            }
 #pragma unroll
             for (uint32_t u = 0; u < 8; u++) {
                 v ^= t[u];
-                words[k + (u + 1) * r.w] = v;
+                words[at[u]] = v;
             }
-            k += 8 * r.w;
         }
-        for (; j < r.z; j++) {
-            k += r.w;
-            v ^= words[k];
-            words[k] = v;
-        }
-    } else if (n <= EXPAND_INLINE_TERMS) {
-        // Terms inline: all seven read together (unused ones name result 0 and are masked).
-        const uint32_t t[EXPAND_INLINE_TERMS] = {r.y, r.z, r.w, q.x, q.y, q.z, q.w};
-        uint32_t w[EXPAND_INLINE_TERMS];
+        if (j < r.z) {
+            const uint32_t last = r.z - j - 1;   // steps after this batch's first
+            uint32_t t[8], at[8];
 #pragma unroll
-        for (uint32_t u = 0; u < EXPAND_INLINE_TERMS; u++) w[u] = words[t[u]];
+            for (uint32_t u = 0; u < 8; u++) {
+                at[u] = m2d_padded(k + (min(u, last) + 1) * r.w);
+                t[u] = words[at[u]];
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < 8; u++) {
+                if (u <= last) v ^= t[u];
+                words[at[u]] = v;
+            }
+        }
+    } else {
+        // Terms inline: all seven read together (unused ones name result 0 and are masked). XORed in with an atomic:
+        // the records that a longer list was cut into add to one result in the same step.
+        const uint32_t t[EXPAND_INLINE_TERMS] = {r.y, r.z, r.w, q.x, q.y, q.z, q.w};
+        uint32_t v = 0, w[EXPAND_INLINE_TERMS];
+#pragma unroll
+        for (uint32_t u = 0; u < EXPAND_INLINE_TERMS; u++) w[u] = words[m2d_padded(t[u])];
 #pragma unroll
         for (uint32_t u = 0; u < EXPAND_INLINE_TERMS; u++) v ^= u < n ? w[u] : 0u;
-        words[k] = v;
-    } else {
-        for (uint32_t t = 0; t < n; t++) v ^= words[E.terms[r.y + t]];
-        words[k] = v;
+        atomicXor(&words[m2d_padded(k)], v);
     }
 }
 
-// Two workgroups per CU (their LDS words allow two): 8 waves per SIMD, at most 64 VGPRs.
-__global__ __launch_bounds__(NT, 8) void expand_kernel(ExpandDev E) {
+// Expansion of detection events into records (semantics in expand.h), laid out as m2d_kernel: E.out.group subtiles
+// of 32 shots per workgroup, a lane per 32-column block of a subtile for the y rows (transposed in registers, each
+// word XORed into its result's word) and again for the record rows. Between them the substitution steps run, a
+// lane per record. With two workgroups per CU they are bound by latency: so the y rows and step 0's
+// records load before anything else, the later steps' records are staged in LDS meanwhile (E.staged), and the
+// last steps, while they have at most 64 records, run on one wave without workgroup barriers. 2^20 shots at d=25:
+// 1.32 ms (3.2 TB/s of y rows read and record rows written), of which the steps are about 0.45; with rows on
+// lanes, staged output and 1024-lane workgroups 1.76.
+// ONE: one subtile per workgroup (no divisions by the counts).
+template <bool ONE>
+__global__ __launch_bounds__(M2D_NT, 4) void expand_kernel(ExpandDev E) {
     extern __shared__ __align__(16) uint32_t words[];
     const M2dParams &P = E.out;
-    const uint32_t tid = threadIdx.x, half = tid >> 5, lane = tid & 31;
-    const uint64_t s0 = (uint64_t)blockIdx.x * 32;
+    const uint32_t tid = threadIdx.x, G = ONE ? 1 : P.group;
+    const uint32_t block = xcd_tile(blockIdx.x, gridDim.x);
+    const uint64_t s0 = (uint64_t)block * 32 * G;
     const uint64_t left = P.shots - s0;
-    const uint32_t valid = left < 32 ? (uint32_t)left : 32u;
-    const bool have = lane < valid;
-    const uint32_t zero = m2d_zero_word(P.blocks, 0);
-    // Phase 0's record range, loaded ahead (phase p + 1's is loaded while phase p runs).
-    // (sched_off holds nphases * NT + 1 offsets: no range without a phase.)
-    uint32_t na = E.nphases ? E.sched_off[tid] : 0u, nb = E.nphases ? E.sched_off[tid + 1] : 0u;
-    for (uint32_t i = tid; i < zero + 4; i += NT) words[i] = 0;
+    const uint32_t shots = left < 32 * G ? (uint32_t)left : 32 * G;
+    const uint32_t subs = ONE ? 1 : (shots + 31) / 32;
+    const uint32_t subw = expand_subtile_words(P.blocks);
+    uint4 *const stage = reinterpret_cast<uint4 *>(words) + (G * subw + 3) / 4;
+    auto split = [&](uint32_t i, uint32_t n, uint32_t &t) {
+        t = ONE ? 0 : i / n;
+        return i - t * n;
+    };
+    // y block i of the workgroup: its rows' words and its columns' slots.
+    uint32_t x[32], slot[16];
+    auto load_block = [&](uint32_t i) {
+        uint32_t t;
+        const uint32_t b = split(i, E.y_blocks, t);
+        load_rows(x, E.in + s0 * E.in_stride, E.in_stride, 32 * t * (uint32_t)E.in_stride, 0, b, false,
+                  min(shots - 32 * t, 32u));
+#pragma unroll
+        for (uint32_t k = 0; k < 16; k++) slot[k] = (E.prim + (size_t)k * E.y_blocks)[b];
+    };
+    if (tid < subs * E.y_blocks) load_block(tid);
+    const uint32_t step0 = E.nsteps ? E.steps[1] : 0, staged = E.staged;
+    // Step 0's records of this lane: tid and tid + M2D_NT.
+    uint4 ra, qa, rb, qb;
+    uint32_t sub;
+    if (tid < subs * step0) {
+        const uint32_t f = split(tid, step0, sub);
+        ra = E.items[2 * f];
+        qa = E.items[2 * f + 1];
+    }
+    if (tid + M2D_NT < subs * step0) {
+        const uint32_t f = split(tid + M2D_NT, step0, sub);
+        rb = E.items[2 * f];
+        qb = E.items[2 * f + 1];
+    }
+    for (uint32_t i = tid; i < 2 * staged; i += M2D_NT) stage[i] = E.items[2 * step0 + i];
+    for (uint32_t i = tid; i < (subs * subw + 3) / 4; i += M2D_NT) reinterpret_cast<uint4 *>(words)[i] = make_uint4(0, 0, 0, 0);
     __syncthreads();
-    // Free results (distinct from every contribution slot, so no ordering with the loads below).
-    const uint64_t tile = E.tile0 + blockIdx.x;
-    const uint32_t k0 = (uint32_t)E.seed, k1 = (uint32_t)(E.seed >> 32);
-    for (uint32_t g = tid; g < (E.nfree + 3) / 4; g += NT) {
+    // Free results (distinct from every y slot, so no ordering with the y words; slots padded, in fours).
+    const uint32_t k0 = (uint32_t)E.seed, k1 = (uint32_t)(E.seed >> 32), fg = (E.nfree + 3) / 4;
+    for (uint32_t i = tid; i < subs * fg; i += M2D_NT) {
+        uint32_t t;
+        const uint32_t g = split(i, fg, t);
+        const uint64_t tile = E.tile0 + (uint64_t)block * G + t;
+        const uint4 at = E.free_slots[g];
         const uint4 r = philox10(make_uint4(g, (uint32_t)tile, (uint32_t)(tile >> 32), TAG_EXPAND), k0, k1);
-        const uint32_t rs[4] = {r.x, r.y, r.z, r.w};
-#pragma unroll
-        for (uint32_t k = 0; k < 4; k++) {
-            if (4 * g + k < E.nfree) words[E.free_slots[4 * g + k]] = rs[k];
-        }
+        uint32_t *const w = words + t * subw;
+        w[at.x] = r.x;
+        w[at.y] = r.y;
+        w[at.z] = r.z;
+        w[at.w] = r.w;
     }
-    // y words, transposed across half-waves like the measurement words of m2d_kernel, XORed into their
-    // slots. Lanes past the tile's shots read the tile's first row: those bits of every word belong to
-    // shots that are never written.
-    // Each lane's slot of its y column is loaded with the rows (it depends on nothing computed), so
-    // a round's loads are all in flight together before the transposes and the XORs.
-    const uint8_t *row = E.in + (s0 + (have ? lane : 0)) * E.in_stride;
-    for (uint32_t g0 = half * UNROLL; g0 < E.in_groups; g0 += HALVES * UNROLL) {
-        uint4 v[UNROLL];
-        uint32_t pr[UNROLL][4];
+    // y words into their slots (two 16-bit padded indices per entry; columns past the last go to the spare word).
+    for (uint32_t i = tid; i < subs * E.y_blocks; i += M2D_NT) {
+        if (i != tid) load_block(i);
+        uint32_t t;
+        const uint32_t b = split(i, E.y_blocks, t);
+        transpose_rows(x);
+        uint32_t *const w = words + t * subw;
 #pragma unroll
-        for (uint32_t u = 0; u < UNROLL; u++) {
-            const uint32_t g = g0 + u < E.in_groups ? g0 + u : E.in_groups - 1;
-            v[u] = *reinterpret_cast<const uint4 *>(row + 16 * (uint64_t)g);
-#pragma unroll
-            for (uint32_t k = 0; k < 4; k++) {
-                const uint32_t y = (4 * (g0 + u) + k) * 32 + lane;
-                pr[u][k] = (g0 + u < E.in_groups && y < E.Y) ? E.prim[y] : 0xFFFFFFFFu;
-            }
+        for (uint32_t k = 0; k < 16; k++) {
+            atomicXor(&w[slot[k] & 0xFFFFu], x[2 * k]);
+            atomicXor(&w[slot[k] >> 16], x[2 * k + 1]);
         }
+        if (E.any_extra) {
 #pragma unroll
-        for (uint32_t u = 0; u < UNROLL; u++) {
-            if (g0 + u < E.in_groups) {
-                const uint32_t xs[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-#pragma unroll
-                for (uint32_t k = 0; k < 4; k++) {
-                    // Every lane of the half-wave takes part in the transpose.
-                    const uint32_t x = transpose32(xs[k], lane);
-                    if (pr[u][k] != 0xFFFFFFFFu) atomicXor(&words[pr[u][k] & 0xFFFFu], x);
-                    if (pr[u][k] != 0xFFFFFFFFu && (pr[u][k] >> 31)) {
-                        const uint32_t y = (4 * (g0 + u) + k) * 32 + lane;
-                        for (uint32_t c = E.extra_off[y]; c < E.extra_off[y + 1]; c++) atomicXor(&words[E.extra[c]], x);
-                    }
-                }
+            for (uint32_t k = 0; k < 32; k++) {
+                const uint32_t y = 32 * b + k;
+                for (uint32_t c = y < E.Y ? E.extra_off[y] : 0; y < E.Y && c < E.extra_off[y + 1]; c++)
+                    atomicXor(&w[m2d_padded(E.extra[c])], x[k]);
             }
         }
     }
-    // Phase 0's first record (record 0 for an empty range; items holds at least one), loaded while
-    // the other waves finish the y pass.
-    uint4 nr = E.items[2 * (na < nb ? na : 0)], nq = E.items[2 * (na < nb ? na : 0) + 1];
     __syncthreads();
-    // Substitution: each thread runs its own items of a phase in record order (its chains need no
-    // barrier); items read results of earlier phases or of the same thread. Each phase's record range
-    // is loaded while the previous phase runs and its first record before the previous barrier.
-    for (uint32_t p = 0; p < E.nphases; p++) {
-        const uint32_t a = na, b = nb;
-        uint4 r = nr, q = nq;
-        if (p + 1 < E.nphases) {
-            na = E.sched_off[(p + 1) * NT + tid];
-            nb = E.sched_off[(p + 1) * NT + tid + 1];
+    // Substitution: a step's records read results of earlier steps (a chain its own, in order).
+    auto step = [&](uint32_t p, uint32_t i0) {
+        const uint32_t at = E.steps[p], n = E.steps[p + 1] - at;
+        for (uint32_t i = i0; i < subs * n; i += M2D_NT) {
+            uint32_t t;
+            const uint32_t f = at + split(i, n, t);
+            uint4 r, q;
+            if (f - step0 < staged) {
+                // An explicit LDS pointer: one that may be either becomes a flat load, which waits for both.
+                typedef __attribute__((address_space(3))) const u32x4 lds_u32x4;
+                lds_u32x4 *const in_lds = (lds_u32x4 *)(stage + 2 * (f - step0));
+                const u32x4 a = in_lds[0], b = in_lds[1];
+                r = make_uint4(a.x, a.y, a.z, a.w);
+                q = make_uint4(b.x, b.y, b.z, b.w);
+            } else {
+                r = E.items[2 * f];
+                q = E.items[2 * f + 1];
+            }
+            expand_record(words + t * subw, r, q);
         }
-        // A thread's records of a phase may depend on each other (through results in LDS only): the
-        // next record's load is issued before the current one runs.
-        for (uint32_t i = a; i < b; i++) {
-            const uint32_t nx = i + 1 < b ? i + 1 : i;
-            const uint4 r2 = E.items[2 * nx], q2 = E.items[2 * nx + 1];
-            expand_record(E, words, r, q);
-            r = r2;
-            q = q2;
+    };
+    if (E.nsteps) {
+        if (tid < subs * step0) {
+            (void)split(tid, step0, sub);
+            expand_record(words + sub * subw, ra, qa);
         }
-        if (p + 1 < E.nphases) {
-            const uint32_t f = na < nb ? na : 0;
-            nr = E.items[2 * f];
-            nq = E.items[2 * f + 1];
+        if (tid + M2D_NT < subs * step0) {
+            (void)split(tid + M2D_NT, step0, sub);
+            expand_record(words + sub * subw, rb, qb);
+        }
+        step(0, tid + 2 * M2D_NT);
+        __syncthreads();
+    }
+    const uint32_t wide = ONE ? max(E.wave_step, 1u) : E.nsteps;
+    for (uint32_t p = 1; p < wide; p++) {
+        step(p, tid);
+        __syncthreads();
+    }
+    if (wide < E.nsteps) {
+        // The final steps on one wave: its LDS accesses complete in order.
+        if (tid < 64) {
+            for (uint32_t p = wide; p < E.nsteps; p++) {
+                step(p, tid);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
         }
         __syncthreads();
     }
-    uint8_t *const img = reinterpret_cast<uint8_t *>(words + zero + 4);
-    emit_identity(words, E.inv, img, P.out, P.out_stride, P.n_out, half, lane, s0, valid);
+    // Records: column m is measurement word m, inverted where the reference sample is 1 (words past the last
+    // measurement are zero, as are their inversion bits).
+    for (uint32_t i = tid; i < subs * P.blocks; i += M2D_NT) {
+        uint32_t t;
+        const uint32_t b = split(i, P.blocks, t);
+        const uint32_t *const w = words + t * subw + 33 * b;
+        const uint32_t inv = E.inv[b];
+#pragma unroll
+        for (uint32_t k = 0; k < 32; k++) x[k] = w[k];
+        transpose_rows(x);
+#pragma unroll
+        for (uint32_t s = 0; s < 32; s++) x[s] ^= inv;
+        store_rows(x, P.out + s0 * P.out_stride, P.out_stride, 32 * t * (uint32_t)P.out_stride, b, (P.n_out + 7) / 8,
+                   min(shots - 32 * t, 32u));
+    }
 }
 
 // ------------------------------------------------------------------ windowed conversion
@@ -538,30 +664,62 @@ hipError_t launch_m2d_win(const M2dParams &P, const M2dWindow &Wn, hipStream_t s
     return hipGetLastError();
 }
 
-hipError_t launch_expand(const ExpandDev &E, hipStream_t stream) {
+// Subtiles per workgroup: as many as fill its lanes with blocks while the words of two or more workgroups fit a CU's
+// LDS (80 KB each), few enough that a small call still spreads over the chip (512 workgroups: two per CU), and
+// rows of a workgroup within the 32-bit offsets its lanes use.
+static uint32_t subtiles(uint64_t tiles, uint32_t blocks, size_t subtile_bytes, uint64_t widest_stride) {
+    uint64_t g = std::min<uint64_t>(M2D_NT / std::max(blocks, 1u), 80 * 1024 / subtile_bytes);
+    g = std::min<uint64_t>(std::min<uint64_t>(g, tiles / 512), (1ull << 31) / 32 / std::max<uint64_t>(widest_stride, 1));
+    return (uint32_t)std::max<uint64_t>(g, 1);
+}
+
+hipError_t launch_expand(ExpandDev E, hipStream_t stream) {
     const uint64_t tiles = (E.out.shots + 31) / 32;
     if (tiles == 0) return hipSuccess;
-    const size_t lds = m2d_lds_bytes(E.out.blocks, 0);
-    static size_t reserved = 0;
-    const hipError_t e = reserve_lds(reinterpret_cast<const void *>(&expand_kernel), lds, reserved);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(expand_kernel, dim3((uint32_t)tiles), dim3(NT), lds, stream, E);
+    const size_t sub = (size_t)expand_subtile_words(E.out.blocks) * 4;
+    E.out.group = subtiles(tiles, std::max(E.out.blocks, E.y_blocks), sub, std::max(E.in_stride, E.out.out_stride));
+    // Records after phase 0 staged in LDS where two workgroups still fit a CU.
+    size_t lds = (sub * E.out.group + 15) / 16 * 16;
+    const size_t later = (size_t)E.staged * 32;
+    if (lds + later <= 80 * 1024) lds += later;
+    else E.staged = 0;
+    const uint64_t grid = (tiles + E.out.group - 1) / E.out.group;
+#define STIM_AMD_LAUNCH(ONE)                                                                              \
+    {                                                                                                     \
+        static size_t reserved = 0;                                                                       \
+        const hipError_t e = reserve_lds(reinterpret_cast<const void *>(&expand_kernel<ONE>), lds, reserved); \
+        if (e != hipSuccess) return e;                                                                    \
+        hipLaunchKernelGGL(expand_kernel<ONE>, dim3((uint32_t)grid), dim3(M2D_NT), lds, stream, E);       \
+    }
+    if (E.out.group == 1) STIM_AMD_LAUNCH(true)
+    else STIM_AMD_LAUNCH(false)
+#undef STIM_AMD_LAUNCH
     return hipGetLastError();
 }
 
-// LDS of a launch: the tile's measurement, sweep and zero words plus the staged output chunk.
+// Limit on a tile's record: its words plus 8 KB.
 size_t m2d_lds_bytes(uint32_t blocks, uint32_t sweep_blocks) {
-    return ((size_t)m2d_zero_word(blocks, sweep_blocks) + 4) * 4 + 32 * PITCH;
+    return ((size_t)m2d_zero_word(blocks, sweep_blocks) + 4) * 4 + 32 * 260;
 }
 
-hipError_t launch_m2d(const M2dParams &P, hipStream_t stream) {
+hipError_t launch_m2d(M2dParams P, hipStream_t stream) {
     const uint64_t tiles = (P.shots + 31) / 32;
     if (tiles == 0) return hipSuccess;
-    const size_t lds = m2d_lds_bytes(P.blocks, P.sweep_blocks);
-    static size_t reserved = 0;
-    const hipError_t e = reserve_lds(reinterpret_cast<const void *>(&m2d_kernel), lds, reserved);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(m2d_kernel, dim3((uint32_t)tiles), dim3(NT), lds, stream, P);
+    const uint32_t nb = std::max(P.blocks, (P.n_out + 31) / 32);
+    const size_t sub = (size_t)m2d_subtile_words(P.blocks, P.sweep_blocks, P.spill_slots) * 4;
+    P.group = subtiles(tiles, nb, sub, std::max(std::max(P.in_stride, P.out_stride), P.sweep_stride));
+    const size_t lds = sub * P.group;
+    const uint64_t grid = (tiles + P.group - 1) / P.group;
+#define STIM_AMD_LAUNCH(SLOW)                                                                          \
+    {                                                                                                  \
+        static size_t reserved = 0;                                                                    \
+        const hipError_t e = reserve_lds(reinterpret_cast<const void *>(&m2d_kernel<SLOW>), lds, reserved); \
+        if (e != hipSuccess) return e;                                                                 \
+        hipLaunchKernelGGL(m2d_kernel<SLOW>, dim3((uint32_t)grid), dim3(M2D_NT), lds, stream, P);      \
+    }
+    if (P.slow) STIM_AMD_LAUNCH(true)
+    else STIM_AMD_LAUNCH(false)
+#undef STIM_AMD_LAUNCH
     return hipGetLastError();
 }
 

@@ -51,7 +51,7 @@ hipError_t launch_sym_fill(const uint8_t *det, uint32_t det_row, const uint8_t *
 hipError_t launch_unpack_rows(const uint8_t *src, uint64_t src_stride, uint8_t *dst, uint64_t dst_stride, uint64_t rows,
                               uint32_t ncols, uint32_t base_char, hipStream_t stream);
 hipError_t launch_philox(const uint32_t *ctr, uint64_t n, uint64_t key, uint32_t *out, hipStream_t stream);
-hipError_t launch_expand(const ExpandDev &E, hipStream_t stream);
+hipError_t launch_expand(ExpandDev E, hipStream_t stream);
 size_t m2d_lds_bytes(uint32_t blocks, uint32_t sweep_blocks);
 }  // namespace sa
 
@@ -98,7 +98,7 @@ inline uint64_t splitmix64(uint64_t x) {
 
 constexpr size_t MAX_LDS = LDS_PER_WORKGROUP;
 constexpr size_t HOST_BATCH_BYTES = (size_t)1 << 30;
-// Threads of an expansion workgroup (m2d_kernel.hip's workgroup size), the width of its schedule.
+// Threads of the expansion's schedule: a run of records each, taken by the workgroup's lanes in turn.
 constexpr uint32_t EXPAND_THREADS = 1024;
 // Host-bound bytes per batch of a call that returns rows in host memory (one of two pipeline slots).
 constexpr size_t PIPE_BATCH_BYTES = (size_t)64 << 20;
@@ -173,7 +173,9 @@ struct mfs_sampler {
     size_t row_pitch_override = 0;        // symptom-engine rows padded to this pitch (0: packed width)
     uint64_t expand_key = 0, expand_tiles = 0;
     uint32_t expand_free = 0, expand_phases = 0, expand_items = 0;
-    DevBuf d_x_prim, d_x_extra_off, d_x_extra, d_x_free, d_x_sched, d_x_items, d_x_terms, d_x_inv, d_x_y;
+    DevBuf d_x_prim, d_x_extra_off, d_x_extra, d_x_free, d_x_steps, d_x_items, d_x_inv, d_x_y;
+    bool expand_extra = false;
+    uint32_t expand_steps = 0, expand_wave_step = 0, expand_later = 0;
     // Detector-error-model samplers: no circuit; the symptom tables come from the model's mechanisms.
     bool dem_mode = false;
     std::vector<uint32_t> dem_col;   // mechanism index (model order) -> symptom column
@@ -529,13 +531,10 @@ struct mfs_sampler {
         // The y rows are the detector sampler's packed rows (observables appended), padded to 16 bytes.
         d->row_pitch_override = std::max<size_t>(((D + O + 7) / 8 + 15) / 16 * 16, 16);
         auto nonempty = [](const std::vector<uint32_t> &v) { return v.empty() ? std::vector<uint32_t>{0, 0} : v; };
-        upload(d_x_prim, nonempty(E.prim), "expansion y slots");
+        upload_expand_slots(E, M);
         upload(d_x_extra_off, E.extra_off, "expansion y slots");
         upload(d_x_extra, nonempty(E.extra), "expansion y slots");
-        upload(d_x_free, nonempty(E.free_slots), "expansion free results");
-        upload(d_x_sched, E.sched_off, "expansion schedule");
-        upload(d_x_items, E.items.empty() ? std::vector<uint32_t>(EXPAND_RECORD_WORDS, 0) : E.items, "expansion items");
-        upload(d_x_terms, nonempty(E.terms), "expansion terms");
+        upload_expand_steps(E);
         // Output inversion: bit m of the words is the reference bit of measurement m (zero past M).
         std::vector<uint32_t> inv((M + 31) / 32 + 1, 0);
         for (uint32_t m = 0; m < M; m++) {
@@ -549,6 +548,65 @@ struct mfs_sampler {
         det_src = std::move(d);
         expand_state = 1;
         return true;
+    }
+
+    // The y columns' slots in the kernel's layout: padded word indices, two 16-bit ones per entry, block-transposed.
+    void upload_expand_slots(const ExpandPlan &E, uint32_t M) {
+        const uint32_t yb = (E.Y + 31) / 32, spare = expand_spare_word((M + 31) / 32);
+        std::vector<uint32_t> slots((size_t)16 * std::max(yb, 1u), spare | (spare << 16));
+        for (uint32_t y = 0; y < E.Y; y++) {
+            if (E.prim[y] == 0xFFFFFFFFu) continue;
+            uint32_t &v = slots[(size_t)(y % 32 / 2) * yb + y / 32];
+            const uint32_t at = m2d_padded(E.prim[y] & 0xFFFFu), sh = 16 * (y & 1);
+            v = (v & ~(0xFFFFu << sh)) | (at << sh);
+        }
+        expand_extra = !E.extra.empty();
+        upload(d_x_prim, slots, "expansion y slots");
+        std::vector<uint32_t> free_at(std::max<size_t>((E.free_slots.size() + 3) / 4 * 4, 4), spare);
+        for (size_t i = 0; i < E.free_slots.size(); i++) free_at[i] = m2d_padded(E.free_slots[i]);
+        upload(d_x_free, free_at, "expansion free results");
+    }
+
+    // The schedule as steps (m2d.h): the threads' first records of a phase, then their second ones, and so on; a list
+    // of more than seven terms as inline records of 2 to 7 terms, on as many lanes (one lane walking the list waits
+    // for a global load per term: at d=25 the observable's 24 terms took 0.2 ms per 2^20 shots, and the one
+    // second record of a thread in phase 0, kept in a loop of dependent loads on that thread, as much again).
+    void upload_expand_steps(const ExpandPlan &E) {
+        std::vector<uint32_t> steps, items;
+        auto records = [&] { return (uint32_t)(items.size() / EXPAND_RECORD_WORDS); };
+        for (uint32_t p = 0; p < E.phases; p++) {
+            const uint32_t *off = E.sched_off.data() + (size_t)p * E.threads;
+            uint32_t most = 0;
+            for (uint32_t t = 0; t < E.threads; t++) most = std::max(most, off[t + 1] - off[t]);
+            for (uint32_t j = 0; j < most; j++) {
+                steps.push_back(records());
+                for (uint32_t t = 0; t < E.threads; t++) {
+                    if (off[t] + j >= off[t + 1]) continue;
+                    const uint32_t *r = E.items.data() + (size_t)(off[t] + j) * EXPAND_RECORD_WORDS;
+                    const uint32_t n = r[0] >> 16;
+                    if (n <= EXPAND_INLINE_TERMS) {
+                        items.insert(items.end(), r, r + EXPAND_RECORD_WORDS);
+                        continue;
+                    }
+                    for (uint32_t done = 0; done < n;) {
+                        const uint32_t left = n - done;
+                        const uint32_t take = std::min(left == EXPAND_INLINE_TERMS + 1 ? left - 2 : left, EXPAND_INLINE_TERMS);
+                        uint32_t rec[EXPAND_RECORD_WORDS] = {(r[0] & 0xFFFFu) | (take << 16)};
+                        for (uint32_t u = 0; u < take; u++) rec[1 + u] = E.terms[r[1] + done + u];
+                        items.insert(items.end(), rec, rec + EXPAND_RECORD_WORDS);
+                        done += take;
+                    }
+                }
+            }
+        }
+        expand_steps = (uint32_t)steps.size();
+        steps.push_back(records());
+        expand_later = expand_steps ? records() - steps[1] : 0;
+        expand_wave_step = expand_steps;
+        while (expand_wave_step > 0 && steps[expand_wave_step] - steps[expand_wave_step - 1] <= 64) expand_wave_step--;
+        if (items.empty()) items.assign(EXPAND_RECORD_WORDS, 0);
+        upload(d_x_steps, steps, "expansion steps");
+        upload(d_x_items, items, "expansion records");
     }
 
     // Whether a measurement-sampler call expands detection events: never with fixed faults or on the
@@ -585,17 +643,19 @@ struct mfs_sampler {
         ExpandDev E{};
         E.in = y;
         E.in_stride = d.row_pitch_override;
-        E.in_groups = (uint32_t)(d.row_pitch_override / 16);
         E.Y = d.prog.num_detectors + d.prog.num_observables;
+        E.y_blocks = (E.Y + 31) / 32;
         E.prim = d_x_prim.as<uint32_t>();
         E.extra_off = d_x_extra_off.as<uint32_t>();
         E.extra = d_x_extra.as<uint32_t>();
-        E.free_slots = d_x_free.as<uint32_t>();
+        E.any_extra = expand_extra ? 1u : 0u;
+        E.free_slots = d_x_free.as<uint4>();
         E.nfree = expand_free;
-        E.nphases = expand_phases;
-        E.sched_off = d_x_sched.as<uint32_t>();
+        E.nsteps = expand_steps;
+        E.steps = d_x_steps.as<uint32_t>();
         E.items = d_x_items.as<uint4>();
-        E.terms = d_x_terms.as<uint32_t>();
+        E.wave_step = expand_wave_step;
+        E.staged = expand_later;
         E.seed = expand_key;
         E.tile0 = tile0;
         M2dParams &P = E.out;
