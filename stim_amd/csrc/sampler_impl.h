@@ -153,6 +153,10 @@ struct mfs_sampler {
     DevBuf d_orecs, d_orec_base, d_orec_sites, d_orec_ovf, d_direct;
     bool sym_direct = false;     // every site has a direct entry
     uint32_t direct_null = 0;
+    // Mechanism records of the mechanism scan (detector error models with few threshold runs).
+    DevBuf d_mechs, d_mech_ovf, d_mech_runs;
+    uint32_t mech_null = 0, mech_runs = 0;
+    bool mech_scan = false;
     uint64_t orec_blocks = 0, orec_records = 0;
     bool sym_fast = false;
     int sym_variant = 0;         // 0: specialised scan kernel where it applies; 1: generic scan kernel
@@ -1182,6 +1186,7 @@ struct mfs_sampler {
                 r32[at + 3] = rec3;
             }
         }
+        if (sym_compact && E < (1ull << 28)) build_mechanism_records(m, thr);
         sym_entries = 0;
         for (const DemError &err : m.errors) sym_entries += err.dets.size() + err.obs.size();
         upload(d_classes, plan.classes, "classes");
@@ -1201,6 +1206,55 @@ struct mfs_sampler {
             upload(d_ovf32, o32, "compact symptom overflow entries");
         }
         sym_state = 1;
+    }
+
+    // Mechanism records and threshold runs of the mechanism scan (symptom.h), when the runs are few.
+    void build_mechanism_records(const DemModel &m, const std::vector<uint32_t> &thr) {
+        std::vector<uint2> runs;
+        for (SymGroup &g : plan.groups) {
+            g.run0 = (uint32_t)runs.size();
+            for (uint32_t s = 0; s < g.nsites; s++) {
+                if (s + 1 < g.nsites && thr[g.site0 + s] == thr[g.site0 + s + 1]) continue;
+                runs.push_back(make_uint2(s + 1, thr[g.site0 + s]));
+                if (runs.size() > SYM_MECH_RUNS) return;
+            }
+            g.runs = 1;
+            while (g.runs < runs.size() - g.run0) g.runs *= 2;
+            runs.resize(g.run0 + g.runs, make_uint2(0xFFFFFFFFu, 0));
+        }
+        if (runs.size() > SYM_MECH_RUNS) return;
+        const uint32_t D = prog.num_detectors;
+        std::vector<uint2> recs;
+        std::vector<uint32_t> lists;
+        for (const SymColumn &c : plan.columns) {
+            const DemError &err = m.errors[c.op];
+            uint32_t d[4] = {}, obs = 0;
+            const size_t nd = err.dets.size();
+            for (uint32_t k : err.obs) obs |= 1u << k;
+            if (nd <= 4) {
+                for (size_t i = 0; i < nd; i++) d[i] = err.dets[i];
+                for (size_t i = nd; i < 4; i++) d[i] = d[0];
+                recs.push_back(make_uint2(d[0] | (d[1] << 14) | (((1u << nd) - 1u) << 28),
+                                          d[2] | (d[3] << 14) | (((obs >> 1) & 1u) << 28) | ((obs & 1u) << 29)));
+                continue;
+            }
+            if (lists.size() >= (1u << 30)) return;
+            recs.push_back(make_uint2(0, SYM_OREC_OVERFLOW | (uint32_t)lists.size()));
+            lists.push_back((uint32_t)(nd + err.obs.size()));
+            lists.insert(lists.end(), err.dets.begin(), err.dets.end());
+            for (uint32_t k : err.obs) lists.push_back(D + k);
+        }
+        mech_null = (uint32_t)recs.size();
+        for (uint32_t l = 0; l < 64; l++) {
+            const uint32_t d = D ? 32 * l % D : 0;
+            recs.push_back(make_uint2(d | (d << 14), d | (d << 14)));
+        }
+        mech_runs = (uint32_t)runs.size();
+        upload(d_groups, plan.groups, "symptom groups");
+        upload(d_mechs, recs, "mechanism records");
+        upload(d_mech_ovf, lists, "mechanism lists");
+        upload(d_mech_runs, runs, "mechanism threshold runs");
+        mech_scan = true;
     }
 
     // Whether a call of `shots` shots runs on the symptom engine. In automatic mode the symptom table
@@ -1273,6 +1327,7 @@ struct mfs_sampler {
         P.orec_sites = nullptr;
         P.orec_ovf = nullptr;
         P.direct = nullptr;
+        P.mechs = nullptr;
         P.err_words = err_words_cur;
         P.err_stride_words = err_stride_cur;
         P.site_mech = dem_mode ? d_site_mech.as<uint32_t>() : nullptr;
@@ -1335,6 +1390,14 @@ struct mfs_sampler {
         if (r.tiles >= (1ull << 31)) throw std::invalid_argument("too many shots in one launch");
         r.scan_ok = scan_ok;
         r.fast = scan_ok && sym_fast && sym_variant == 0 && !P.err_words;
+        if (mech_scan && scan_ok && sym_variant == 0 && !P.err_words) {
+            P.mechs = d_mechs.as<uint2>();
+            P.mech_ovf = d_mech_ovf.as<uint32_t>();
+            P.mech_run_table = d_mech_runs.as<uint2>();
+            P.mech_null = mech_null;
+            P.mech_runs = mech_runs;
+            r.lds_scan = std::max(r.lds_scan, image + 8 * (size_t)mech_runs);
+        }
         if (r.fast) {
             P.orecs = d_orecs.as<uint2>();
             P.orec_base = d_orec_base.as<uint32_t>();

@@ -54,7 +54,8 @@ struct SymGroup {
     uint32_t nout[4];
     uint32_t woff[4];
     uint32_t flags;      // SYM_THIN, SYM_DEM_SLOTS (see below)
-    uint32_t pad[3];
+    uint32_t run0, runs; // the group's threshold runs in the run table, padded to a power of two
+    uint32_t pad;
 };
 static_assert(sizeof(SymGroup) == 96, "SymGroup layout");
 // Thinned group (detector error models, whose mechanisms have many distinct probabilities): the group
@@ -151,12 +152,21 @@ struct SymDevParams {
     // Direct site entries of the specialised scan kernel, indexed as orec_sites (null when some site
     // reaches more than SYM_DIRECT_DETECTORS detectors: its hits then read orec_sites and orecs).
     const uint4 *direct;
+    // Detector error models with few threshold runs (null otherwise, and while a launch records errors): an 8-byte
+    // record per site (the outcome record's layout with absolute detectors; overflow lists in mech_ovf), 64 null
+    // records from mech_null, and the groups' runs of equal thresholds as (site after the run, threshold).
+    const uint2 *mechs;
+    const uint32_t *mech_ovf;
+    const uint2 *mech_run_table;
+    uint32_t mech_null, mech_runs;
     uint32_t direct_null;          // first of 64 null entries (no flips; their fields name words spread over a row)
 };
 // Direct site entry (16 bytes): x = d0 | d1 << 14 | nout << 28, y = d2 | d3 << 14, z = d4 | d5 << 14 with the
 // detectors that the site's basis columns reach (unused fields repeat d0, or are 0), w = byte j: bit e < 6
 // set when basis column j flips detector d_e, bits 6 and 7 when it flips observable 0 and 1.
 constexpr uint32_t SYM_DIRECT_DETECTORS = 6;
+// Run table entries that go into LDS beside a tile's image (8 bytes each); models with more runs keep the generic scan.
+constexpr uint32_t SYM_MECH_RUNS = 512;
 // Outcome record (8 bytes): x = e0 | e1 << 14 | valid << 28, y = e2 | e3 << 14 | obs1 << 28 | obs0 << 29;
 // entries are relative to the site's base detector, valid has bit e set for each of the n = 0..4
 // entries in use (bits 0 .. n - 1), unused entries are 0. A symptom with more than four detectors has

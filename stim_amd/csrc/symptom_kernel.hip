@@ -948,6 +948,182 @@ __device__ __forceinline__ void scan_tile_fast(const SymDevParams &P, uint32_t b
                    P.obs.ptr + s0 * P.obs.stride, P.obs.stride);
 }
 
+// Applies a lane's K draws of a detector error model from its mechanisms' own records (8 bytes, the outcome record's
+// layout with absolute detectors): at[k] = the record's byte offset, a null record for no hit or a hit that
+// thinning drops. Branches and null lanes as in apply_outcomes and apply_direct.
+template <bool OBS, uint32_t K>
+__device__ __forceinline__ void apply_mechanisms(const SymDevParams &P, const Sink &sink, const uint32_t *at,
+                                                 const uint32_t *shot) {
+    uint2 rec[K];
+#pragma unroll
+    for (uint32_t k = 0; k < K; k++)
+        rec[k] = *reinterpret_cast<const uint2 *>(reinterpret_cast<const char *>(P.mechs) + at[k]);
+    uint32_t rare = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < K; k++) {
+        const uint32_t dbase = __umul24(shot[k], sink.det_bits) + sink.det_col0;
+        const uint32_t x = rec[k].x, y = rec[k].y, ry = (y & SYM_OREC_OVERFLOW) ? 0u : y;
+        lds_xor_bit(dbase + (x & 0x3FFFu), (x >> 28) & 1u);
+        lds_xor_bit(dbase + ((x >> 14) & 0x3FFFu), (x >> 29) & 1u);
+        lds_xor_bit(dbase + (ry & 0x3FFFu), (x >> 30) & 1u);
+        lds_xor_bit(dbase + ((ry >> 14) & 0x3FFFu), x >> 31);
+        rare |= y;
+    }
+    if (rare >> 28) {
+#pragma unroll
+        for (uint32_t k = 0; k < K; k++) {
+            const uint32_t y = rec[k].y;
+            if (!(y >> 28)) continue;
+            const uint32_t obase = sink.obs_base + __umul24(shot[k], sink.obs_bits) + sink.obs_col0;
+            if (y & SYM_OREC_OVERFLOW) {
+                const uint32_t dbase = __umul24(shot[k], sink.det_bits) + sink.det_col0;
+                const uint32_t *list = P.mech_ovf + (y & ~SYM_OREC_OVERFLOW);
+                const uint32_t cnt = list[0];
+                for (uint32_t e = 0; e < cnt; e++) {
+                    const uint32_t v = list[1 + e];
+                    if (v < sink.D) xor_bit(sink, dbase + v);
+                    else if (OBS) xor_bit(sink, obase + (v - sink.D));
+                }
+            } else if (OBS) {
+                if ((y >> 29) & 1u) xor_bit(sink, obase);
+                if ((y >> 28) & 1u) xor_bit(sink, obase + 1);
+            }
+        }
+    }
+}
+
+// Draws of a wave's range of a group: M gaps and outcome words per lane, in order of lanes, from Philox draws
+// draw .. draw + M / 2 - 1 of `lane_word`; m = M or M - 1 of them count. Positions and hits as in scan_tile_waves
+// (same counters, so rows are bit-identical); returns the total of the wave's gaps.
+template <bool OBS, uint32_t M>
+__device__ __forceinline__ uint32_t mech_round(const SymDevParams &P, const Sink &sink, const SymGroup &G,
+                                               const uint2 *runs, uint32_t lo, uint32_t N, uint32_t m, uint32_t base,
+                                               uint32_t draw, uint32_t lane_word, uint32_t tile, uint32_t tag,
+                                               uint32_t k0, uint32_t k1) {
+    uint32_t g[M + (M & 1)], oc[M + (M & 1)];
+#pragma unroll
+    for (uint32_t k = 0; 2 * k < M; k++) {
+        const uint4 r = philox10(make_uint4(draw + k, lane_word, tile, tag), k0, k1);
+        g[2 * k] = gap32(r.x, G.inv_log);
+        oc[2 * k] = r.y;
+        g[2 * k + 1] = gap32(r.z, G.inv_log);
+        oc[2 * k + 1] = r.w;
+    }
+    uint32_t sum = m == M ? g[M - 1] : 0u;
+#pragma unroll
+    for (uint32_t k = 0; k + 1 < M; k++) sum = sat_add(sum, g[k]);
+    const uint2 sc = wave_scan(sat_add(sum, m));
+    uint32_t pos = min(sat_add(base, sc.x), N);
+    uint32_t srel[M], shot[M], run[M], at[M];
+    bool hit[M];
+#pragma unroll
+    for (uint32_t k = 0; k < M; k++) {
+        pos = min(pos + g[k], N);
+        hit[k] = pos < N && (k + 1 < M || m == M);
+        srel[k] = (lo + pos) >> P.tile_log2;
+        shot[k] = (lo + pos) & (P.shots_per_tile - 1);
+        run[k] = 0;
+        pos += 1;
+    }
+    // Threshold of each site: the group's runs of equal thresholds, padded to a power of two.
+    for (uint32_t half = G.runs >> 1; half; half >>= 1) {
+#pragma unroll
+        for (uint32_t k = 0; k < M; k++) run[k] += runs[run[k] + half - 1].x <= srel[k] ? half : 0u;
+    }
+    const uint32_t null_at = (P.mech_null + (threadIdx.x & 63)) << 3;
+#pragma unroll
+    for (uint32_t k = 0; k < M; k++) {
+        const bool fired = hit[k] && oc[k] <= runs[run[k]].y;
+        at[k] = fired ? (G.site0 + srel[k]) << 3 : null_at;
+    }
+    apply_mechanisms<OBS, M>(P, sink, at, shot);
+    return sc.y;
+}
+
+// scan_tile_waves for models whose thresholds lie in few runs (mechanisms are sampled in order of probability, so
+// equal ones are neighbours): the run table sits in LDS, so that a hit's threshold costs no gather and a hit
+// that thinning drops no gather either, and a mechanism's record is 8 bytes, so that 356,321 of them (2.9 MB) stay
+// in an XCD's 4 MB of L2, where the generic records (16 bytes a site, 5.7 MB) do not: a wave's 64 scattered loads
+// take about 145 cycles of its CU's L1 from L2 and 326 from beyond it. A range's first round takes up to 8 gaps
+// a lane; what the first 512 draws leave is mostly under 100 hits, drawn 128 at a time (two a lane, the same
+// draws in the same order) instead of another 512. 2^20 shots of the d=25 model: 0.683 ms, 1.25 ms with
+// scan_tile_waves (now 1.21). It stays for models of more runs and for launches that record errors.
+template <bool OBS>
+__device__ __forceinline__ void scan_tile_mechs(const SymDevParams &P, uint32_t btile, uint32_t *lds) {
+    const uint32_t S = P.shots_per_tile;
+    const uint32_t det_words = (S * P.det_row_bytes + 15) / 16 * 4;
+    const uint32_t obs_words = (S * P.obs_row_bytes + 15) / 16 * 4;
+    uint2 *const runs = reinterpret_cast<uint2 *>(lds + det_words + obs_words);
+    const uint32_t tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    {
+        uint4 *const v = reinterpret_cast<uint4 *>(lds);
+        for (uint32_t i = tid; i < (det_words + obs_words) / 4; i += NT) v[i] = make_uint4(0, 0, 0, 0);
+    }
+    for (uint32_t i = tid; i < P.mech_runs; i += NT) runs[i] = P.mech_run_table[i];
+    const Sink sink = make_sink(P, lds, det_words);
+    float total = 0.0f;
+    for (uint32_t gi = 0; gi < P.ngroups; gi++) {
+        const SymGroup G = P.groups[gi];
+        if (G.p > 0.0f) total += (float)(G.nsites << P.tile_log2) * G.p;
+    }
+    const float a0 = total * (float)wave / (float)(NT / 64), a1 = total * (float)(wave + 1) / (float)(NT / 64);
+    __syncthreads();
+
+    const uint64_t s0 = (uint64_t)btile * S;
+    const uint64_t tile64 = P.tile0 + btile;
+    const uint32_t tile = (uint32_t)tile64, lane_word = sym_lane_word(tid, tile64);
+    const uint32_t k0 = (uint32_t)P.seed, k1 = (uint32_t)(P.seed >> 32);
+    float c = 0.0f;
+    for (uint32_t gi = 0; gi < P.ngroups; gi++) {
+        const SymGroup G = P.groups[gi];
+        if (!(G.p > 0.0f)) continue;
+        const uint32_t Ng = G.nsites << P.tile_log2;
+        const float h = (float)Ng * G.p;
+        const uint32_t lo = __builtin_amdgcn_readfirstlane(draw_position(a0, c, G.p, Ng));
+        const uint32_t hi = __builtin_amdgcn_readfirstlane(wave + 1 == NT / 64 ? Ng : draw_position(a1, c, G.p, Ng));
+        c += h;
+        if (hi <= lo) continue;
+        const uint32_t N = hi - lo;
+        const float mu = (float)N * G.p;
+        uint32_t m = __builtin_amdgcn_readfirstlane((uint32_t)((mu + 3.0f * sqrtf(mu) + 4.0f) / 64) + 1);
+        if (m > SCAN_M_MAX) m = SCAN_M_MAX;
+        const uint2 *const r = runs + G.run0;
+        const uint32_t tag = TAG_SCAN | gi;
+        uint32_t base = 0;
+        for (uint32_t round = 0; base < N; round++) {
+            const uint32_t draw0 = round * (SCAN_M_MAX / 2);
+            if (m == SCAN_M_MAX && (float)(N - base) * G.p < 256.0f) {
+                // The round's draws in order, 128 at a time: 16 lanes' eight, two on each lane.
+                for (uint32_t part = 0; part < 4 && base < N; part++) {
+                    const uint32_t t = mech_round<OBS, 2>(P, sink, G, r, lo, N, 2, base, draw0 + (lane & 3),
+                                                          sym_lane_word(64 * wave + 16 * part + (lane >> 2), tile64),
+                                                          tile, tag, k0, k1);
+                    base = min(sat_add(base, t), N);
+                }
+                continue;
+            }
+            uint32_t t;
+#define STIM_AMD_ROUND(M) t = mech_round<OBS, M>(P, sink, G, r, lo, N, m, base, draw0, lane_word, tile, tag, k0, k1)
+            if (m > 6) STIM_AMD_ROUND(8);
+            else if (m > 4) STIM_AMD_ROUND(6);
+            else if (m > 2) STIM_AMD_ROUND(4);
+            else if (m > 1) STIM_AMD_ROUND(2);
+            else STIM_AMD_ROUND(1);
+#undef STIM_AMD_ROUND
+            base = min(sat_add(base, t), N);
+        }
+    }
+    __syncthreads();
+
+    const uint64_t valid = P.shots > s0 ? (P.shots - s0 < S ? P.shots - s0 : S) : 0;
+    if (P.dets.enabled)
+        write_rows(reinterpret_cast<const uint8_t *>(lds), P.det_row_bytes, (uint32_t)valid,
+                   P.dets.ptr + s0 * P.dets.stride, P.dets.stride);
+    if (P.obs.enabled && P.obs_row_bytes)
+        write_rows(reinterpret_cast<const uint8_t *>(lds + det_words), P.obs_row_bytes, (uint32_t)valid,
+                   P.obs.ptr + s0 * P.obs.stride, P.obs.stride);
+}
+
 // Both scan kernels ask for 6 waves per SIMD (at most 80 VGPRs, no spills): the sampler is bound by
 // instruction issue and latency, so resident waves matter more than registers.
 __global__ __launch_bounds__(NT, 6) void sym_scan_kernel(SymDevParams P) {
@@ -959,6 +1135,12 @@ __global__ __launch_bounds__(NT, 6) void sym_scan_kernel(SymDevParams P) {
 __global__ __launch_bounds__(NT, 6) void sym_scan_waves_kernel(SymDevParams P) {
     extern __shared__ __align__(16) uint32_t lds[];
     scan_tile_waves(P, blockIdx.x, lds);
+}
+
+template <bool OBS>
+__global__ __launch_bounds__(NT, 5) void sym_scan_mechs_kernel(SymDevParams P) {
+    extern __shared__ __align__(16) uint32_t lds[];
+    scan_tile_mechs<OBS>(P, blockIdx.x, lds);
 }
 
 // The specialised form holds a round's entry loads in registers; at d=25 its 31 KB tile image allows 5
@@ -978,6 +1160,9 @@ __device__ __forceinline__ void batch_tile(const SymDevParams &P, uint32_t btile
     } else if (P.orecs) {
         if (P.obs_mode != 0) scan_tile_fast<true, false>(P, btile, lds);
         else scan_tile_fast<false, false>(P, btile, lds);
+    } else if (P.mechs) {
+        if (P.obs_mode != 0) scan_tile_mechs<true>(P, btile, lds);
+        else scan_tile_mechs<false>(P, btile, lds);
     } else if (P.wave_split) {
         scan_tile_waves(P, btile, lds);
     } else {
@@ -1199,6 +1384,19 @@ hipError_t launch_sym_scan(const SymDevParams &P, uint32_t tiles, size_t lds, hi
             if (P.direct) STIM_AMD_LAUNCH(false, true)
             else STIM_AMD_LAUNCH(false, false)
         }
+#undef STIM_AMD_LAUNCH
+        return hipGetLastError();
+    }
+    if (P.mechs) {
+#define STIM_AMD_LAUNCH(OBS)                                                                          \
+    {                                                                                                 \
+        static size_t reserved_mechs = 0;                                                             \
+        const hipError_t e = reserve_lds((const void *)sym_scan_mechs_kernel<OBS>, lds, reserved_mechs); \
+        if (e != hipSuccess) return e;                                                                \
+        hipLaunchKernelGGL(sym_scan_mechs_kernel<OBS>, dim3(tiles), dim3(NT), lds, stream, P);        \
+    }
+        if (P.obs_mode != 0) STIM_AMD_LAUNCH(true)
+        else STIM_AMD_LAUNCH(false)
 #undef STIM_AMD_LAUNCH
         return hipGetLastError();
     }

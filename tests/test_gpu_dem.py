@@ -364,3 +364,34 @@ def test_sample_write_err_out_and_replay_files(golden, tmp_path, fmt):
                                 obs_out_format=fmt, replay_err_in_file=paths['e'], replay_err_in_format=fmt)
     np.testing.assert_array_equal(formats.read_rows(paths['d2'], fmt, D, [('D', D)]), d)
     np.testing.assert_array_equal(formats.read_rows(paths['o2'], fmt, O, [('L', O)]), o)
+
+
+def _random_model(rng, mechanisms, probabilities, detectors, observables, most):
+    lines = [f'detector D{detectors - 1}']
+    for _ in range(mechanisms):
+        n = int(rng.integers(0, most + 1))
+        targets = [f'D{d}' for d in rng.choice(detectors, size=min(n, detectors), replace=False)]
+        targets += [f'L{k}' for k in range(observables) if rng.random() < 0.2]
+        lines.append(f'error({float(rng.choice(probabilities))!r}) ' + ' '.join(targets))
+    return '\n'.join(lines) + '\n'
+
+
+@pytest.mark.parametrize('mechanisms, probabilities, detectors, observables, most, shots', [
+    (1, [0.3], 1, 0, 1, 1),
+    (40, [1.0, 0.4, 0.0, 1e-3], 7, 2, 4, 4097),             # certain, impossible and thinned mechanisms
+    (700, [0.01, 0.009, 0.0051, 0.005], 50, 1, 8, 20001),   # lists of more than four detectors
+    (900, [2e-4], 3000, 2, 4, 3001),                        # one run per group
+    (3000, [0.02 * 0.97 ** k for k in range(120)], 400, 1, 4, 700),      # many runs, several rounds a wave
+    (2000, list(0.003 + 1e-6 * np.arange(1500)), 900, 1, 3, 500),        # more runs than the table takes
+])
+def test_mechanism_scan_equals_generic(mechanisms, probabilities, detectors, observables, most, shots):
+    """The scan over 8-byte mechanism records and threshold runs gives the generic scan's rows bit for bit."""
+    import stim_amd
+    from stim_amd import _native as N
+    text = _random_model(np.random.default_rng(mechanisms), mechanisms, probabilities, detectors, observables, most)
+    model = stim_amd.DetectorErrorModel(text)
+    a, b = model.compile_sampler(seed=3), model.compile_sampler(seed=3)
+    N.check(N.lib().mfs_set_scan_variant(b._h, 1))
+    for _ in range(2):
+        for x, y in zip(a.sample(shots, bit_packed=True)[:2], b.sample(shots, bit_packed=True)[:2]):
+            np.testing.assert_array_equal(x, y)
