@@ -41,6 +41,7 @@ enum {
     MFS_APPEND_OBSERVABLES = 1u << 2,
     MFS_SEPARATE_OBSERVABLES = 1u << 3, /* write observables to obs (reference: separate_observables or obs_out) */
     MFS_DEVICE_OUTPUT = 1u << 4,     /* dets/obs are device pointers (results stay in HBM) */
+    MFS_BYTE_INPUT = 1u << 5,        /* mfs_m2d_convert*: host measurement rows hold one byte per result (0 or not 0) */
 };
 
 /* Compiles .stim circuit text. seed is used when has_seed != 0 (reference: seed=None draws
@@ -82,7 +83,8 @@ void mfs_m2d_destroy(mfs_m2d *c);
 /* out[0..3] = num_measurements, num_detectors, num_observables, num_sweep_bits (largest sweep[k]
  * index plus one). */
 int mfs_m2d_stats(const mfs_m2d *c, uint64_t out[4]);
-/* Converts `shots` bit-packed little-endian measurement rows (meas_stride bytes apart) into detection
+/* Converts `shots` bit-packed little-endian measurement rows (meas_stride bytes apart; with MFS_BYTE_INPUT,
+ * host rows of one byte per result) into detection
  * event rows (with observables appended when MFS_APPEND_OBSERVABLES) and, with
  * MFS_SEPARATE_OBSERVABLES, observable rows; MFS_BIT_PACKED selects packed outputs (else one byte per
  * entry); MFS_DEVICE_OUTPUT means every pointer is device memory. Each detector (observable) is the

@@ -20,6 +20,7 @@ MFS_PREPEND_OBSERVABLES = 1 << 1
 MFS_APPEND_OBSERVABLES = 1 << 2
 MFS_SEPARATE_OBSERVABLES = 1 << 3
 MFS_DEVICE_OUTPUT = 1 << 4
+MFS_BYTE_INPUT = 1 << 5
 
 EXPORTED = [
     'mfs_compile', 'mfs_destroy', 'mfs_circuit_stats', 'mfs_parse_stats', 'mfs_sample', 'mfs_sample_write',

@@ -1,12 +1,18 @@
 // Double-buffered delivery of batch outputs from device memory to the caller's host rows.
 //
 // A call that returns rows in host memory runs in batches. Batch i's kernels write into device slot
-// i % 2; a copy engine moves the slot's rows to pinned host buffer i % 2 on a second stream; host
-// threads then copy them from the pinned buffer to the caller's rows (pageable, any row stride). While
-// batch i's rows cross PCIe and are copied on the host, batch i + 1's kernels run into the other slot.
+// i % 2; a copy engine moves the slot's rows to pinned host buffer i % 2 on a second stream, a chunk of rows at
+// a time; host threads copy each chunk that has arrived from the pinned buffer to the caller's rows (pageable,
+// any row stride), or expand its bits to one byte per entry (a transfer of an eighth of the bytes). So the
+// host copy of a chunk runs while the next one crosses PCIe, also in a call of one batch, and while
+// batch i's rows travel, batch i + 1's kernels run into the other slot. 131,071 rows of 274 bytes (36 MB, 0.63 ms
+// at the link's 57 GB/s) into new numpy arrays, whose pages are touched for the first time here: 1.17 ms, and 1.1
+// to 1.5 ms with one transfer and then one copy of the whole batch; 20,001 rows of 1,798 entries as bytes 1.4 instead of
+// 1.8 ms. Inputs in host memory (m2d) take the same way in: 50,001 records of 181 bytes converted in 0.72 ms, where
+// a pitched copy from pageable memory took 9 us for each row, 460 ms.
 // Per slot, three orderings keep the buffers consistent:
 //   - the DMA of batch i waits for batch i's kernels (event `produced`, a wait on the copy stream);
-//   - batch i + 2's kernels wait for batch i's DMA out of the slot (event `copied`, a wait on the
+//   - batch i + 2's kernels wait for batch i's DMA out of the slot (the last event `arrived`, a wait on the
 //     compute stream: the host does not block);
 //   - batch i + 2's DMA into the pinned buffer waits for the host copy of batch i out of it (a join of
 //     that batch's host threads, before the DMA is queued).
@@ -14,13 +20,22 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <emmintrin.h>
 #include <sched.h>
 
 #include <algorithm>
+#include <array>
+#include <atomic>
+#include <chrono>
+#include <condition_variable>
 #include <cstdint>
 #include <cstring>
+#include <deque>
+#include <functional>
+#include <mutex>
 #include <stdexcept>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -36,10 +51,92 @@ inline hipError_t copy_rows_async(void *dst, size_t dst_pitch, const void *src, 
     return hipMemcpy2DAsync(dst, dst_pitch, src, src_pitch, width, rows, kind, stream);
 }
 
+// Expands `n` bits of src to bytes base + bit.
+inline void expand_bits(const uint8_t *src, uint8_t *dst, size_t n, uint8_t base) {
+    static const std::array<uint64_t, 256> table = [] {
+        std::array<uint64_t, 256> t{};
+        for (uint32_t b = 0; b < 256; b++)
+            for (uint32_t k = 0; k < 8; k++) t[b] |= (uint64_t)((b >> k) & 1) << (8 * k);
+        return t;
+    }();
+    const uint64_t add = 0x0101010101010101ull * base;
+    size_t i = 0;
+    for (; i + 8 <= n; i += 8) {
+        const uint64_t v = table[src[i >> 3]] + add;
+        std::memcpy(dst + i, &v, 8);
+    }
+    for (; i < n; i++) dst[i] = (uint8_t)(((src[i >> 3] >> (i & 7)) & 1u) + base);
+}
+
+// Packs `n` bytes into bits (1 where the byte is not 0), padding bits 0.
+inline void pack_bytes(const uint8_t *src, uint8_t *dst, size_t n) {
+    size_t i = 0;
+    for (; i + 16 <= n; i += 16) {
+        const __m128i x = _mm_loadu_si128(reinterpret_cast<const __m128i *>(src + i));
+        const uint16_t m = (uint16_t)~_mm_movemask_epi8(_mm_cmpeq_epi8(x, _mm_setzero_si128()));
+        std::memcpy(dst + (i >> 3), &m, 2);
+    }
+    for (; i < n; i += 8) {
+        uint8_t b = 0;
+        for (size_t k = 0; k < 8 && i + k < n; k++) b |= (uint8_t)((src[i + k] != 0) << k);
+        dst[i >> 3] = b;
+    }
+}
+
+// Host threads of all pipelines in the process: at most as many as a batch uses (HostPipe::host_threads), started when
+// work waits and no thread is idle, and ended after a second without work. Starting threads anew for
+// each batch took about 15 us each, as much as a 1 MB transfer.
+class CopyPool {
+   public:
+    static CopyPool &get() {
+        static CopyPool *pool = new CopyPool;   // never destroyed: a thread may still be idle at exit
+        return *pool;
+    }
+    // Queues f to run on some thread; false when none could be started and none will take it.
+    bool run(std::function<void()> f, int most) {
+        std::unique_lock<std::mutex> lock(mu_);
+        if (idle_ <= (int)queue_.size() && alive_ < most) {
+            try {
+                std::thread([this] { serve(); }).detach();
+                alive_++;
+            } catch (const std::system_error &) {
+                if (alive_ == 0) return false;
+            }
+        }
+        queue_.push_back(std::move(f));
+        lock.unlock();
+        cv_.notify_one();
+        return true;
+    }
+
+   private:
+    void serve() {
+        std::unique_lock<std::mutex> lock(mu_);
+        for (;;) {
+            idle_++;
+            cv_.wait_for(lock, std::chrono::seconds(1), [&] { return !queue_.empty(); });
+            idle_--;
+            if (queue_.empty()) break;
+            std::function<void()> f = std::move(queue_.front());
+            queue_.pop_front();
+            lock.unlock();
+            f();
+            lock.lock();
+        }
+        alive_--;
+    }
+    std::mutex mu_;
+    std::condition_variable cv_;
+    std::deque<std::function<void()>> queue_;
+    int alive_ = 0, idle_ = 0;
+};
+
 class HostPipe {
    public:
-    // One output of a batch: `rows` rows of `row` bytes at `dev` (stride `dev_stride`) go to `host`
-    // (stride `host_stride`); when `newline_at` >= 0 each host row also gets '\n' at that byte.
+    // One output of a batch: `rows` rows of `row` bytes at `dev` (stride `dev_stride`, little more than `row`; the
+    // buffer holds rows * dev_stride bytes) go to `host`
+    // (stride `host_stride`); when `newline_at` >= 0 each host row also gets '\n' at that byte. With `bits`, a row
+    // holds that many bits, which become bytes base + bit on the host.
     struct Part {
         const uint8_t *dev;
         size_t dev_stride;
@@ -47,6 +144,8 @@ class HostPipe {
         uint8_t *host;
         size_t host_stride;
         long newline_at;
+        size_t bits = 0;
+        uint8_t base = 0;
     };
 
     HostPipe() = default;
@@ -57,8 +156,12 @@ class HostPipe {
         for (int s = 0; s < 2; s++) {
             if (dev_[s]) (void)hipFree(dev_[s]);
             if (pin_[s]) (void)hipHostFree(pin_[s]);
+            if (pin_in_[s]) (void)hipHostFree(pin_in_[s]);
             if (produced_[s]) (void)hipEventDestroy(produced_[s]);
-            if (copied_[s]) (void)hipEventDestroy(copied_[s]);
+            if (consumed_[s]) (void)hipEventDestroy(consumed_[s]);
+            for (hipEvent_t e : arrived_[s]) {
+                if (e) (void)hipEventDestroy(e);
+            }
         }
         if (copy_) (void)hipStreamDestroy(copy_);
     }
@@ -71,18 +174,21 @@ class HostPipe {
         return std::max(1, std::min(n, 8));
     }
 
-    // Prepares a call on `compute`: both device slots hold at least `dev_bytes`, both pinned buffers
-    // at least `host_bytes`. Nothing of an earlier call is in flight (finish() or drain ended it).
-    void begin(hipStream_t compute, size_t dev_bytes, size_t host_bytes) {
+    // Prepares a call on `compute` of one batch or several: the device slots hold at least `dev_bytes`, the pinned
+    // buffers at least `host_bytes`, the pinned input buffers `in_bytes` (the first of each for one batch). Nothing
+    // of an earlier call is in flight (finish() or drain ended it).
+    void begin(hipStream_t compute, bool several, size_t dev_bytes, size_t host_bytes, size_t in_bytes = 0) {
         compute_ = compute;
+        chk(hipGetDevice(&device_), "device");
         if (!copy_) {
             chk(hipStreamCreateWithFlags(&copy_, hipStreamNonBlocking), "copy stream");
             for (int s = 0; s < 2; s++) {
                 chk(hipEventCreateWithFlags(&produced_[s], hipEventDisableTiming), "event");
-                chk(hipEventCreateWithFlags(&copied_[s], hipEventDisableTiming), "event");
+                chk(hipEventCreateWithFlags(&consumed_[s], hipEventDisableTiming), "event");
+                for (hipEvent_t &e : arrived_[s]) chk(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event");
             }
         }
-        for (int s = 0; s < 2; s++) {
+        for (int s = 0; s < (several ? 2 : 1); s++) {
             if (dev_cap_[s] < dev_bytes) {
                 if (dev_[s]) chk(hipFree(dev_[s]), "hipFree");
                 dev_[s] = nullptr;
@@ -90,16 +196,11 @@ class HostPipe {
                 chk(hipMalloc(reinterpret_cast<void **>(&dev_[s]), dev_bytes), "hipMalloc (host pipeline slot)");
                 dev_cap_[s] = dev_bytes;
             }
-            if (pin_cap_[s] < host_bytes) {
-                if (pin_[s]) chk(hipHostFree(pin_[s]), "hipHostFree");
-                pin_[s] = nullptr;
-                pin_cap_[s] = 0;
-                chk(hipHostMalloc(reinterpret_cast<void **>(&pin_[s]), host_bytes, hipHostMallocDefault),
-                    "hipHostMalloc (host pipeline buffer)");
-                pin_cap_[s] = host_bytes;
-            }
-            used_[s] = false;
+            pinned(pin_[s], pin_cap_[s], host_bytes);
+            pinned(pin_in_[s], pin_in_cap_[s], in_bytes);
         }
+        for (int s = 0; s < 2; s++) used_[s] = in_used_[s] = false;
+        in_at_ = 0;
         batch_ = 0;
         pending_ = -1;
         nthreads_ = host_threads();
@@ -109,17 +210,50 @@ class HostPipe {
     // of the batch that last used the slot has read it.
     uint8_t *next_slot(size_t *cap) {
         const int s = batch_ & 1;
-        if (used_[s]) chk(hipStreamWaitEvent(compute_, copied_[s], 0), "wait for slot");
+        if (used_[s]) chk(hipStreamWaitEvent(compute_, arrived_[s][batches_[s].chunks - 1], 0), "wait for slot");
         *cap = dev_cap_[s];
         return dev_[s];
     }
 
-    // Queues the DMA of the batch whose kernels were just queued into next_slot()'s slot, then starts
-    // the host copy of the batch before it (waiting for that batch's DMA to end).
+    // Queues the copy of `rows` host rows into device rows of `pitch` bytes on the compute stream, through the batch's
+    // pinned input buffer: rows of `row` bytes, or, with `bytes`, of that many bytes to pack into bits (row = packed
+    // bytes). Inputs of a batch are queued before its kernels, each at its own offset of the buffer.
+    void input(uint8_t *dev, size_t pitch, const uint8_t *host, size_t host_stride, size_t row, uint64_t rows,
+               size_t bytes = 0) {
+        const int s = batch_ & 1;
+        if (!row || !rows) return;
+        if (in_used_[s] && in_at_ == 0) chk(hipEventSynchronize(consumed_[s]), "input buffer");
+        if (in_at_ + pitch * rows > pin_in_cap_[s]) throw std::logic_error("host pipeline input exceeds its pinned buffer");
+        uint8_t *const pin = pin_in_[s] + in_at_;
+        in_at_ += pitch * rows;
+        auto copy = [=](uint64_t r0, uint64_t r1) {
+            if (bytes) {
+                for (uint64_t r = r0; r < r1; r++) pack_bytes(host + r * host_stride, pin + r * pitch, bytes);
+            } else if (host_stride == row && pitch == row) {
+                std::memcpy(pin + r0 * row, host + r0 * row, (r1 - r0) * row);
+            } else {
+                for (uint64_t r = r0; r < r1; r++) std::memcpy(pin + r * pitch, host + r * host_stride, row);
+            }
+        };
+        const size_t total = std::max(row, bytes) * rows;
+        const int k = (int)std::max<uint64_t>(1, std::min<uint64_t>(nthreads_, total >> 20));
+        Team team;
+        team.start(k - 1, nthreads_, [&, k](int t) { copy(rows * t / k, rows * (t + 1) / k); }, k);
+        team.finish();
+        chk(hipMemcpyAsync(dev, pin, pitch * rows, hipMemcpyHostToDevice, compute_), "copy from pinned buffer");
+        chk(hipEventRecord(consumed_[s], compute_), "record");
+        in_used_[s] = true;
+    }
+
+    // Queues the DMA of the batch whose kernels were just queued (a chunk of rows after another), and has
+    // the batch's host threads take the chunks as they arrive.
     void submit(const std::vector<Part> &parts, uint64_t rows) {
         const int s = batch_ & 1;
-        size_t need = 0;
-        for (const Part &p : parts) need += p.row * rows;
+        size_t need = 0, host_bytes = 0;
+        for (const Part &p : parts) {
+            need += p.dev_stride * rows;
+            host_bytes += (p.bits ? p.bits : p.row) * rows;
+        }
         if (need > pin_cap_[s]) throw std::logic_error("host pipeline batch exceeds its pinned buffer");
         join(s);
         chk(hipEventRecord(produced_[s], compute_), "record");
@@ -127,26 +261,41 @@ class HostPipe {
         Batch &b = batches_[s];
         b.parts.clear();
         b.rows = rows;
+        b.chunks = (int)std::max<uint64_t>(1, std::min<uint64_t>({(uint64_t)MAX_CHUNKS, host_bytes / CHUNK_BYTES, rows}));
         size_t off = 0;
         for (const Part &p : parts) {
-            if (p.row && rows) {
-                chk(copy_rows_async(pin_[s] + off, p.row, p.dev, p.dev_stride, p.row, rows, hipMemcpyDeviceToHost,
-                                    copy_),
-                    "copy to pinned buffer");
-            }
-            b.parts.push_back(Part{pin_[s] + off, p.row, p.row, p.host, p.host_stride, p.newline_at});
-            off += p.row * rows;
+            Part q = p;
+            q.dev = pin_[s] + off;
+            b.parts.push_back(q);
+            off += p.dev_stride * rows;
         }
-        chk(hipEventRecord(copied_[s], copy_), "record");
+        for (int c = 0; c < b.chunks; c++) {
+            const uint64_t r0 = rows * c / b.chunks, r1 = rows * (c + 1) / b.chunks;
+            for (size_t i = 0; i < parts.size(); i++) {
+                const Part &p = parts[i];
+                // Whole device rows, padding included: the runtime splits a pitched copy into per-row transfers.
+                if (p.row && r1 > r0)
+                    chk(hipMemcpyAsync(const_cast<uint8_t *>(b.parts[i].dev) + r0 * p.dev_stride, p.dev + r0 * p.dev_stride,
+                                       (r1 - r0) * p.dev_stride, hipMemcpyDeviceToHost, copy_),
+                        "copy to pinned buffer");
+            }
+            chk(hipEventRecord(arrived_[s][c], copy_), "record");
+        }
         used_[s] = true;
-        if (pending_ >= 0) start_host_copy(pending_);
-        pending_ = s;
+        // Threads only where each gets at least 1 MiB; a smaller batch is copied by the caller, at the next
+        // submit() or finish().
+        b.nthreads = (int)std::min<uint64_t>(nthreads_, host_bytes >> 20);
+        if (pending_ >= 0) copy_small(pending_);
+        pending_ = -1;
+        if (b.nthreads > 1) start(s);
+        else pending_ = s;
+        in_at_ = 0;
         batch_++;
     }
 
     // Delivers the last batch and waits for every host copy.
     void finish() {
-        if (pending_ >= 0) start_host_copy(pending_);
+        if (pending_ >= 0) copy_small(pending_);
         pending_ = -1;
         join(0);
         join(1);
@@ -154,67 +303,153 @@ class HostPipe {
 
     // Ends whatever is in flight without reporting errors (used when a call is unwinding).
     void drain_noexcept() {
-        for (int s = 0; s < 2; s++) join(s);
+        for (int s = 0; s < 2; s++) {
+            if (batches_[s].team.total) batches_[s].team.finish();
+            batches_[s].error = hipSuccess;
+            if (in_used_[s]) (void)hipEventSynchronize(consumed_[s]);
+        }
         if (copy_) (void)hipStreamSynchronize(copy_);
         pending_ = -1;
+        in_at_ = 0;
     }
 
    private:
+    static constexpr int MAX_CHUNKS = 16;
+    static constexpr size_t CHUNK_BYTES = (size_t)2 << 20;   // host bytes per chunk, at least
+
+    // Shares 0 .. total - 1 of some work, taken by up to `helpers` pool threads and by the thread that finishes it.
+    struct Team {
+        std::function<void(int)> share;
+        int total = 0;
+        std::atomic<int> next{0};
+        int helping = 0;
+        std::mutex mu;
+        std::condition_variable cv;
+
+        void work() {
+            for (int i = next++; i < total; i = next++) share(i);
+        }
+        void start(int helpers, int most, std::function<void(int)> f, int n) {
+            share = std::move(f);
+            next = 0;
+            total = n;
+            for (int h = 0; h < helpers; h++) {
+                {
+                    std::lock_guard<std::mutex> lock(mu);
+                    helping++;
+                }
+                auto leave = [this] {
+                    std::lock_guard<std::mutex> lock(mu);
+                    if (--helping == 0) cv.notify_all();
+                };
+                if (!CopyPool::get().run([this, leave] { work(); leave(); }, most)) leave();
+            }
+        }
+        void finish() {
+            work();
+            std::unique_lock<std::mutex> lock(mu);
+            cv.wait(lock, [&] { return helping == 0; });
+            total = 0;
+        }
+    };
+
     struct Batch {
-        std::vector<Part> parts;   // dev = pinned source rows (dense), dev_stride = row
+        std::vector<Part> parts;   // dev = pinned source rows, at the device rows' stride
         uint64_t rows = 0;
-        std::vector<std::thread> workers;
+        int chunks = 1, nthreads = 1;
+        std::atomic<int> ready{0};     // chunks that have arrived; -1: an error ended the wait
+        std::atomic_flag waiting = ATOMIC_FLAG_INIT;   // some thread waits for the next chunk
+        hipError_t error = hipSuccess;
+        Team team;
     };
 
     static void chk(hipError_t e, const char *what) {
         if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
     }
 
+    static void pinned(uint8_t *&p, size_t &cap, size_t bytes) {
+        if (cap >= bytes) return;
+        if (p) chk(hipHostFree(p), "hipHostFree");
+        p = nullptr;
+        cap = 0;
+        chk(hipHostMalloc(reinterpret_cast<void **>(&p), bytes, hipHostMallocDefault), "hipHostMalloc (host pipeline buffer)");
+        cap = bytes;
+    }
+
     static void copy_rows(const Batch &b, uint64_t r0, uint64_t r1) {
         for (const Part &p : b.parts) {
             if (!p.row && p.newline_at < 0) continue;
-            const uint8_t *src = p.dev + r0 * p.row;
+            const uint8_t *src = p.dev + r0 * p.dev_stride;
             uint8_t *dst = p.host + r0 * p.host_stride;
-            if (p.host_stride == p.row && p.newline_at < 0) {
+            if (p.host_stride == p.row && p.dev_stride == p.row && p.newline_at < 0 && !p.bits) {
                 std::memcpy(dst, src, (r1 - r0) * p.row);
                 continue;
             }
-            for (uint64_t r = r0; r < r1; r++, src += p.row, dst += p.host_stride) {
-                std::memcpy(dst, src, p.row);
+            for (uint64_t r = r0; r < r1; r++, src += p.dev_stride, dst += p.host_stride) {
+                if (p.bits) expand_bits(src, dst, p.bits, p.base);
+                else std::memcpy(dst, src, p.row);
                 if (p.newline_at >= 0) dst[p.newline_at] = '\n';
             }
         }
     }
 
-    void start_host_copy(int s) {
-        chk(hipEventSynchronize(copied_[s]), "copy to pinned buffer");
+    // A batch too small for threads: waits for its last chunk and copies it here.
+    void copy_small(int s) {
         Batch &b = batches_[s];
-        const uint64_t rows = b.rows;
-        size_t bytes = 0;
-        for (const Part &p : b.parts) bytes += p.row * rows;
-        // Threads only where each gets at least 1 MiB.
-        const uint64_t k = std::max<uint64_t>(1, std::min<uint64_t>(nthreads_, bytes >> 20));
-        if (k == 1) {
-            copy_rows(b, 0, rows);
-            return;
-        }
-        for (uint64_t t = 0; t < k; t++) {
-            const uint64_t r0 = rows * t / k, r1 = rows * (t + 1) / k;
-            b.workers.emplace_back([&b, r0, r1] { copy_rows(b, r0, r1); });
-        }
+        chk(hipEventSynchronize(arrived_[s][b.chunks - 1]), "copy to pinned buffer");
+        copy_rows(b, 0, b.rows);
+    }
+
+    // Has pool threads take the batch's shares (chunk * nthreads + part of the chunk) as the chunks arrive: of the threads
+    // that need a chunk, one waits for its event and the others for that one.
+    void start(int s) {
+        Batch &b = batches_[s];
+        b.ready = 0;
+        b.error = hipSuccess;
+        auto share = [&b, s, this](int i) {
+            const int c = i / b.nthreads, part = i % b.nthreads;
+            int ready, polls = 0;
+            while ((ready = b.ready.load(std::memory_order_acquire)) >= 0 && ready <= c) {
+                if (!b.waiting.test_and_set(std::memory_order_acquire)) {
+                    ready = b.ready.load(std::memory_order_acquire);
+                    if (ready >= 0 && ready <= c) {
+                        hipError_t e = hipSetDevice(device_);
+                        if (e == hipSuccess) e = hipEventSynchronize(arrived_[s][ready]);
+                        if (e != hipSuccess) b.error = e;
+                        b.ready.store(e == hipSuccess ? ready + 1 : -1, std::memory_order_release);
+                    }
+                    b.waiting.clear(std::memory_order_release);
+                } else if (++polls < 1000) {
+                    std::this_thread::yield();
+                } else {
+                    std::this_thread::sleep_for(std::chrono::microseconds(20));   // a long kernel
+                }
+            }
+            if (ready < 0) return;
+            const uint64_t a = b.rows * c / b.chunks, n = b.rows * (c + 1) / b.chunks - a;
+            copy_rows(b, a + n * part / b.nthreads, a + n * (part + 1) / b.nthreads);
+        };
+        b.team.start(b.nthreads, nthreads_, share, b.chunks * b.nthreads);
     }
 
     void join(int s) {
-        for (std::thread &t : batches_[s].workers) t.join();
-        batches_[s].workers.clear();
+        Batch &b = batches_[s];
+        if (b.team.total) b.team.finish();
+        const hipError_t e = b.error;
+        b.error = hipSuccess;
+        chk(e, "copy to pinned buffer");
     }
 
     hipStream_t compute_ = nullptr, copy_ = nullptr;
-    hipEvent_t produced_[2] = {nullptr, nullptr}, copied_[2] = {nullptr, nullptr};
+    int device_ = 0;
+    hipEvent_t produced_[2] = {nullptr, nullptr}, consumed_[2] = {nullptr, nullptr};
+    hipEvent_t arrived_[2][MAX_CHUNKS] = {};
     uint8_t *dev_[2] = {nullptr, nullptr};
     uint8_t *pin_[2] = {nullptr, nullptr};
-    size_t dev_cap_[2] = {0, 0}, pin_cap_[2] = {0, 0};
-    bool used_[2] = {false, false};
+    uint8_t *pin_in_[2] = {nullptr, nullptr};
+    size_t dev_cap_[2] = {0, 0}, pin_cap_[2] = {0, 0}, pin_in_cap_[2] = {0, 0};
+    bool used_[2] = {false, false}, in_used_[2] = {false, false};
+    size_t in_at_ = 0;   // bytes of the next batch's pinned input buffer in use
     Batch batches_[2];
     uint64_t batch_ = 0;
     int pending_ = -1;

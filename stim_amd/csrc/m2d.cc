@@ -192,7 +192,7 @@ struct mfs_m2d {
     std::vector<uint4> spill;
     uint32_t spill_slots = 0, slow = 0;
     DevBuf d_terms, d_block_info, d_spill;
-    DevBuf d_cols, d_ovf, d_in, d_out, d_obs, d_tmp, d_sweep;
+    DevBuf d_cols, d_ovf, d_in, d_out, d_obs, d_sweep;
     // Windowed kernel (no sweep bits), one plan per output layout: 0 = observables appended, 1 =
     // observables separate, 2 = detectors only, 3 = observables appended and separate. kernel_mode:
     // 0 = the whole-record kernel where the tile's record fits in LDS, else windowed; 1 = whole-record
@@ -203,6 +203,7 @@ struct mfs_m2d {
     int kernel_mode = 0;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    HostPipe pipe;
 
     ~mfs_m2d() {
         if (ev0) (void)hipEventDestroy(ev0);
@@ -330,6 +331,51 @@ struct mfs_m2d {
         check(launch_m2d(P, stream), "m2d launch");
     }
 };
+
+// Conversion of host rows: batches through the host pipeline, the rows packed (where they are bytes) and the
+// results expanded on the host, whole rows in one linear transfer each way. The windowed kernel reads rows at the
+// 16-byte stride, the whole-record kernel tight ones.
+static void convert_host(mfs_m2d &c, uint64_t shots, const uint8_t *meas, size_t meas_stride, bool bytes, const uint8_t *sweep,
+                         size_t sweep_stride, uint8_t *dets, size_t dets_stride, uint32_t n_out, uint8_t *obs,
+                         size_t obs_stride, uint32_t n_obs, bool packed) {
+    const bool tight = c.whole_fits() && c.kernel_mode != 2;
+    const size_t in_pitch = tight ? c.in_row() : std::max<size_t>(c.in_vec_stride(), 16);
+    const size_t srow = sweep ? c.sweep_row() : 0, out_row = (n_out + 7) / 8, obs_row = (n_obs + 7) / 8;
+    // Batches of about HOST_CONVERT_BYTES of host rows each way, so that the host's copies of one overlap the transfers
+    // and the kernel of another.
+    constexpr size_t HOST_CONVERT_BYTES = (size_t)16 << 20;
+    const size_t host_row = std::max<size_t>({bytes ? c.M : c.in_row(), (packed ? out_row : n_out) + (packed ? obs_row : n_obs), 1});
+    const uint64_t batch = std::min<uint64_t>(shots, std::max<uint64_t>(32, HOST_CONVERT_BYTES / host_row / 32 * 32));
+    struct Drain {
+        HostPipe &p;
+        ~Drain() { p.drain_noexcept(); }
+    } drain{c.pipe};
+    auto up = [](size_t n) { return (n + 255) / 256 * 256; };
+    const size_t in_bytes = up(batch * in_pitch), sweep_bytes = up(batch * srow), out_bytes = up(batch * out_row);
+    c.pipe.begin(c.stream, batch < shots, in_bytes + sweep_bytes + out_bytes + up(batch * obs_row) + 256,
+                 std::max<size_t>(batch * (out_row + obs_row), 256), batch * (in_pitch + srow));
+    for (uint64_t s0 = 0; s0 < shots; s0 += batch) {
+        const uint64_t n = std::min(batch, shots - s0);
+        size_t cap;
+        uint8_t *const d_in = c.pipe.next_slot(&cap), *const d_sweep = d_in + in_bytes, *const d_out = d_sweep + sweep_bytes,
+                *const d_obs = d_out + out_bytes;
+        if (c.M) c.pipe.input(d_in, in_pitch, meas + s0 * meas_stride, meas_stride, c.in_row(), n, bytes ? c.M : 0);
+        M2dParams P = c.params(n, d_in, in_pitch, d_out, std::max<size_t>(out_row, 1), n_out, d_obs,
+                               std::max<size_t>(obs_row, 1), n_obs);
+        if (sweep) {
+            c.pipe.input(d_sweep, srow, sweep + s0 * sweep_stride, sweep_stride, srow, n);
+            P.sweep = d_sweep;
+            P.sweep_stride = srow;
+        }
+        c.launch(P);
+        std::vector<HostPipe::Part> parts;
+        if (n_out) parts.push_back({d_out, out_row, out_row, dets + s0 * dets_stride, dets_stride, -1L, packed ? 0u : n_out, 0});
+        if (n_obs) parts.push_back({d_obs, obs_row, obs_row, obs + s0 * obs_stride, obs_stride, -1L, packed ? 0u : n_obs, 0});
+        c.pipe.submit(parts, n);
+    }
+    c.pipe.finish();
+    check(hipStreamSynchronize(c.stream), "m2d");
+}
 
 extern "C" {
 
@@ -488,7 +534,9 @@ int mfs_m2d_convert_sweep(mfs_m2d *c, uint64_t shots, const uint8_t *meas, size_
         if (shots == 0) return;
         const uint32_t n_out = c->D + (append ? c->O : 0), n_obs = separate ? c->O : 0;
         const size_t out_row = (n_out + 7) / 8, obs_row = (n_obs + 7) / 8;
-        if (c->M && (!meas || meas_stride < c->in_row())) throw std::invalid_argument("measurement rows are too short");
+        const bool bytes = flags & MFS_BYTE_INPUT;
+        if (bytes && device) throw std::invalid_argument("measurement rows in device memory must be bit packed");
+        if (c->M && (!meas || meas_stride < (bytes ? c->M : c->in_row()))) throw std::invalid_argument("measurement rows are too short");
         if (n_out && (!dets || dets_stride < (packed ? out_row : n_out))) throw std::invalid_argument("detection event rows are too short");
         if (n_obs && (!obs || obs_stride < (packed ? obs_row : n_obs))) throw std::invalid_argument("observable rows are too short");
         if (device && packed) {
@@ -499,51 +547,38 @@ int mfs_m2d_convert_sweep(mfs_m2d *c, uint64_t shots, const uint8_t *meas, size_
             check(hipStreamSynchronize(c->stream), "m2d");
             return;
         }
-        // Staged: batches of shots through device buffers (input rows at the vector stride).
+        if (!device) {
+            convert_host(*c, shots, meas, meas_stride, bytes, sweep, sweep_stride, dets, dets_stride, n_out, obs, obs_stride,
+                         n_obs, packed);
+            return;
+        }
+        // Device rows of one byte per entry: batches of shots through device buffers (input rows at the vector stride).
         const size_t vs = std::max<size_t>(c->in_vec_stride(), 16);
         const size_t srow = sweep ? c->sweep_row() : 0;
-        const size_t per_shot = vs + srow + out_row + obs_row + (packed ? 0 : n_out + n_obs);
+        const size_t per_shot = vs + srow + out_row + obs_row + n_out + n_obs;
         const uint64_t batch = std::max<uint64_t>(32, (HOST_BATCH_BYTES / std::max<size_t>(per_shot, 1)) / 32 * 32);
         for (uint64_t s0 = 0; s0 < shots; s0 += batch) {
             const uint64_t n = std::min(batch, shots - s0);
             c->d_in.ensure(n * vs);
             c->d_out.ensure(n * std::max<size_t>(out_row, 1));
             c->d_obs.ensure(n * std::max<size_t>(obs_row, 1));
-            if (c->M) {
-                if (device) {
-                    check(copy_rows_async(c->d_in.p, vs, meas + s0 * meas_stride, meas_stride, c->in_row(), n,
-                                           hipMemcpyDeviceToDevice, c->stream), "copy measurements");
-                } else {
-                    check(copy_rows_async(c->d_in.p, vs, meas + s0 * meas_stride, meas_stride, c->in_row(), n,
-                                           hipMemcpyHostToDevice, c->stream), "copy measurements");
-                }
-            }
+            if (c->M)
+                check(copy_rows_async(c->d_in.p, vs, meas + s0 * meas_stride, meas_stride, c->in_row(), n,
+                                       hipMemcpyDeviceToDevice, c->stream), "copy measurements");
             M2dParams P = c->params(n, c->d_in.as<uint8_t>(), vs, c->d_out.as<uint8_t>(), std::max<size_t>(out_row, 1),
                                     n_out, c->d_obs.as<uint8_t>(), std::max<size_t>(obs_row, 1), n_obs);
             if (sweep) {
                 c->d_sweep.ensure(n * srow);
                 check(copy_rows_async(c->d_sweep.p, srow, sweep + s0 * sweep_stride, sweep_stride, srow, n,
-                                       device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, c->stream),
-                      "copy sweep bits");
+                                       hipMemcpyDeviceToDevice, c->stream), "copy sweep bits");
                 P.sweep = c->d_sweep.as<uint8_t>();
                 P.sweep_stride = srow;
             }
             c->launch(P);
-            const hipMemcpyKind back = device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
             auto deliver = [&](DevBuf &src, size_t row, uint32_t ncols, uint8_t *dst, size_t dst_stride) {
                 if (!ncols) return;
-                const uint8_t *from = src.as<uint8_t>();
-                size_t from_stride = row, width = row;
-                if (!packed) {
-                    c->d_tmp.ensure(n * ncols);
-                    check(launch_unpack_rows(from, row, c->d_tmp.as<uint8_t>(), ncols, n, ncols, 0, c->stream), "unpack");
-                    from = c->d_tmp.as<uint8_t>();
-                    from_stride = ncols;
-                    width = ncols;
-                }
-                check(copy_rows_async(dst + s0 * dst_stride, dst_stride, from, from_stride, width, n, back, c->stream),
-                      "copy results");
-                check(hipStreamSynchronize(c->stream), "m2d");
+                check(launch_unpack_rows(src.as<uint8_t>(), row, dst + s0 * dst_stride, dst_stride, n, ncols, 0, c->stream),
+                      "unpack");
             };
             deliver(c->d_out, std::max<size_t>(out_row, 1), n_out, dets, dets_stride);
             deliver(c->d_obs, std::max<size_t>(obs_row, 1), n_obs, obs, obs_stride);

@@ -100,8 +100,10 @@ constexpr size_t MAX_LDS = LDS_PER_WORKGROUP;
 constexpr size_t HOST_BATCH_BYTES = (size_t)1 << 30;
 // Threads of the expansion's schedule: a run of records each, taken by the workgroup's lanes in turn.
 constexpr uint32_t EXPAND_THREADS = 1024;
-// Host-bound bytes per batch of a call that returns rows in host memory (one of two pipeline slots).
-constexpr size_t PIPE_BATCH_BYTES = (size_t)64 << 20;
+// Host-bound bytes per batch of a call that returns rows in host memory (one of two pipeline slots): 16 MiB, 0.3 ms of
+// the link's time, where the kernels need far less than that; 64 MiB on the frame engine, whose launches need
+// many tiles to fill the chip. Pinned memory takes about 0.1 ms per MiB to allocate on a sampler's first call.
+constexpr size_t PIPE_BATCH_BYTES = (size_t)16 << 20, PIPE_FRAME_BATCH_BYTES = (size_t)64 << 20;
 
 // Records the message of a failed C-ABI call (read back by mfs_last_error) and returns its kind.
 int record_error(const std::exception &e, int kind);
@@ -148,7 +150,7 @@ struct mfs_sampler {
     DevBuf d_classes, d_sotab, d_recs, d_ovf, d_sym_tmp, d_fix_off, d_fix_cols, d_recs32, d_ovf32, d_groups, d_thr;
     // Detector-error-model samplers: sampled site -> mechanism index, and the fired-mechanism rows of
     // the launch in progress (set only while a call returns errors).
-    DevBuf d_site_mech, d_err, d_err_tmp;
+    DevBuf d_site_mech, d_err;
     // Outcome records of the specialised scan kernel (built with the symptom table when it applies).
     DevBuf d_orecs, d_orec_base, d_orec_sites, d_orec_ovf, d_direct;
     bool sym_direct = false;     // every site has a direct entry
@@ -396,18 +398,27 @@ struct mfs_sampler {
                                                         : std::max<uint64_t>(W64, (HOST_BATCH_BYTES / std::max<size_t>(row_bytes, 1)) / W64 * W64);
         if (device_out && L.via_unpacked) batch = arena_batch(batch, L.ncols, W64);
         const bool piped = !device_out;
+        // Host rows of one byte per entry: packed rows on the device and across the link, expanded on the host (where
+        // observables in the same row start at a byte).
+        const Layout H = L;
+        const bool expand = piped && !L.packed && !((L.prepend && prog.num_observables % 8) || (L.append && prog.num_detectors % 8));
+        if (expand) {
+            L.packed = true;
+            L.det_row = (L.ncols + 7) / 8;
+            L.obs_row = (prog.num_observables + 7) / 8;
+        }
         if (piped) {
-            // Host rows travel through the pipeline: batches of about PIPE_BATCH_BYTES of host rows.
-            const size_t host_row = std::max<size_t>(L.det_row + (L.separate ? L.obs_row : 0), 1);
-            batch = std::max<uint64_t>(W64, PIPE_BATCH_BYTES / host_row / W64 * W64);
+            // Host rows travel through the pipeline: batches of about PIPE_FRAME_BATCH_BYTES of host rows.
+            const size_t host_row = std::max<size_t>(H.det_row + (L.separate ? H.obs_row : 0), 1);
+            batch = std::max<uint64_t>(W64, PIPE_FRAME_BATCH_BYTES / host_row / W64 * W64);
         }
         batch = std::min(batch, shots);
         PipeCall pipe_call{this, piped};
         if (piped) {
             const size_t dev_row = (L.via_unpacked ? L.ncols : 0) + std::max<size_t>(L.det_row, 1) +
                                    (L.separate ? std::max<size_t>(L.obs_row, 1) : 0);
-            const size_t host_row = L.det_row + (L.separate ? L.obs_row : 0);
-            pipe.begin(stream, batch * dev_row + 4 * 256, std::max<size_t>(batch * host_row, 256));
+            const size_t pin_row = L.det_row + (L.separate ? L.obs_row : 0);
+            pipe.begin(stream, batch < shots, batch * dev_row + 4 * 256, std::max<size_t>(batch * pin_row, 256));
         }
         const bool fixed = faults != nullptr;
         const uint64_t call_tile0 = tiles_used;
@@ -467,12 +478,14 @@ struct mfs_sampler {
             }
             if (piped) {
                 std::vector<HostPipe::Part> parts;
+                const uint8_t base = (uint8_t)base_char;
                 if (dets && (L.det_row || newline)) {
                     parts.push_back({det_dst, det_stride_dev, L.det_row, dets + s0 * dets_stride, dets_stride,
-                                     newline ? (long)L.ncols : -1L});
+                                     newline ? (long)L.ncols : -1L, expand ? L.ncols : 0u, base});
                 }
                 if (L.separate && obs && L.obs_row && obs_dst) {
-                    parts.push_back({obs_dst, obs_stride_dev, L.obs_row, obs + s0 * obs_stride, obs_stride, -1L});
+                    parts.push_back({obs_dst, obs_stride_dev, L.obs_row, obs + s0 * obs_stride, obs_stride, -1L,
+                                     expand ? prog.num_observables : 0u, base});
                 }
                 pipe.submit(parts, n);
             }
@@ -689,14 +702,15 @@ struct mfs_sampler {
         const uint64_t unit = std::max<uint64_t>(S, 32);
         const bool piped = !device_out;
         const size_t host_row = L.packed ? prow : M;
-        uint64_t batch = std::max<uint64_t>(unit, HOST_BATCH_BYTES / (ypitch + prow) / unit * unit);
+        // Packed device rows stage only y rows: up to 2 GiB of them (2^20 shots at d=25 in one batch instead of four).
+        const size_t staged = device_out && L.packed ? (ypitch + 1) / 2 : ypitch + prow;
+        uint64_t batch = std::max<uint64_t>(unit, HOST_BATCH_BYTES / staged / unit * unit);
         if (piped) batch = std::max<uint64_t>(unit, PIPE_BATCH_BYTES / std::max<size_t>(host_row, 1) / unit * unit);
         if (device_out) batch = arena_batch(batch, ypitch + (L.packed ? 0 : prow), unit);
         batch = std::min(batch, shots);
         PipeCall pipe_call{this, piped};
         if (piped) {
-            const size_t dev_row = ypitch + prow + (L.packed ? 0 : M);
-            pipe.begin(stream, batch * dev_row + 6 * 256, std::max<size_t>(batch * host_row, 256));
+            pipe.begin(stream, batch < shots, batch * (ypitch + prow) + 6 * 256, std::max<size_t>(batch * prow, 256));
         }
         const uint64_t d_tile0 = d.tiles_used, x_tile0 = expand_tiles;
         uint64_t d_tiles = 0;
@@ -717,17 +731,14 @@ struct mfs_sampler {
                 pd_stride = prow;
             }
             check(launch_expand(expand_params(n, y, pd, pd_stride, x_tile0 + s0 / 32), stream), "expansion launch");
-            if (!L.packed) {
-                uint8_t *ud = device_out ? out + s0 * out_stride : staging(d_tmp, n * std::max<size_t>(M, 1));
-                const size_t ud_stride = device_out ? out_stride : M;
-                check(launch_unpack_rows(pd, pd_stride, ud, ud_stride, n, M, (uint8_t)base_char, stream), "unpack");
-                pd = ud;
-                pd_stride = ud_stride;
-            }
+            if (!L.packed && device_out)
+                check(launch_unpack_rows(pd, pd_stride, out + s0 * out_stride, out_stride, n, M, (uint8_t)base_char, stream),
+                      "unpack");
             if (piped) {
+                // Bytes or characters are expanded from the bits on the host.
                 std::vector<HostPipe::Part> parts;
-                if (out) parts.push_back({pd, pd_stride, host_row, out + s0 * out_stride, out_stride,
-                                          newline ? (long)M : -1L});
+                if (out) parts.push_back({pd, pd_stride, prow, out + s0 * out_stride, out_stride, newline ? (long)M : -1L,
+                                          L.packed ? 0u : M, (uint8_t)base_char});
                 pipe.submit(parts, n);
             }
         }
@@ -1461,10 +1472,9 @@ struct mfs_sampler {
                                     (want_err ? erow : 0);
             batch = std::max<uint64_t>(S, PIPE_BATCH_BYTES / std::max<size_t>(host_row, 1) / S * S);
             batch = std::min(batch, shots);
-            const size_t dev_row = std::max<size_t>(pdet, 1) + (want_obs ? std::max<size_t>(pobs, 1) : 0) +
-                                   (L.packed ? 0 : std::max<size_t>(L.ncols + O, 1)) +
-                                   (want_err ? 4 * ew + (L.packed ? 0 : E) : 0);
-            pipe.begin(stream, batch * dev_row + 6 * 256, std::max<size_t>(batch * host_row, 256));
+            // Packed rows (bytes or characters are expanded from the bits on the host).
+            const size_t pin_row = pdet + (want_obs ? pobs : 0) + (want_err ? 4 * ew : 0);
+            pipe.begin(stream, batch < shots, batch * (pin_row + 2) + 6 * 256, std::max<size_t>(batch * pin_row, 256));
         }
         const uint64_t call_tile0 = tiles_used;
         uint64_t tiles_total = 0;
@@ -1517,13 +1527,8 @@ struct mfs_sampler {
             std::vector<HostPipe::Part> parts;
             if (want_err && E && piped) {
                 // Little-endian 32-bit words hold the bits in the packed byte order.
-                if (L.packed) {
-                    parts.push_back({err_dev, ew * 4, erow, errs + s0 * errs_stride, errs_stride, -1L});
-                } else {
-                    uint8_t *eu = staging(d_err_tmp, n * E);
-                    check(launch_unpack_rows(err_dev, ew * 4, eu, E, n, (uint32_t)E, 0, stream), "unpack error rows");
-                    parts.push_back({eu, E, E, errs + s0 * errs_stride, errs_stride, -1L});
-                }
+                parts.push_back({err_dev, ew * 4, (E + 7) / 8, errs + s0 * errs_stride, errs_stride, -1L,
+                                 L.packed ? 0u : (size_t)E});
             } else if (want_err && E) {
                 // Device rows: copied (packed) or expanded to bytes in place.
                 if (L.packed) {
@@ -1535,31 +1540,22 @@ struct mfs_sampler {
                                              stream), "unpack error rows");
                 }
             }
-            if (!L.packed) {
-                // Expand bits to bytes (bool) or characters.
-                uint8_t *ud = device_out ? dets + s0 * dets_stride : nullptr;
-                uint8_t *uo = device_out && want_obs ? obs + s0 * obs_stride : nullptr;
-                size_t ud_stride = dets_stride, uo_stride = obs_stride;
-                if (!device_out) {
-                    ud = staging(d_tmp, n * std::max<size_t>(L.ncols + O, 1));
-                    ud_stride = L.ncols;
-                    uo = ud + n * L.ncols;
-                    uo_stride = O;
-                }
-                check(launch_unpack_rows(pd, pd_stride, ud, ud_stride, n, L.ncols, (uint8_t)base_char, stream), "unpack");
-                if (want_obs) check(launch_unpack_rows(po, po_stride, uo, uo_stride, n, O, (uint8_t)base_char, stream), "unpack");
-                pd = ud;
-                pd_stride = ud_stride;
-                po = uo;
-                po_stride = uo_stride;
+            if (!L.packed && device_out) {
+                check(launch_unpack_rows(pd, pd_stride, dets + s0 * dets_stride, dets_stride, n, L.ncols, (uint8_t)base_char,
+                                         stream), "unpack");
+                if (want_obs)
+                    check(launch_unpack_rows(po, po_stride, obs + s0 * obs_stride, obs_stride, n, O, (uint8_t)base_char, stream),
+                          "unpack");
             }
             if (piped) {
-                const size_t drow = L.packed ? pdet : L.ncols, orow = L.packed ? pobs : O;
-                if (dets && (drow || newline)) {
-                    parts.push_back({pd, pd_stride, drow, dets + s0 * dets_stride, dets_stride,
-                                     newline ? (long)L.ncols : -1L});
+                const uint8_t base = (uint8_t)base_char;
+                if (dets && (pdet || newline)) {
+                    parts.push_back({pd, pd_stride, pdet, dets + s0 * dets_stride, dets_stride, newline ? (long)L.ncols : -1L,
+                                     L.packed ? 0u : (size_t)L.ncols, base});
                 }
-                if (want_obs && orow) parts.push_back({po, po_stride, orow, obs + s0 * obs_stride, obs_stride, -1L});
+                if (want_obs && pobs)
+                    parts.push_back({po, po_stride, pobs, obs + s0 * obs_stride, obs_stride, -1L, L.packed ? 0u : (size_t)O,
+                                     base});
                 pipe.submit(parts, n);
             }
         }

@@ -117,6 +117,7 @@ struct mfs_server {
     std::vector<uint64_t> active, finished;
     Arena arena;
     hipStream_t stream = nullptr;
+    HostPipe pipe;   // results on their way to host rows
     DevBuf d_jobs, d_prefix, d_counter;
     SymDevParams *h_jobs = nullptr;   // pinned staging for the work list
     uint64_t *h_prefix = nullptr;
@@ -404,13 +405,24 @@ int mfs_server_copy_result(mfs_server *v, uint64_t id, uint8_t *dets, size_t det
     return guarded([&] {
         auto &r = v->get(id);
         if (r.state != mfs_server::DONE) throw std::invalid_argument("request has not finished");
-        if (dets && r.det_row)
-            check(copy_rows_async(dets, dets_stride, r.dets, r.det_row, r.det_row, r.shots, hipMemcpyDeviceToHost,
-                                   v->stream), "copy result");
-        if (obs && r.obs_row)
-            check(copy_rows_async(obs, obs_stride, r.obs, r.obs_row, r.obs_row, r.shots, hipMemcpyDeviceToHost,
-                                   v->stream), "copy result");
-        check(hipStreamSynchronize(v->stream), "copy result");
+        // Through pinned buffers, a batch of rows at a time.
+        const size_t row = r.det_row + r.obs_row;
+        if (!row || !r.shots) return;
+        const uint64_t batch = std::min<uint64_t>(r.shots, std::max<uint64_t>(1, PIPE_BATCH_BYTES / row));
+        struct Drain {
+            HostPipe &p;
+            ~Drain() { p.drain_noexcept(); }
+        } drain{v->pipe};
+        v->pipe.begin(v->stream, batch < r.shots, 0, batch * row);
+        for (uint64_t s0 = 0; s0 < r.shots; s0 += batch) {
+            std::vector<HostPipe::Part> parts;
+            if (dets && r.det_row)
+                parts.push_back({r.dets + s0 * r.det_row, r.det_row, r.det_row, dets + s0 * dets_stride, dets_stride, -1L});
+            if (obs && r.obs_row)
+                parts.push_back({r.obs + s0 * r.obs_row, r.obs_row, r.obs_row, obs + s0 * obs_stride, obs_stride, -1L});
+            v->pipe.submit(parts, std::min(batch, r.shots - s0));
+        }
+        v->pipe.finish();
     });
 }
 

@@ -40,7 +40,8 @@ class CompiledMeasurementsToDetectionEventsConverter:
         extra = ', skip_reference_sample=True' if self._skip else ''
         return f'stim_amd.CompiledMeasurementsToDetectionEventsConverter(stim_amd.Circuit({str(self._circuit)!r}){extra})'
 
-    def _packed_measurements(self, measurements):
+    def _measurement_rows(self, measurements):
+        """Contiguous rows, one byte per result (bool) or bit-packed (uint8)."""
         m = np.asarray(measurements)
         M = self.num_measurements
         if m.ndim != 2:
@@ -48,7 +49,7 @@ class CompiledMeasurementsToDetectionEventsConverter:
         if m.dtype == np.bool_:
             if m.shape[1] != M:
                 raise ValueError(f'measurements.shape[1] != num_measurements ({m.shape[1]} != {M})')
-            return np.ascontiguousarray(np.packbits(m, axis=1, bitorder='little')) if M else np.zeros((m.shape[0], 1), np.uint8)
+            return np.ascontiguousarray(m) if M else np.zeros((m.shape[0], 1), np.uint8)
         if m.dtype == np.uint8:
             if m.shape[1] != (M + 7) // 8:
                 raise ValueError(f'bit packed measurements.shape[1] != ceil(num_measurements / 8)')
@@ -89,7 +90,7 @@ class CompiledMeasurementsToDetectionEventsConverter:
         separate = bool(separate_observables)
         append = bool(append_observables)
         packed = bool(bit_packed or bit_pack_result)
-        meas = self._packed_measurements(measurements)
+        meas = self._measurement_rows(measurements)
         shots = meas.shape[0]
         sweep = self._packed_sweep_bits(sweep_bits, shots) if sweep_bits is not None else None
         D, O = self.num_detectors, self.num_observables
@@ -98,7 +99,7 @@ class CompiledMeasurementsToDetectionEventsConverter:
         dets = np.zeros((shots, (n_out + 7) // 8 if packed else n_out), dtype=dtype)
         obs = np.zeros((shots, (O + 7) // 8 if packed else O), dtype=dtype) if separate else None
         flags = (N.MFS_BIT_PACKED if packed else 0) | (N.MFS_APPEND_OBSERVABLES if append else 0) | \
-                (N.MFS_SEPARATE_OBSERVABLES if separate else 0)
+                (N.MFS_SEPARATE_OBSERVABLES if separate else 0) | (N.MFS_BYTE_INPUT if meas.dtype == np.bool_ else 0)
         if shots:
             N.check(N.lib().mfs_m2d_convert_sweep(
                 self._h, shots, meas.ctypes.data, meas.shape[1],
