@@ -13,8 +13,7 @@
 // Layout rules the kernel relies on:
 //   * no two items of one frame op touch the same qubit (instructions are cut into segments);
 //   * record slots written by one op are contiguous (ops are cut at the ring wrap);
-//   * a frame op's words fit one LDS staging buffer (ops are capped at STAGE_WORDS words) and an
-//     epoch (ops between barriers) fits one staging buffer;
+//   * a frame op's words fit the smallest LDS staging buffer (ops are capped at OP_WORDS_MAX words);
 //   * CSR headers hold offsets relative to the op's first word.
 #include "compiler.h"
 
@@ -43,6 +42,9 @@ struct Tracker {
 };
 
 enum Kind : char { KR = 'r', KW = 'w', KA = 'a' };
+
+// LDS bytes that both staging buffers take beyond the smallest ones.
+size_t extra_bytes(uint32_t stage_words) { return 2 * (size_t)(stage_words - OP_STAGE_WORDS) * 4; }
 
 struct Builder {
     Program P;
@@ -222,6 +224,8 @@ struct Builder {
             nout = 1;
         }
         P.otab[P.otab.size() - 2] = 0xFFFFFFFFu;
+        if (nout > noise_outcomes(code)) throw std::logic_error("too many outcomes of one noise op");
+        for (uint32_t k = nout; k < noise_outcomes(code); k++) P.otab.insert(P.otab.end(), {0xFFFFFFFFu, 0u});
         uint32_t chunk_log2 = 6;
         if (p > 0 && p < 1) {
             double want = std::ceil(1.0 / p);
@@ -541,74 +545,66 @@ struct Builder {
         if (P.tgt.size() >= (1ull << 32) || P.ntgt.size() >= (1ull << 32)) {
             throw std::invalid_argument("circuit program too large");
         }
-        build_epochs();
+        build_pages(P.small);
+        P.large = P.small;
+        const uint32_t large = large_stage();
+        if (large > OP_STAGE_WORDS) {
+            P.large.stage_words = large;
+            build_pages(P.large);
+        }
     }
 
-    // Groups ops into barrier-free runs whose blob (header + op headers + words) fits one staging
-    // buffer, then packs the blobs.
-    void build_epochs() {
-        uint32_t b = 0;
-        uint64_t tbegin = 0, tend = 0;
-        bool any = false;
-        auto close = [&](uint32_t e) {
-            DevEpoch ep{};
-            ep.op_begin = b;
-            ep.op_end = e;
-            ep.tbegin = any ? (uint32_t)tbegin : 0;
-            ep.tlen = any ? (uint32_t)(tend - tbegin) : 0;
-            P.epochs.push_back(ep);
+    // Packs the ops into pages of at most set.stage_words words (program.h).
+    void build_pages(PageSet &set) {
+        const uint32_t n = (uint32_t)P.ops.size();
+        auto padded = [](uint32_t words) { return (words + 3) & ~3u; };
+        set.at = P.blob.size();
+        size_t before = 0;  // the page before the one that is laid
+        for (uint32_t b = 0; b < n;) {
+            uint32_t e = b, words = BLOB_HEADER;
+            while (e < n && padded(words + BLOB_HEADER + op_tlen[e]) <= set.stage_words) words += BLOB_HEADER + op_tlen[e++];
+            if (e == b) throw std::logic_error("an op exceeds the staging buffer");
+            const size_t at = P.blob.size();
+            const uint32_t len = padded(words);
+            P.blob.resize(at + len, 0);
+            uint32_t *page = P.blob.data() + at;
+            page[0] = e - b;
+            page[3] = b;
+            if (b) {
+                P.blob[before + 1] = (uint32_t)(at - set.at);
+                P.blob[before + 2] = len;
+            } else {
+                set.page0_len = len;
+            }
+            before = at;
+            uint32_t w = BLOB_HEADER * (1 + e - b);
+            for (uint32_t j = b; j < e; j++) {
+                DevOp op = P.ops[j];
+                std::copy_n(P.tgt.begin() + (op_tlen[j] ? op.toff : 0), op_tlen[j], page + w);
+                if (op_tlen[j] || !is_noise(op.code & 0xFF)) op.toff = op_tlen[j] ? w : 0;
+                std::memcpy(page + BLOB_HEADER * (1 + j - b), &op, sizeof(DevOp));
+                w += op_tlen[j];
+            }
             b = e;
-            any = false;
-        };
-        for (uint32_t i = 0; i < (uint32_t)P.ops.size(); i++) {
-            const uint32_t len = op_tlen[i];
-            const uint64_t s = P.ops[i].toff, e = s + len;
-            const uint64_t words = (uint64_t)BLOB_HEADER * (i - b + 2) + (len ? e - (any ? tbegin : s) : (any ? tend - tbegin : 0));
-            if (i > b && words > STAGE_WORDS) {
-                // Would overflow the staging buffer: barrier before this op.
-                if (!(P.ops[i - 1].code & OPF_SYNC)) {
-                    P.ops[i - 1].code |= OPF_SYNC;
-                    P.num_syncs++;
-                }
-                close(i);
-            }
-            if (len) {
-                if (!any) {
-                    tbegin = s;
-                    any = true;
-                }
-                tend = e;
-            }
-            if (P.ops[i].code & OPF_SYNC) close(i + 1);
         }
-        if (b < P.ops.size()) close((uint32_t)P.ops.size());
-        // Pack blobs.
-        std::vector<uint32_t> offs(P.epochs.size() + 1, 0);
-        for (size_t e = 0; e < P.epochs.size(); e++) {
-            const DevEpoch &ep = P.epochs[e];
-            offs[e + 1] = offs[e] + BLOB_HEADER * (1 + ep.op_end - ep.op_begin) + ep.tlen;
-            if (offs[e + 1] - offs[e] > STAGE_WORDS) throw std::logic_error("epoch blob exceeds the staging buffer");
-        }
-        P.blob.assign(offs.back(), 0);
-        P.blob0_len = P.epochs.empty() ? 0 : offs[1];
-        for (size_t e = 0; e < P.epochs.size(); e++) {
-            const DevEpoch &ep = P.epochs[e];
-            uint32_t *blob = P.blob.data() + offs[e];
-            const uint32_t nops = ep.op_end - ep.op_begin;
-            blob[0] = nops;
-            blob[1] = offs[e + 1];
-            blob[2] = e + 1 < P.epochs.size() ? offs[e + 2] - offs[e + 1] : 0;
-            blob[3] = ep.op_begin;
-            const uint32_t words0 = BLOB_HEADER * (1 + nops);
-            for (uint32_t j = 0; j < nops; j++) {
-                DevOp op = P.ops[ep.op_begin + j];
-                if (op_tlen[ep.op_begin + j] || !is_noise(op.code & 0xFF)) {
-                    op.toff = op_tlen[ep.op_begin + j] ? words0 + (op.toff - ep.tbegin) : 0;
-                }
-                std::memcpy(blob + BLOB_HEADER * (1 + j), &op, sizeof(DevOp));
+        if (P.blob.size() - set.at >= (1ull << 32)) throw std::invalid_argument("circuit program too large");
+    }
+
+    // Buffers of two or four times the smallest size, as far as the program fills them and every tile width that fits
+    // with the smallest still fits.
+    uint32_t large_stage() const {
+        size_t words = 0;
+        for (uint32_t t : op_tlen) words += BLOB_HEADER + t;
+        uint32_t best = OP_STAGE_WORDS;
+        for (uint32_t stage = 2 * OP_STAGE_WORDS; stage <= 4 * OP_STAGE_WORDS && words > stage / 2; stage *= 2) {
+            bool fits = true;
+            for (int t : {1, 2, 4}) {
+                const size_t bytes = tile_bytes(P, t);
+                fits = fits && (bytes > LDS_PER_WORKGROUP || bytes + extra_bytes(stage) <= LDS_PER_WORKGROUP);
             }
-            for (uint32_t k = 0; k < ep.tlen; k++) blob[words0 + k] = P.tgt[ep.tbegin + k];
+            if (fits) best = stage;
         }
+        return best;
     }
 
     static bool is_noise(uint32_t code) {
@@ -906,9 +902,26 @@ void resolve_fault(const Program &prog, uint32_t k, uint32_t j, uint32_t *op, ui
     throw std::out_of_range("instruction " + std::to_string(k) + " has no noise site " + std::to_string(j));
 }
 
-size_t lds_bytes(const Program &prog, int T) {
+size_t tile_bytes(const Program &prog, int T) {
     size_t rows = 2 * (size_t)prog.num_qubits + prog.ring + STAGE_ROWS + prog.num_observables + 1;
-    return rows * 4 * (size_t)T + 2 * STAGE_WORDS * 4;
+    return rows * 4 * (size_t)T + 2 * OP_STAGE_WORDS * 4;
+}
+
+// A tile is bound by its chain of steps: page turns, barriers, header -> words -> rows. Where the launch has a tile or two
+// to a CU, larger pages and (as an op has up to 1008 items) 512 lanes shorten that chain, and the LDS they take is free.
+// With more tiles, other tiles fill the waits, and the smallest buffers and 256 lanes let most of them run at once.
+// Measured, small | large: 5000 qubits, 20 layers, 512 tiles 0.405 | 0.313 ms; 5000 qubits, 10 layers, 4096 tiles 1.168 |
+// 1.175; surface d = 25, 256 tiles 0.661 | 0.567, 512 tiles 0.746 | 0.676, 1024 tiles 0.927 | 1.328; d = 13 (18 KB),
+// 256 tiles 0.206 | 0.202, 512 tiles 0.232 | 0.241. A tile that leaves no room for another gets 1024 lanes: 12000 qubits,
+// 5 layers, 512 tiles 0.276 ms before pages, 0.193 with them.
+FrameLaunch choose_launch(const Program &prog, int T, uint64_t tiles) {
+    constexpr uint64_t CUS = 256;
+    const size_t small = tile_bytes(prog, T), large = small + extra_bytes(prog.large.stage_words);
+    const uint64_t fit_small = LDS_PER_WORKGROUP / small, fit_large = LDS_PER_WORKGROUP / large;
+    if (fit_small <= 1) return {&prog.large, large, 1024};
+    if (prog.large.stage_words > OP_STAGE_WORDS && tiles <= CUS * std::min<uint64_t>(fit_large, fit_small <= 4 ? 2 : 1))
+        return {&prog.large, large, 512};
+    return {&prog.small, small, fit_small == 2 ? 512u : 256u};
 }
 
 }  // namespace sa

@@ -30,11 +30,6 @@ using namespace sa;
 
 namespace {
 
-// Workgroup widths: 256 lanes, or 1024 for circuits whose tile fills most of a CU's LDS (one
-// workgroup per CU), so that the CU still has 16 waves to run.
-constexpr int NT_SMALL = 256;
-constexpr int NT_LARGE = 1024;
-
 template <int T>
 struct alignas(4 * T) Wd {
     uint32_t v[T];
@@ -64,6 +59,8 @@ constexpr uint32_t TAG_RAND = 1u << 28;
 constexpr uint32_t TAG_INIT = 2u << 28;
 constexpr uint32_t TAG_DENSE = 3u << 28;
 
+__device__ __forceinline__ uint32_t scalar(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+
 struct Rng {
     uint32_t k0, k1;
     uint32_t tile;
@@ -73,12 +70,10 @@ struct Rng {
 };
 
 // Geometric gap: number of failures before the next success of a Bernoulli(p) process,
-// floor(log(u) / log(1 - p)) with u uniform in (0, 1].
-__device__ __forceinline__ uint64_t geometric_gap(uint32_t r, float inv_log2_1mp) {
-    float u = ((float)(r >> 8) + 1.0f) * (1.0f / 16777216.0f);
-    float g = __log2f(u) * inv_log2_1mp;
-    if (!(g < 1.0e12f)) return (uint64_t)1 << 40;
-    return (uint64_t)g;
+// floor(log(u) / log(1 - p)) with u uniform in (0, 1]; at most 2^30, which is past the end of every chunk.
+__device__ __forceinline__ uint32_t geometric_gap(uint32_t r, float inv_log2_1mp) {
+    const float u = ((float)(r >> 8) + 1.0f) * (1.0f / 16777216.0f);
+    return (uint32_t)fminf(__log2f(u) * inv_log2_1mp, 1073741824.0f);
 }
 
 __device__ __forceinline__ uint32_t pick_outcome(const uint32_t *otab, uint32_t woff, uint32_t nout, uint32_t r) {
@@ -201,6 +196,113 @@ __device__ void flush_rows(const uint32_t *rows, uint32_t n, uint32_t base, cons
     }
 }
 
+// One position of a sparse noise op that fired, with the words that its application needs on their way from memory.
+struct Hit {
+    uint32_t site, shot, code, a, b;
+    bool live;
+};
+
+// Sparse noise of kind CODE (NOISE1, NOISE2, MFLIP or HERALD). The tile's (site, shot) positions are cut into chunks
+// spread over all lanes (at most ~4/p positions each); each chunk walks its own geometric gaps, two hits per Philox
+// block (gap, outcome, gap, outcome). A hit needs its site's qubits and its outcome from memory: both loads of both hits
+// of a block are started together, and the next block is drawn while they are on their way. The outcome is the number
+// of thresholds below the draw; these wait in scalar registers.
+template <int T, int NT, uint32_t CODE>
+__device__ __forceinline__ void sparse_noise(const Tile<T> &t, const DevOp &op, const uint32_t *__restrict__ ntgt,
+                                             const uint32_t *__restrict__ otab, const Rng &rng, uint32_t oi,
+                                             uint32_t clog, uint64_t N) {
+    constexpr uint32_t W = 32 * T;
+    constexpr uint32_t OUTCOMES = noise_outcomes(CODE);
+    const uint32_t *__restrict__ tab = otab + op.woff;
+    const uint32_t *__restrict__ tgt = ntgt + op.toff;
+    uint32_t threshold[OUTCOMES];
+#pragma unroll
+    for (uint32_t i = 0; i + 1 < OUTCOMES; i++) threshold[i] = tab[2 * i];
+    auto fetch = [&](bool live, uint64_t pos, uint32_t r) __attribute__((always_inline)) {
+        Hit h = {0, 0, 0, 0, 0, live};
+        if (!live) return h;
+        h.site = (uint32_t)(pos / W);
+        h.shot = (uint32_t)(pos % W);
+        uint32_t k = 0;
+#pragma unroll
+        for (uint32_t i = 0; i + 1 < OUTCOMES; i++) k += r > threshold[i];
+        h.code = tab[2 * k + 1];
+        if (CODE == OP_NOISE1 || CODE == OP_HERALD) h.a = tgt[h.site];
+        if (CODE == OP_NOISE2) {
+            h.a = tgt[2 * h.site];
+            h.b = tgt[2 * h.site + 1];
+        }
+        return h;
+    };
+    auto apply = [&](Hit h) __attribute__((always_inline)) {
+        if (!h.live) return;
+        const uint32_t w = h.shot >> 5, bit = 1u << (h.shot & 31);
+        if (CODE == OP_MFLIP || CODE == OP_HERALD) {
+            uint32_t *const rec = &t.REC[(op.base + h.site) * T + w];
+            if (CODE == OP_MFLIP) {
+                if (h.code & 1) atomicXor(rec, bit);
+            } else if (h.code & 4) {
+                atomicOr(rec, bit);
+            }
+        }
+        if (CODE != OP_MFLIP) {
+            if (h.code & 1) atomicXor(&t.X[h.a * T + w], bit);
+            if (h.code & 2) atomicXor(&t.Z[h.a * T + w], bit);
+        }
+        if (CODE == OP_NOISE2) {
+            if (h.code & 4) atomicXor(&t.X[h.b * T + w], bit);
+            if (h.code & 8) atomicXor(&t.Z[h.b * T + w], bit);
+        }
+    };
+    const uint64_t nch = (N + ((uint64_t)1 << clog) - 1) >> clog;
+    for (uint64_t ch = threadIdx.x; ch < nch; ch += NT) {
+        const uint64_t lo = ch << clog;
+        const uint32_t len = (uint32_t)(N - lo < ((uint64_t)1 << clog) ? N - lo : (uint64_t)1 << clog);
+        uint32_t pos = 0, ctr = 0;
+        Hit a = {0, 0, 0, 0, 0, false}, b = a;
+        while (true) {
+            const uint4 r = rng.draw(ctr++, (uint32_t)ch, TAG_NOISE | oi);
+            const uint32_t pa = pos + geometric_gap(r.x, op.inv_log);
+            const uint32_t pb = pa + 1 + geometric_gap(r.z, op.inv_log);
+            const bool la = pa < len, lb = la && pb < len;
+            apply(a);
+            apply(b);
+            a = fetch(la, lo + pa, r.y);
+            b = fetch(lb, lo + pb, r.w);
+            pos = pb + 1;
+            if (!lb || pos >= len) break;
+        }
+        apply(a);
+        apply(b);
+    }
+}
+
+// The same for one Pauli product of a chain (OP_CORR, a single site).
+template <int T, int NT>
+__device__ __forceinline__ void sparse_chain(const Tile<T> &t, const DevOp &op, const uint32_t *__restrict__ ntgt,
+                                             const uint32_t *__restrict__ otab, const Rng &rng, uint32_t oi,
+                                             uint32_t clog, uint64_t N) {
+    constexpr uint32_t W = 32 * T;
+    const uint64_t nch = (N + ((uint64_t)1 << clog) - 1) >> clog;
+    for (uint64_t ch = threadIdx.x; ch < nch; ch += NT) {
+        const uint64_t lo = ch << clog;
+        const uint32_t len = (uint32_t)(N - lo < ((uint64_t)1 << clog) ? N - lo : (uint64_t)1 << clog);
+        uint32_t pos = 0, ctr = 0;
+        while (pos < len) {
+            const uint4 r = rng.draw(ctr++, (uint32_t)ch, TAG_NOISE | oi);
+            pos += geometric_gap(r.x, op.inv_log);
+            if (pos >= len) break;
+            apply_hit<T>(t, op, ntgt, (uint32_t)((lo + pos) / W), (uint32_t)((lo + pos) % W),
+                         pick_outcome(otab, op.woff, op.nout & 0xFFFF, r.y));
+            pos += 1 + geometric_gap(r.z, op.inv_log);
+            if (pos >= len) break;
+            apply_hit<T>(t, op, ntgt, (uint32_t)((lo + pos) / W), (uint32_t)((lo + pos) % W),
+                         pick_outcome(otab, op.woff, op.nout & 0xFFFF, r.w));
+            pos++;
+        }
+    }
+}
+
 template <int T>
 __device__ __forceinline__ Wd<T> rand_words(const Rng &rng, uint32_t op_i, uint32_t item) {
     uint4 r = rng.draw(item, op_i, TAG_RAND);
@@ -211,16 +313,147 @@ __device__ __forceinline__ Wd<T> rand_words(const Rng &rng, uint32_t op_i, uint3
     return out;
 }
 
+// The items of a Clifford op are independent (no two share a qubit), so that a lane reads the rows of several before it
+// writes the first. A lane without a further item repeats its first one: it has read the same rows, and writes the same
+// values once more, which costs less than a branch around each item.
+template <int T, int NT, uint32_t CODE, int ITEMS>
+__device__ __forceinline__ void one_qubit_items(const Tile<T> &t, const uint32_t *w, uint32_t n) {
+    for (uint32_t i = threadIdx.x; i < n; i += ITEMS * NT) {
+        uint32_t q[ITEMS];
+        Wd<T> x[ITEMS], z[ITEMS];
+#pragma unroll
+        for (int k = 0; k < ITEMS; k++) q[k] = w[i + k * NT < n ? i + k * NT : i];
+#pragma unroll
+        for (int k = 0; k < ITEMS; k++) {
+            x[k] = row<T>(t.X, q[k]);
+            z[k] = row<T>(t.Z, q[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < ITEMS; k++) {
+            if (CODE == OP_H) {
+                row<T>(t.X, q[k]) = z[k];
+                row<T>(t.Z, q[k]) = x[k];
+            }
+            if (CODE == OP_HXY) row<T>(t.Z, q[k]) = wxor(z[k], x[k]);
+            if (CODE == OP_HYZ) row<T>(t.X, q[k]) = wxor(x[k], z[k]);
+            if (CODE == OP_CXYZ) {
+                row<T>(t.X, q[k]) = wxor(x[k], z[k]);
+                row<T>(t.Z, q[k]) = x[k];
+            }
+            if (CODE == OP_CZYX) {
+                row<T>(t.X, q[k]) = z[k];
+                row<T>(t.Z, q[k]) = wxor(z[k], x[k]);
+            }
+        }
+    }
+}
+template <int T, int NT, uint32_t CODE>
+__device__ __forceinline__ void one_qubit(const Tile<T> &t, const uint32_t *w, uint32_t n) {
+    if (T > 2 || n <= NT) one_qubit_items<T, NT, CODE, 1>(t, w, n);
+    else if (n <= 2 * NT) one_qubit_items<T, NT, CODE, 2>(t, w, n);
+    else one_qubit_items<T, NT, CODE, 4>(t, w, n);
+}
+
+template <int T, uint32_t CODE>
+__device__ __forceinline__ void two_qubit_rule(Wd<T> &x1, Wd<T> &z1, Wd<T> &x2, Wd<T> &z2) {
+    switch (CODE) {
+        case OP_CX: z1 = wxor(z1, z2); x2 = wxor(x2, x1); break;
+        case OP_CY: z1 = wxor(z1, wxor(x2, z2)); z2 = wxor(z2, x1); x2 = wxor(x2, x1); break;
+        case OP_CZ: z1 = wxor(z1, x2); z2 = wxor(z2, x1); break;
+        case OP_SWAP: { Wd<T> a = x1; x1 = x2; x2 = a; a = z1; z1 = z2; z2 = a; } break;
+        case OP_ISWAP: {
+            Wd<T> dx = wxor(x1, x2);
+            Wd<T> t1 = wxor(z1, dx), t2 = wxor(z2, dx);
+            z1 = t2; z2 = t1;
+            Wd<T> a = x1; x1 = x2; x2 = a;
+        } break;
+        case OP_CXSWAP: z2 = wxor(z2, z1); z1 = wxor(z1, z2); x1 = wxor(x1, x2); x2 = wxor(x2, x1); break;
+        case OP_CZSWAP: {
+            Wd<T> a = x1; x1 = x2; x2 = a; a = z1; z1 = z2; z2 = a;
+            z1 = wxor(z1, x2); z2 = wxor(z2, x1);
+        } break;
+        case OP_SWAPCX: z1 = wxor(z1, z2); z2 = wxor(z2, z1); x2 = wxor(x2, x1); x1 = wxor(x1, x2); break;
+        case OP_SQRTXX: { Wd<T> d = wxor(z1, z2); x1 = wxor(x1, d); x2 = wxor(x2, d); } break;
+        case OP_SQRTYY: {
+            Wd<T> d = wxor(wxor(x1, z1), wxor(x2, z2));
+            x1 = wxor(x1, d); z1 = wxor(z1, d); x2 = wxor(x2, d); z2 = wxor(z2, d);
+        } break;
+        case OP_SQRTZZ: { Wd<T> d = wxor(x1, x2); z1 = wxor(z1, d); z2 = wxor(z2, d); } break;
+        case OP_XCX: x1 = wxor(x1, z2); x2 = wxor(x2, z1); break;
+        case OP_XCY: x1 = wxor(x1, wxor(x2, z2)); x2 = wxor(x2, z1); z2 = wxor(z2, z1); break;
+        case OP_YCX: x2 = wxor(x2, wxor(x1, z1)); x1 = wxor(x1, z2); z1 = wxor(z1, z2); break;
+        case OP_YCY: {
+            Wd<T> y1 = wxor(x1, z1), y2 = wxor(x2, z2);
+            x1 = wxor(x1, y2); z1 = wxor(z1, y2); x2 = wxor(x2, y1); z2 = wxor(z2, y1);
+        } break;
+        default: break;
+    }
+}
+
+template <int T, int NT, uint32_t CODE, int ITEMS>
+__device__ __forceinline__ void two_qubit_items(const Tile<T> &t, const uint32_t *w, uint32_t n) {
+    for (uint32_t i = threadIdx.x; i < n; i += ITEMS * NT) {
+        uint32_t qa[ITEMS], qb[ITEMS];
+        Wd<T> x1[ITEMS], z1[ITEMS], x2[ITEMS], z2[ITEMS];
+#pragma unroll
+        for (int k = 0; k < ITEMS; k++) {
+            const uint32_t item = i + k * NT < n ? i + k * NT : i;
+            qa[k] = w[2 * item];
+            qb[k] = w[2 * item + 1];
+        }
+#pragma unroll
+        for (int k = 0; k < ITEMS; k++) {
+            x1[k] = row<T>(t.X, qa[k]);
+            z1[k] = row<T>(t.Z, qa[k]);
+            x2[k] = row<T>(t.X, qb[k]);
+            z2[k] = row<T>(t.Z, qb[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < ITEMS; k++) {
+            two_qubit_rule<T, CODE>(x1[k], z1[k], x2[k], z2[k]);
+            row<T>(t.X, qa[k]) = x1[k];
+            row<T>(t.Z, qa[k]) = z1[k];
+            row<T>(t.X, qb[k]) = x2[k];
+            row<T>(t.Z, qb[k]) = z2[k];
+        }
+    }
+}
+template <int T, int NT, uint32_t CODE>
+__device__ __forceinline__ void two_qubit(const Tile<T> &t, const uint32_t *w, uint32_t n) {
+    if (T > 2 || n <= NT) two_qubit_items<T, NT, CODE, 1>(t, w, n);
+    else two_qubit_items<T, NT, CODE, 2>(t, w, n);
+}
+
+// An op's header in scalar registers: all lanes run the same op, so its fields steer scalar branches.
+__device__ __forceinline__ DevOp scalar_op(const uint4 &lo, const uint4 &hi) {
+    DevOp op;
+    op.code = scalar(lo.x);
+    op.n = scalar(lo.y);
+    op.toff = scalar(lo.z);
+    op.base = scalar(lo.w);
+    op.p = __uint_as_float(scalar(hi.x));
+    op.inv_log = __uint_as_float(scalar(hi.y));
+    op.woff = scalar(hi.z);
+    op.nout = scalar(hi.w);
+    return op;
+}
+
+// What bounds it is a tile's chain of dependent steps (compiler.cc, choose_launch, has the launch shapes): a launch of 63
+// tiles takes 0.83 of the time of one of 512. So ops are staged a page at a time and not from one barrier to the next
+// (5000 qubits, 20 layers: 388 page turns before, 58 with the large pages, and 97 barriers, where ops share rows), and
+// steer scalar branches; a lane handles several items of an op at once; and noise keeps its loads in flight while it
+// draws. 16384 shots of that circuit 0.548 -> 0.313 ms, of which noise takes 0.10 and the Clifford ops 0.21 (LDS
+// transfers alone: 0.07); 1000 shots of the surface code of d = 5 0.110 -> 0.072 ms; 2^18 shots of d = 25 5.06 -> 3.42 ms.
 template <int T, int NT>
 __global__ __launch_bounds__(NT) void frame_sim_kernel(const uint32_t *__restrict__ blob,
                                                        const uint32_t *__restrict__ ntgt,
                                                        const uint32_t *__restrict__ otab, LaunchParams P) {
-    extern __shared__ uint32_t lds[];
-    // LDS layout: two blob staging buffers, then the tile (frame rows, record ring, staged
-    // detector rows, observable rows, chain mask).
-    uint32_t *const STAGE = lds;
+    extern __shared__ uint4 lds4[];
+    uint32_t *const lds = reinterpret_cast<uint32_t *>(lds4);
+    // LDS layout: two staging buffers, then the tile (frame rows, record ring, staged detector rows, observable rows,
+    // chain mask).
     Tile<T> t;
-    t.X = lds + 2 * STAGE_WORDS;
+    t.X = lds + 2 * P.stage_words;
     t.Z = t.X + P.num_qubits * T;
     t.REC = t.Z + P.num_qubits * T;
     t.STG = t.REC + P.ring * T;
@@ -238,7 +471,7 @@ __global__ __launch_bounds__(NT) void frame_sim_kernel(const uint32_t *__restric
         row<T>(t.Z, i) = randomize ? rand_words<T>(rng, 0xFFFFFFFFu, i) : wzero<T>();
     }
     for (uint32_t i = tid; i < (P.num_obs + 1) * T; i += NT) t.OBS[i] = 0;
-    for (uint32_t i = tid; i < P.blob0_len; i += NT) STAGE[i] = blob[i];
+    for (uint32_t i = tid; i < P.page0_len; i += NT) lds[i] = blob[i];
     __syncthreads();
 
     uint32_t fptr = 0, fend = 0;
@@ -248,111 +481,49 @@ __global__ __launch_bounds__(NT) void frame_sim_kernel(const uint32_t *__restric
     }
 
     uint32_t buf = 0;
-    while (P.blob0_len) {
-        const uint32_t *cur = STAGE + buf * STAGE_WORDS;
-        const uint32_t n_ops = cur[0], nbeg = cur[1], nlen = cur[2], op0 = cur[3];
-        // Prefetch the next blob into registers; it lands in the other staging buffer after this
-        // epoch's ops, so its latency hides behind this epoch's work.
-        uint32_t pre[STAGE_WORDS / NT];
-#pragma unroll
-        for (uint32_t k = 0; k < STAGE_WORDS / NT; k++) {
-            const uint32_t idx = tid + k * NT;
-            pre[k] = idx < nlen ? blob[nbeg + idx] : 0u;
-        }
-        const DevOp *hdrs = reinterpret_cast<const DevOp *>(cur + BLOB_HEADER);
+    while (P.page0_len) {
+        const uint32_t *cur = lds + buf * P.stage_words;
+        const uint4 head = *reinterpret_cast<const uint4 *>(cur);
+        const uint32_t n_ops = scalar(head.x), nbeg = scalar(head.y), nlen = scalar(head.z), op0 = scalar(head.w);
+        // Prefetch the next page into registers (a lane takes at most two pieces: stage_words <= 8 * NT); it lands in
+        // the other staging buffer after this page's ops, so its latency hides behind their work.
+        const uint4 *const next = reinterpret_cast<const uint4 *>(blob + nbeg);
+        uint4 pre0 = make_uint4(0, 0, 0, 0), pre1 = pre0;
+        if (4 * tid < nlen) pre0 = next[tid];
+        if (4 * (tid + NT) < nlen) pre1 = next[tid + NT];
+        const uint4 *hdrs = reinterpret_cast<const uint4 *>(cur + BLOB_HEADER);
+        uint4 next_lo = hdrs[0], next_hi = hdrs[1];
 
         for (uint32_t j = 0; j < n_ops; j++) {
-            const DevOp op = hdrs[j];
+            const DevOp op = scalar_op(next_lo, next_hi);
+            const uint32_t nj = j + 1 < n_ops ? j + 1 : j;
+            next_lo = hdrs[2 * nj];
+            next_hi = hdrs[2 * nj + 1];
             const uint32_t oi = op0 + j;
             const uint32_t code = op.code & 0xFF;
             const bool rnd = randomize && (op.code & OPF_RANDOMIZE);
             const uint32_t *w = cur + op.toff;
             switch (code) {
-                case OP_H:
-                    for (uint32_t i = tid; i < op.n; i += NT) {
-                        const uint32_t q = w[i];
-                        Wd<T> x = row<T>(t.X, q), z = row<T>(t.Z, q);
-                        row<T>(t.X, q) = z;
-                        row<T>(t.Z, q) = x;
-                    }
-                    break;
-                case OP_HXY:
-                    for (uint32_t i = tid; i < op.n; i += NT) {
-                        const uint32_t q = w[i];
-                        row<T>(t.Z, q) = wxor(row<T>(t.Z, q), row<T>(t.X, q));
-                    }
-                    break;
-                case OP_HYZ:
-                    for (uint32_t i = tid; i < op.n; i += NT) {
-                        const uint32_t q = w[i];
-                        row<T>(t.X, q) = wxor(row<T>(t.X, q), row<T>(t.Z, q));
-                    }
-                    break;
-                case OP_CXYZ:
-                    for (uint32_t i = tid; i < op.n; i += NT) {
-                        const uint32_t q = w[i];
-                        Wd<T> x = row<T>(t.X, q), z = row<T>(t.Z, q);
-                        x = wxor(x, z);
-                        z = wxor(z, x);
-                        row<T>(t.X, q) = x;
-                        row<T>(t.Z, q) = z;
-                    }
-                    break;
-                case OP_CZYX:
-                    for (uint32_t i = tid; i < op.n; i += NT) {
-                        const uint32_t q = w[i];
-                        Wd<T> x = row<T>(t.X, q), z = row<T>(t.Z, q);
-                        z = wxor(z, x);
-                        x = wxor(x, z);
-                        row<T>(t.X, q) = x;
-                        row<T>(t.Z, q) = z;
-                    }
-                    break;
-                case OP_CX: case OP_CY: case OP_CZ: case OP_SWAP: case OP_ISWAP: case OP_CXSWAP: case OP_CZSWAP:
-                case OP_SWAPCX: case OP_SQRTXX: case OP_SQRTYY: case OP_SQRTZZ: case OP_XCX: case OP_XCY:
-                case OP_YCX: case OP_YCY:
-                    for (uint32_t i = tid; i < op.n; i += NT) {
-                        const uint32_t qa = w[2 * i], qb = w[2 * i + 1];
-                        Wd<T> x1 = row<T>(t.X, qa), z1 = row<T>(t.Z, qa);
-                        Wd<T> x2 = row<T>(t.X, qb), z2 = row<T>(t.Z, qb);
-                        switch (code) {
-                            case OP_CX: z1 = wxor(z1, z2); x2 = wxor(x2, x1); break;
-                            case OP_CY: z1 = wxor(z1, wxor(x2, z2)); z2 = wxor(z2, x1); x2 = wxor(x2, x1); break;
-                            case OP_CZ: z1 = wxor(z1, x2); z2 = wxor(z2, x1); break;
-                            case OP_SWAP: { Wd<T> a = x1; x1 = x2; x2 = a; a = z1; z1 = z2; z2 = a; } break;
-                            case OP_ISWAP: {
-                                Wd<T> dx = wxor(x1, x2);
-                                Wd<T> t1 = wxor(z1, dx), t2 = wxor(z2, dx);
-                                z1 = t2; z2 = t1;
-                                Wd<T> a = x1; x1 = x2; x2 = a;
-                            } break;
-                            case OP_CXSWAP: z2 = wxor(z2, z1); z1 = wxor(z1, z2); x1 = wxor(x1, x2); x2 = wxor(x2, x1); break;
-                            case OP_CZSWAP: {
-                                Wd<T> a = x1; x1 = x2; x2 = a; a = z1; z1 = z2; z2 = a;
-                                z1 = wxor(z1, x2); z2 = wxor(z2, x1);
-                            } break;
-                            case OP_SWAPCX: z1 = wxor(z1, z2); z2 = wxor(z2, z1); x2 = wxor(x2, x1); x1 = wxor(x1, x2); break;
-                            case OP_SQRTXX: { Wd<T> d = wxor(z1, z2); x1 = wxor(x1, d); x2 = wxor(x2, d); } break;
-                            case OP_SQRTYY: {
-                                Wd<T> d = wxor(wxor(x1, z1), wxor(x2, z2));
-                                x1 = wxor(x1, d); z1 = wxor(z1, d); x2 = wxor(x2, d); z2 = wxor(z2, d);
-                            } break;
-                            case OP_SQRTZZ: { Wd<T> d = wxor(x1, x2); z1 = wxor(z1, d); z2 = wxor(z2, d); } break;
-                            case OP_XCX: x1 = wxor(x1, z2); x2 = wxor(x2, z1); break;
-                            case OP_XCY: x1 = wxor(x1, wxor(x2, z2)); x2 = wxor(x2, z1); z2 = wxor(z2, z1); break;
-                            case OP_YCX: x2 = wxor(x2, wxor(x1, z1)); x1 = wxor(x1, z2); z1 = wxor(z1, z2); break;
-                            case OP_YCY: {
-                                Wd<T> y1 = wxor(x1, z1), y2 = wxor(x2, z2);
-                                x1 = wxor(x1, y2); z1 = wxor(z1, y2); x2 = wxor(x2, y1); z2 = wxor(z2, y1);
-                            } break;
-                            default: break;
-                        }
-                        row<T>(t.X, qa) = x1;
-                        row<T>(t.Z, qa) = z1;
-                        row<T>(t.X, qb) = x2;
-                        row<T>(t.Z, qb) = z2;
-                    }
-                    break;
+                case OP_H: one_qubit<T, NT, OP_H>(t, w, op.n); break;
+                case OP_HXY: one_qubit<T, NT, OP_HXY>(t, w, op.n); break;
+                case OP_HYZ: one_qubit<T, NT, OP_HYZ>(t, w, op.n); break;
+                case OP_CXYZ: one_qubit<T, NT, OP_CXYZ>(t, w, op.n); break;
+                case OP_CZYX: one_qubit<T, NT, OP_CZYX>(t, w, op.n); break;
+                case OP_CX: two_qubit<T, NT, OP_CX>(t, w, op.n); break;
+                case OP_CY: two_qubit<T, NT, OP_CY>(t, w, op.n); break;
+                case OP_CZ: two_qubit<T, NT, OP_CZ>(t, w, op.n); break;
+                case OP_SWAP: two_qubit<T, NT, OP_SWAP>(t, w, op.n); break;
+                case OP_ISWAP: two_qubit<T, NT, OP_ISWAP>(t, w, op.n); break;
+                case OP_CXSWAP: two_qubit<T, NT, OP_CXSWAP>(t, w, op.n); break;
+                case OP_CZSWAP: two_qubit<T, NT, OP_CZSWAP>(t, w, op.n); break;
+                case OP_SWAPCX: two_qubit<T, NT, OP_SWAPCX>(t, w, op.n); break;
+                case OP_SQRTXX: two_qubit<T, NT, OP_SQRTXX>(t, w, op.n); break;
+                case OP_SQRTYY: two_qubit<T, NT, OP_SQRTYY>(t, w, op.n); break;
+                case OP_SQRTZZ: two_qubit<T, NT, OP_SQRTZZ>(t, w, op.n); break;
+                case OP_XCX: two_qubit<T, NT, OP_XCX>(t, w, op.n); break;
+                case OP_XCY: two_qubit<T, NT, OP_XCY>(t, w, op.n); break;
+                case OP_YCX: two_qubit<T, NT, OP_YCX>(t, w, op.n); break;
+                case OP_YCY: two_qubit<T, NT, OP_YCY>(t, w, op.n); break;
                 case OP_FEEDBACK:
                     for (uint32_t i = tid; i < op.n; i += NT) {
                         const uint32_t slot = w[3 * i], q = w[3 * i + 1], mask = w[3 * i + 2];
@@ -526,46 +697,34 @@ __global__ __launch_bounds__(NT) void frame_sim_kernel(const uint32_t *__restric
                         }
                         break;
                     }
-                    // The tile's (site, shot) positions are cut into chunks spread over all lanes (at
-                    // most ~4/p positions each); each chunk walks its own geometric gaps, two hits per
-                    // Philox block (gap, outcome, gap, outcome).
                     const uint64_t N = (uint64_t)op.n * W;
+                    // Chunks of 64 positions or more, up to 2^(cmax + 2), so that there are at most 2^chunk_log of them if that allows it.
                     const uint32_t cmax = (op.nout >> 16) & 0xFF;
-                    uint32_t clog = 6;
-                    while (clog < cmax + 2 && ((uint64_t)NT << clog) < N) clog++;
-                    const uint64_t C = (uint64_t)1 << clog;
-                    const uint64_t nch = (N + C - 1) >> clog;
-                    for (uint64_t ch = tid; ch < nch; ch += NT) {
-                        const uint64_t lo = ch << clog;
-                        const uint64_t hi = lo + C < N ? lo + C : N;
-                        uint64_t pos = lo;
-                        uint32_t ctr = 0;
-                        while (true) {
-                            const uint4 r = rng.draw(ctr++, (uint32_t)ch, TAG_NOISE | oi);
-                            pos += geometric_gap(r.x, op.inv_log);
-                            if (pos >= hi) break;
-                            apply_hit<T>(t, op, ntgt, (uint32_t)(pos / W), (uint32_t)(pos % W),
-                                         pick_outcome(otab, op.woff, nout, r.y));
-                            pos += 1 + geometric_gap(r.z, op.inv_log);
-                            if (pos >= hi) break;
-                            apply_hit<T>(t, op, ntgt, (uint32_t)(pos / W), (uint32_t)(pos % W),
-                                         pick_outcome(otab, op.woff, nout, r.w));
-                            pos++;
-                        }
+                    const uint64_t each = (N + (1u << P.chunk_log) - 1) >> P.chunk_log;
+                    const uint32_t clog = min(cmax + 2, max(6u, each > 1 ? 64u - (uint32_t)__clzll(each - 1) : 0u));
+                    if (code == OP_NOISE1) {
+                        sparse_noise<T, NT, OP_NOISE1>(t, op, ntgt, otab, rng, oi, clog, N);
+                    } else if (code == OP_NOISE2) {
+                        sparse_noise<T, NT, OP_NOISE2>(t, op, ntgt, otab, rng, oi, clog, N);
+                    } else if (code == OP_MFLIP) {
+                        sparse_noise<T, NT, OP_MFLIP>(t, op, ntgt, otab, rng, oi, clog, N);
+                    } else if (code == OP_HERALD) {
+                        sparse_noise<T, NT, OP_HERALD>(t, op, ntgt, otab, rng, oi, clog, N);
+                    } else {
+                        sparse_chain<T, NT>(t, op, ntgt, otab, rng, oi, clog, N);
                     }
                     break;
                 }
                 default:
                     break;
             }
+            // The last op of a page has the page turn's barrier.
+            if ((op.code & OPF_SYNC) && j + 1 < n_ops) __syncthreads();
         }
         if (nlen == 0) break;
-        uint32_t *nst = STAGE + (buf ^ 1) * STAGE_WORDS;
-#pragma unroll
-        for (uint32_t k = 0; k < STAGE_WORDS / NT; k++) {
-            const uint32_t idx = tid + k * NT;
-            if (idx < nlen) nst[idx] = pre[k];
-        }
+        uint4 *nst = reinterpret_cast<uint4 *>(lds + (buf ^ 1) * P.stage_words);
+        if (4 * tid < nlen) nst[tid] = pre0;
+        if (4 * (tid + NT) < nlen) nst[tid + NT] = pre1;
         __syncthreads();
         buf ^= 1;
     }
@@ -593,29 +752,29 @@ __global__ void pack_rows_kernel(const uint8_t *src, size_t src_stride, uint8_t 
 namespace sa {
 
 hipError_t launch_frame_kernel(int T, const DevProgram &prog, const LaunchParams &P, uint32_t num_tiles, size_t lds,
-                               hipStream_t stream) {
+                               uint32_t lanes, hipStream_t stream) {
     if (num_tiles == 0) return hipSuccess;
-    // A tile of more than 64 KB leaves room for at most two workgroups per CU: use the wide workgroup.
-    const bool wide = lds > 64 * 1024;
-    dim3 grid(num_tiles), block(wide ? NT_LARGE : NT_SMALL);
-#define STIM_AMD_LAUNCH(TW, NB)                                                                                 \
-    {                                                                                                           \
-        static size_t reserved = 0;                                                                             \
-        const hipError_t e = reserve_lds((const void *)frame_sim_kernel<TW, NB>, lds, reserved);                \
-        if (e != hipSuccess) return e;                                                                          \
-    }                                                                                                           \
-    hipLaunchKernelGGL((frame_sim_kernel<TW, NB>), grid, block, lds, stream, prog.blob, prog.ntgt, prog.otab, P);
-    switch (T * 2 + (wide ? 1 : 0)) {
-        case 2: STIM_AMD_LAUNCH(1, NT_SMALL) break;
-        case 3: STIM_AMD_LAUNCH(1, NT_LARGE) break;
-        case 4: STIM_AMD_LAUNCH(2, NT_SMALL) break;
-        case 5: STIM_AMD_LAUNCH(2, NT_LARGE) break;
-        case 8: STIM_AMD_LAUNCH(4, NT_SMALL) break;
-        case 9: STIM_AMD_LAUNCH(4, NT_LARGE) break;
-        default: return hipErrorInvalidValue;
+    if (P.stage_words > 8 * lanes) return hipErrorInvalidValue;
+#define STIM_AMD_LAUNCH(TW, NB)                                                                                   \
+    if (T == TW && lanes == NB) {                                                                                 \
+        static size_t reserved = 0;                                                                               \
+        const hipError_t e = reserve_lds((const void *)frame_sim_kernel<TW, NB>, lds, reserved);                  \
+        if (e != hipSuccess) return e;                                                                            \
+        hipLaunchKernelGGL((frame_sim_kernel<TW, NB>), dim3(num_tiles), dim3(NB), lds, stream, prog.blob,         \
+                           prog.ntgt, prog.otab, P);                                                              \
+        return hipGetLastError();                                                                                 \
     }
+    STIM_AMD_LAUNCH(1, 256)
+    STIM_AMD_LAUNCH(1, 512)
+    STIM_AMD_LAUNCH(1, 1024)
+    STIM_AMD_LAUNCH(2, 256)
+    STIM_AMD_LAUNCH(2, 512)
+    STIM_AMD_LAUNCH(2, 1024)
+    STIM_AMD_LAUNCH(4, 256)
+    STIM_AMD_LAUNCH(4, 512)
+    STIM_AMD_LAUNCH(4, 1024)
 #undef STIM_AMD_LAUNCH
-    return hipGetLastError();
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_pack_rows(const uint8_t *src, size_t src_stride, uint8_t *dst, size_t dst_stride, uint64_t rows,

@@ -63,7 +63,7 @@ constexpr uint32_t TERM_QMASK = (1u << 24) - 1;
 struct DevOp {
     uint32_t code;   // opcode | flags
     uint32_t n;      // items (sites for noise ops)
-    uint32_t toff;   // frame ops: word offset in the epoch blob; noise ops: offset into ntgt
+    uint32_t toff;   // frame ops: word offset in the page; noise ops: offset into ntgt
     uint32_t base;   // record slot base / detector base / term count (CORR)
     float p;         // total firing probability (noise)
     float inv_log;   // 1 / log2(1 - p) for geometric gaps (noise)
@@ -73,25 +73,31 @@ struct DevOp {
 static_assert(sizeof(DevOp) == 32, "DevOp layout");
 
 // A run of ops with no barrier inside (host bookkeeping).
-struct DevEpoch {
-    uint32_t op_begin, op_end;
-    uint32_t tbegin, tlen;
-};
+// Entries of a noise op's outcome table, at least: it is filled up with thresholds that no draw exceeds, so that the
+// kernel compares with all of them at once.
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+constexpr uint32_t noise_outcomes(uint32_t code) {
+    return code == OP_NOISE2 ? 16 : code == OP_NOISE1 || code == OP_HERALD ? 4 : 1;
+}
 
-// The device walks the program as a chain of epoch blobs. Blob layout (32-bit words):
-//   [0] ops in this epoch  [1] word offset of the next blob  [2] its length (0: last)
-//   [3] global index of this epoch's first op  [4..7] unused
+// The device walks the program as a chain of pages. A page holds as many successive ops as one staging buffer takes,
+// whatever barriers lie between them. Page layout (32-bit words):
+//   [0] ops in this page  [1] word offset of the next page  [2] its length (0: last)
+//   [3] global index of this page's first op  [4..7] unused
 //   [8 .. 8 + 8*ops)        DevOp headers
-//   [8 + 8*ops .. len)      the frame ops' words (targets, CSR lists); DevOp::toff is relative
-//                           to the blob start.
-// Each blob is copied into one of two LDS staging buffers while the previous epoch runs, so the
-// op loop reads headers and targets from LDS only.
+//   [8 + 8*ops .. len)      the frame ops' words (targets, CSR lists); DevOp::toff is relative to the page's start.
+// Lengths are multiples of four words. Each page is copied into one of two LDS staging buffers while the page before it
+// runs, so the op loop reads headers and targets from LDS only.
 // LDS one workgroup may use on gfx950.
 constexpr uint32_t LDS_PER_WORKGROUP = 160 * 1024;
 
 constexpr uint32_t BLOB_HEADER = 8;
-constexpr uint32_t STAGE_WORDS = 1024;  // staged words per epoch blob (4 KB; double-buffered)
-constexpr uint32_t OP_WORDS_MAX = STAGE_WORDS - 2 * BLOB_HEADER;  // words of one frame op
+// Staging buffers hold 1024 words (4 KB), or twice or four times that where the tile leaves the room (compiler.cc). An op
+// fits the smallest: where instructions are cut into ops fixes the numbering of the random streams.
+constexpr uint32_t OP_STAGE_WORDS = 1024;
+constexpr uint32_t OP_WORDS_MAX = OP_STAGE_WORDS - 2 * BLOB_HEADER;  // words of one frame op
 
 constexpr uint32_t STAGE_ROWS = 256;   // detectors staged per flush
 
@@ -121,7 +127,9 @@ struct LaunchParams {
     uint64_t seed;
     uint64_t shots;            // valid shots in this launch
     uint64_t tile0;            // global tile index of block 0 (RNG stream)
-    uint32_t blob0_len;        // length of the first epoch blob (it starts at word 0)
+    uint32_t page0_len;        // length of the first page (it starts at word 0)
+    uint32_t stage_words;      // words of one staging buffer
+    uint32_t chunk_log;        // log2 of the chunks that a noise op's positions are cut into (fixes the noise streams)
     uint32_t num_qubits;       // dense qubit rows
     uint32_t ring;             // record ring rows
     uint32_t num_obs;
@@ -132,7 +140,7 @@ struct LaunchParams {
 
 // Device-resident program buffers.
 struct DevProgram {
-    const uint32_t *blob;      // epoch blobs
+    const uint32_t *blob;      // pages
     const uint32_t *ntgt;      // noise-op words (read on hits)
     const uint32_t *otab;      // outcome table (threshold, code) pairs
 };

@@ -311,7 +311,7 @@ int mfs_parse_stats(const char *stim_text, size_t len, uint64_t out[10]) {
         out[6] = prog.num_syncs;
         out[7] = prog.num_noise_ops;
         out[8] = prog.ring;
-        out[9] = lds_bytes(prog, 2);
+        out[9] = tile_bytes(prog, 2);
     });
 }
 

@@ -34,7 +34,7 @@
 
 namespace sa {
 hipError_t launch_frame_kernel(int T, const DevProgram &prog, const LaunchParams &P, uint32_t num_tiles, size_t lds,
-                               hipStream_t stream);
+                               uint32_t lanes, hipStream_t stream);
 hipError_t launch_pack_rows(const uint8_t *src, size_t src_stride, uint8_t *dst, size_t dst_stride, uint64_t rows,
                             uint32_t ncols, hipStream_t stream);
 hipError_t launch_sym_sample(const SymDevParams &P, uint32_t tiles, size_t lds, hipStream_t stream);
@@ -259,25 +259,25 @@ struct mfs_sampler {
 
     void pick_tile_words(int want) {
         if (want) {
-            size_t need = lds_bytes(prog, want);
-            if (need > MAX_LDS) throw std::invalid_argument("tile does not fit in LDS for this circuit");
+            if (tile_bytes(prog, want) > MAX_LDS) throw std::invalid_argument("tile does not fit in LDS for this circuit");
             T = want;
-        } else if (lds_bytes(prog, 2) <= 64 * 1024) {
+        } else if (tile_bytes(prog, 2) <= FRAME_T2_BYTES) {
             T = 2;
-        } else if (lds_bytes(prog, 1) <= MAX_LDS) {
+        } else if (tile_bytes(prog, 1) <= MAX_LDS) {
             T = 1;
         } else {
             throw std::invalid_argument(
                 "circuit's frame does not fit in LDS (" + std::to_string(prog.num_qubits) + " qubits, record ring " +
                 std::to_string(prog.ring) + " rows)");
         }
-        lds = lds_bytes(prog, T);
+        lds = tile_bytes(prog, T);
     }
 
     LaunchParams base_params() {
         LaunchParams P{};
         P.seed = key;
-        P.blob0_len = prog.blob0_len;
+        // 256 chunks, or 1024 where the tile takes more than 64 KB.
+        P.chunk_log = tile_bytes(prog, T) > 64 * 1024 ? 10 : 8;
         P.num_qubits = prog.num_qubits;
         P.ring = prog.ring;
         P.num_obs = prog.num_observables;
@@ -285,10 +285,13 @@ struct mfs_sampler {
         return P;
     }
 
-    void launch(const LaunchParams &P, uint64_t tiles) {
+    void launch(LaunchParams P, uint64_t tiles) {
         if (tiles >= (1ull << 31)) throw std::invalid_argument("too many shots in one launch");
-        DevProgram dp{d_blob.as<uint32_t>(), d_ntgt.as<uint32_t>(), d_otab.as<uint32_t>()};
-        check(launch_frame_kernel(T, dp, P, (uint32_t)tiles, lds, stream), "frame kernel launch");
+        const FrameLaunch how = choose_launch(prog, T, tiles);
+        P.page0_len = how.pages->page0_len;
+        P.stage_words = how.pages->stage_words;
+        DevProgram dp{d_blob.as<uint32_t>() + how.pages->at, d_ntgt.as<uint32_t>(), d_otab.as<uint32_t>()};
+        check(launch_frame_kernel(T, dp, P, (uint32_t)tiles, how.lds, how.lanes, stream), "frame kernel launch");
     }
 
     // Output layout of one sample call.
