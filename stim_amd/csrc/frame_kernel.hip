@@ -277,7 +277,8 @@ __device__ __forceinline__ void sparse_noise(const Tile<T> &t, const DevOp &op, 
     }
 }
 
-// The same for one Pauli product of a chain (OP_CORR, a single site).
+// The same for one Pauli product of a chain (OP_CORR, a single site). No barrier parts the products of a chain: sampled
+// sparsely or densely, all of them run on the first wave, in order.
 template <int T, int NT>
 __device__ __forceinline__ void sparse_chain(const Tile<T> &t, const DevOp &op, const uint32_t *__restrict__ ntgt,
                                              const uint32_t *__restrict__ otab, const Rng &rng, uint32_t oi,

@@ -127,6 +127,40 @@ __device__ __forceinline__ void store_rows(uint32_t (&x)[32], uint8_t *base, uin
     }
 }
 
+// Rows on lanes: a half-wave's lane loads, or stores, the word of its own row (row < valid) of one block. For launches so
+// small that a lane per block leaves most of the chip idle (launch_m2d, rows_on_lanes).
+__device__ __forceinline__ uint32_t load_row(const uint8_t *r, uint32_t row_bytes, uint32_t b, bool exact) {
+    if (exact && row_bytes < 4) {
+        uint32_t v = 0;
+        for (uint32_t k = 0; k < row_bytes; k++) v |= (uint32_t)r[k] << (8 * k);
+        return v;
+    }
+    const uint32_t at = exact && 4 * b + 4 > row_bytes ? row_bytes - 4 : 4 * b;
+    return *reinterpret_cast<const unaligned_u32 *>(r + at) >> (8 * (4 * b - at));
+}
+__device__ __forceinline__ void store_row(uint32_t v, uint8_t *r, uint32_t row_bytes, uint32_t b) {
+    const uint32_t left = row_bytes - 4 * b;
+    r += 4 * b;
+    if (left >= 4) {
+        *reinterpret_cast<unaligned_u32 *>(r) = v;
+    } else {
+        r[0] = (uint8_t)v;
+        if (left > 1) r[1] = (uint8_t)(v >> 8);
+        if (left > 2) r[2] = (uint8_t)(v >> 16);
+    }
+}
+// Loads row blocks [0, blocks) of each subtile into its words from word `at` on.
+__device__ __forceinline__ void load_by_rows(uint32_t *words, uint32_t subw, uint32_t at, const uint8_t *in,
+                                             uint64_t stride, uint32_t row_bytes, uint32_t blocks, bool exact,
+                                             uint32_t shots) {
+    const uint32_t lane = threadIdx.x & 31, subs = (shots + 31) / 32;
+    for (uint32_t i = threadIdx.x >> 5; i < subs * blocks; i += M2D_NT / 32) {
+        const uint32_t t = i / blocks, b = i - t * blocks;
+        const uint32_t x = load_row(in + min(32 * t + lane, shots - 1) * stride, row_bytes, b, exact);
+        words[t * subw + at + 33 * b + lane] = transpose32(x, lane);
+    }
+}
+
 // XOR of a column's words (first and second plane entries a, b; column `col` when listed).
 // (a word's LDS address, base + 4 * index, is one multiply-add of a 16-bit half of the entry).
 __device__ __forceinline__ uint32_t terms_word(const uint32_t *w, uint32_t a) {
@@ -182,7 +216,7 @@ __device__ __forceinline__ void store_observables(const M2dParams &P, const uint
 // rather than rows on lanes (32x32 transposes across half-waves, output staged in LDS 64 blocks at a time) take
 // 0.96 instead of 1.53 ms per 2^20 shots at d=25 (4.3 TB/s); without its loads and stores the kernel takes 0.52.
 // Resident workgroups that prefetch the next tile's rows spill and wait for their stores: 2.1 ms.
-template <bool SLOW>
+template <bool SLOW, bool ROWS>
 __global__ __launch_bounds__(M2D_NT, 4) void m2d_kernel(M2dParams P) {
     extern __shared__ __align__(16) uint32_t words[];
     const uint32_t tid = threadIdx.x, G = P.group;
@@ -200,7 +234,8 @@ __global__ __launch_bounds__(M2D_NT, 4) void m2d_kernel(M2dParams P) {
 
     // Rows whose stride covers whole words are read past their last byte (never past the buffer's
     // shots * stride bytes); the bits there belong to no measurement.
-    for (uint32_t i = tid; i < subs * P.blocks; i += M2D_NT) {
+    if (ROWS) load_by_rows(words, subw, 0, P.in + s0 * P.in_stride, P.in_stride, P.in_row_bytes, P.blocks, !P.in_vec, shots);
+    for (uint32_t i = tid; !ROWS && i < subs * P.blocks; i += M2D_NT) {
         const uint32_t t = i / P.blocks, b = i - t * P.blocks;
         uint32_t x[32];
         load_rows(x, P.in + s0 * P.in_stride, P.in_stride, 32 * t * (uint32_t)P.in_stride, P.in_row_bytes, b, !P.in_vec,
@@ -212,7 +247,11 @@ __global__ __launch_bounds__(M2D_NT, 4) void m2d_kernel(M2dParams P) {
     }
     if (P.sweep_blocks) {
         const uint32_t sw0 = m2d_padded(m2d_sweep_word(P.blocks));
-        for (uint32_t i = tid; i < subs * P.sweep_blocks; i += M2D_NT) {
+        const bool by_rows = ROWS && P.sweep;
+        if (by_rows)
+            load_by_rows(words, subw, sw0, P.sweep + s0 * P.sweep_stride, P.sweep_stride, P.sweep_row_bytes,
+                         P.sweep_blocks, true, shots);
+        for (uint32_t i = tid; !by_rows && i < subs * P.sweep_blocks; i += M2D_NT) {
             const uint32_t t = i / P.sweep_blocks, b = i - t * P.sweep_blocks;
             uint32_t x[32];
 #pragma unroll
@@ -239,7 +278,22 @@ __global__ __launch_bounds__(M2D_NT, 4) void m2d_kernel(M2dParams P) {
     }
 
     const uint32_t nb = (P.n_out + 31) / 32, TB = P.total_blocks;
-    for (uint32_t i = tid; i < subs * nb; i += M2D_NT) {
+    const uint32_t lane = tid & 31;
+    for (uint32_t i = tid >> 5; ROWS && i < subs * nb; i += M2D_NT / 32) {
+        const uint32_t t = i / nb, b = i - t * nb;
+        const uint32_t *const w = words + t * subw;
+        const uint2 info = P.block_info[b];
+        const uint32_t a = (P.terms + (size_t)lane * TB)[b];
+        uint32_t x;
+        if (SLOW && a == 0xFFFFFFFFu) x = listed_word(P, w, 32 * b + lane);
+        else x = terms_word(w, a);
+        if (info.y) x ^= terms_word(w, (P.terms + (size_t)(32 + lane) * TB)[b]);
+        x = transpose32(x, lane) ^ info.x;
+        const uint32_t live = P.n_out - 32 * b;
+        if (live < 32) x &= (1u << live) - 1;
+        if (32 * t + lane < shots) store_row(x, P.out + (s0 + 32 * t + lane) * P.out_stride, (P.n_out + 7) / 8, b);
+    }
+    for (uint32_t i = tid; !ROWS && i < subs * nb; i += M2D_NT) {
         const uint32_t t = i / nb, b = i - t * nb;
         const uint32_t *const w = words + t * subw;
         const uint2 info = P.block_info[b];
@@ -337,7 +391,7 @@ __device__ __forceinline__ void expand_record(uint32_t *words, uint4 r, uint4 q)
 // 1.32 ms (3.2 TB/s of y rows read and record rows written), of which the steps are about 0.45; with rows on
 // lanes, staged output and 1024-lane workgroups 1.76.
 // ONE: one subtile per workgroup (no divisions by the counts).
-template <bool ONE>
+template <bool ONE, bool ROWS>
 __global__ __launch_bounds__(M2D_NT, 4) void expand_kernel(ExpandDev E) {
     extern __shared__ __align__(16) uint32_t words[];
     const M2dParams &P = E.out;
@@ -363,7 +417,7 @@ __global__ __launch_bounds__(M2D_NT, 4) void expand_kernel(ExpandDev E) {
 #pragma unroll
         for (uint32_t k = 0; k < 16; k++) slot[k] = (E.prim + (size_t)k * E.y_blocks)[b];
     };
-    if (tid < subs * E.y_blocks) load_block(tid);
+    if (!ROWS && tid < subs * E.y_blocks) load_block(tid);
     const uint32_t step0 = E.nsteps ? E.steps[1] : 0, staged = E.staged;
     // Step 0's records of this lane: tid and tid + M2D_NT.
     uint4 ra, qa, rb, qb;
@@ -396,7 +450,18 @@ __global__ __launch_bounds__(M2D_NT, 4) void expand_kernel(ExpandDev E) {
         w[at.w] = r.w;
     }
     // y words into their slots (two 16-bit padded indices per entry; columns past the last go to the spare word).
-    for (uint32_t i = tid; i < subs * E.y_blocks; i += M2D_NT) {
+    const uint32_t lane = tid & 31;
+    for (uint32_t i = tid >> 5; ROWS && i < subs * E.y_blocks; i += M2D_NT / 32) {
+        uint32_t t;
+        const uint32_t b = split(i, E.y_blocks, t), y = 32 * b + lane;
+        uint32_t v = load_row(E.in + (s0 + min(32 * t + lane, shots - 1)) * E.in_stride, 0, b, false);
+        v = transpose32(v, lane);
+        uint32_t *const w = words + t * subw;
+        atomicXor(&w[(E.prim[(size_t)(lane / 2) * E.y_blocks + b] >> (16 * (lane & 1))) & 0xFFFFu], v);
+        for (uint32_t c = E.any_extra && y < E.Y ? E.extra_off[y] : 0; E.any_extra && y < E.Y && c < E.extra_off[y + 1]; c++)
+            atomicXor(&w[m2d_padded(E.extra[c])], v);
+    }
+    for (uint32_t i = tid; !ROWS && i < subs * E.y_blocks; i += M2D_NT) {
         if (i != tid) load_block(i);
         uint32_t t;
         const uint32_t b = split(i, E.y_blocks, t);
@@ -468,7 +533,13 @@ __global__ __launch_bounds__(M2D_NT, 4) void expand_kernel(ExpandDev E) {
     }
     // Records: column m is measurement word m, inverted where the reference sample is 1 (words past the last
     // measurement are zero, as are their inversion bits).
-    for (uint32_t i = tid; i < subs * P.blocks; i += M2D_NT) {
+    for (uint32_t i = tid >> 5; ROWS && i < subs * P.blocks; i += M2D_NT / 32) {
+        uint32_t t;
+        const uint32_t b = split(i, P.blocks, t);
+        const uint32_t v = transpose32(words[t * subw + 33 * b + lane], lane) ^ E.inv[b];
+        if (32 * t + lane < shots) store_row(v, P.out + (s0 + 32 * t + lane) * P.out_stride, (P.n_out + 7) / 8, b);
+    }
+    for (uint32_t i = tid; !ROWS && i < subs * P.blocks; i += M2D_NT) {
         uint32_t t;
         const uint32_t b = split(i, P.blocks, t);
         const uint32_t *const w = words + t * subw + 33 * b;
@@ -673,10 +744,20 @@ static uint32_t subtiles(uint64_t tiles, uint32_t blocks, size_t subtile_bytes, 
     return (uint32_t)std::max<uint64_t>(g, 1);
 }
 
+// Small launches put rows on lanes, a half-wave per block: a lane per block takes a wave through two transposes of 500
+// instructions (5 us) while most SIMDs have no wave at all. With more than a block or two for each of a workgroup's 16
+// half-waves, or a wave for each SIMD, blocks on lanes win. Conversion, rows | blocks on lanes: 5 blocks per subtile, 4000
+// shots 6.2 | 9.0 us, 250,000 shots 12.6 | 13.6; 37 blocks, 1000 shots 8.8 | 9.6, 16,000 shots 11.7 | 10.5; 127 blocks, 250
+// shots 28.5 | 11.4. Expansion: 4 blocks, 4000 shots 7.9 | 15.6 us, 250,000 shots 15.1 | 25.5.
+static bool rows_on_lanes(uint64_t tiles, uint32_t blocks) {
+    return blocks <= 48 && tiles * blocks * ((blocks + 15) / 16) <= 48 * 1024;
+}
+
 hipError_t launch_expand(ExpandDev E, hipStream_t stream) {
     const uint64_t tiles = (E.out.shots + 31) / 32;
     if (tiles == 0) return hipSuccess;
     const size_t sub = (size_t)expand_subtile_words(E.out.blocks) * 4;
+    const bool rows = rows_on_lanes(tiles, std::max(E.out.blocks, E.y_blocks));
     E.out.group = subtiles(tiles, std::max(E.out.blocks, E.y_blocks), sub, std::max(E.in_stride, E.out.out_stride));
     // Records after phase 0 staged in LDS where two workgroups still fit a CU.
     size_t lds = (sub * E.out.group + 15) / 16 * 16;
@@ -684,15 +765,16 @@ hipError_t launch_expand(ExpandDev E, hipStream_t stream) {
     if (lds + later <= 80 * 1024) lds += later;
     else E.staged = 0;
     const uint64_t grid = (tiles + E.out.group - 1) / E.out.group;
-#define STIM_AMD_LAUNCH(ONE)                                                                              \
-    {                                                                                                     \
-        static size_t reserved = 0;                                                                       \
-        const hipError_t e = reserve_lds(reinterpret_cast<const void *>(&expand_kernel<ONE>), lds, reserved); \
-        if (e != hipSuccess) return e;                                                                    \
-        hipLaunchKernelGGL(expand_kernel<ONE>, dim3((uint32_t)grid), dim3(M2D_NT), lds, stream, E);       \
+#define STIM_AMD_LAUNCH(ONE, ROWS)                                                                               \
+    {                                                                                                            \
+        static size_t reserved = 0;                                                                              \
+        const hipError_t e = reserve_lds(reinterpret_cast<const void *>(&expand_kernel<ONE, ROWS>), lds, reserved); \
+        if (e != hipSuccess) return e;                                                                           \
+        hipLaunchKernelGGL((expand_kernel<ONE, ROWS>), dim3((uint32_t)grid), dim3(M2D_NT), lds, stream, E);       \
     }
-    if (E.out.group == 1) STIM_AMD_LAUNCH(true)
-    else STIM_AMD_LAUNCH(false)
+    if (rows) STIM_AMD_LAUNCH(false, true)
+    else if (E.out.group == 1) STIM_AMD_LAUNCH(true, false)
+    else STIM_AMD_LAUNCH(false, false)
 #undef STIM_AMD_LAUNCH
     return hipGetLastError();
 }
@@ -710,15 +792,18 @@ hipError_t launch_m2d(M2dParams P, hipStream_t stream) {
     P.group = subtiles(tiles, nb, sub, std::max(std::max(P.in_stride, P.out_stride), P.sweep_stride));
     const size_t lds = sub * P.group;
     const uint64_t grid = (tiles + P.group - 1) / P.group;
-#define STIM_AMD_LAUNCH(SLOW)                                                                          \
-    {                                                                                                  \
-        static size_t reserved = 0;                                                                    \
-        const hipError_t e = reserve_lds(reinterpret_cast<const void *>(&m2d_kernel<SLOW>), lds, reserved); \
-        if (e != hipSuccess) return e;                                                                 \
-        hipLaunchKernelGGL(m2d_kernel<SLOW>, dim3((uint32_t)grid), dim3(M2D_NT), lds, stream, P);      \
+#define STIM_AMD_LAUNCH(SLOW, ROWS)                                                                              \
+    {                                                                                                            \
+        static size_t reserved = 0;                                                                              \
+        const hipError_t e = reserve_lds(reinterpret_cast<const void *>(&m2d_kernel<SLOW, ROWS>), lds, reserved); \
+        if (e != hipSuccess) return e;                                                                           \
+        hipLaunchKernelGGL((m2d_kernel<SLOW, ROWS>), dim3((uint32_t)grid), dim3(M2D_NT), lds, stream, P);         \
     }
-    if (P.slow) STIM_AMD_LAUNCH(true)
-    else STIM_AMD_LAUNCH(false)
+    const bool rows = rows_on_lanes(tiles, nb);
+    if (P.slow && rows) STIM_AMD_LAUNCH(true, true)
+    else if (P.slow) STIM_AMD_LAUNCH(true, false)
+    else if (rows) STIM_AMD_LAUNCH(false, true)
+    else STIM_AMD_LAUNCH(false, false)
 #undef STIM_AMD_LAUNCH
     return hipGetLastError();
 }

@@ -40,6 +40,8 @@ def _expected(meas, cols):
     (1, 1, 0, 1, 1), (3, 2, 1, 2, 33), (24, 31, 2, 3, 64), (31, 32, 9, 5, 95), (33, 33, 1, 12, 31),
     (145, 120, 1, 4, 40001), (2049, 2057, 3, 2, 65), (4160, 4095, 1, 6, 70), (16400, 16417, 1, 3, 33),
     (30000, 12000, 2, 8, 40),   # too many long columns for slots next to the record: listed
+    # Both sides of the line between rows on lanes and blocks on lanes: 48 and 49 blocks, many shots of few blocks.
+    (1536, 1535, 1, 6, 100), (1500, 1537, 2, 6, 100), (3, 2, 1, 2, 1600001), (33, 33, 1, 12, 800001),
 ])
 def test_whole_record_kernel_layout_edges(M, D, O, terms, shots):
     import torch
@@ -74,7 +76,8 @@ def test_whole_record_kernel_layout_edges(M, D, O, terms, shots):
 
 
 @pytest.mark.parametrize('family, d, r, shots', [('repetition_code:memory', 3, 2, 1), ('surface_code:rotated_memory_z', 3, 3, 33),
-                                                 ('surface_code:rotated_memory_x', 5, 4, 40001), ('surface_code:rotated_memory_z', 13, 9, 4099)])
+                                                 ('surface_code:rotated_memory_x', 5, 4, 40001), ('surface_code:rotated_memory_z', 13, 9, 4099),
+                                                 ('surface_code:rotated_memory_z', 25, 3, 321), ('repetition_code:memory', 3, 2, 1700001)])
 def test_expanded_records_keep_their_detection_events(family, d, r, shots):
     """Expanded records, with several subtiles per workgroup (many shots) and with one: the reference sample only
     inverts columns, so records with and without it convert to the same detection events; and a call in two parts
