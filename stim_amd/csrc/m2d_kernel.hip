@@ -128,7 +128,7 @@ __device__ __forceinline__ void store_rows(uint32_t (&x)[32], uint8_t *base, uin
 }
 
 // Rows on lanes: a half-wave's lane loads, or stores, the word of its own row (row < valid) of one block. For launches so
-// small that a lane per block leaves most of the chip idle (launch_m2d, rows_on_lanes).
+// small that a lane per block leaves most of the chip idle (lanes_by_rows).
 __device__ __forceinline__ uint32_t load_row(const uint8_t *r, uint32_t row_bytes, uint32_t b, bool exact) {
     if (exact && row_bytes < 4) {
         uint32_t v = 0;
@@ -150,11 +150,12 @@ __device__ __forceinline__ void store_row(uint32_t v, uint8_t *r, uint32_t row_b
     }
 }
 // Loads row blocks [0, blocks) of each subtile into its words from word `at` on.
+template <int NT>
 __device__ __forceinline__ void load_by_rows(uint32_t *words, uint32_t subw, uint32_t at, const uint8_t *in,
                                              uint64_t stride, uint32_t row_bytes, uint32_t blocks, bool exact,
                                              uint32_t shots) {
     const uint32_t lane = threadIdx.x & 31, subs = (shots + 31) / 32;
-    for (uint32_t i = threadIdx.x >> 5; i < subs * blocks; i += M2D_NT / 32) {
+    for (uint32_t i = threadIdx.x >> 5; i < subs * blocks; i += NT / 32) {
         const uint32_t t = i / blocks, b = i - t * blocks;
         const uint32_t x = load_row(in + min(32 * t + lane, shots - 1) * stride, row_bytes, b, exact);
         words[t * subw + at + 33 * b + lane] = transpose32(x, lane);
@@ -184,11 +185,11 @@ __device__ __forceinline__ uint32_t listed_word(const M2dParams &P, const uint32
 }
 
 // Separate observable rows (a few columns) of a workgroup's shots: one lane per shot and byte.
-template <bool SLOW>
+template <bool SLOW, int NT>
 __device__ __forceinline__ void store_observables(const M2dParams &P, const uint32_t *words, uint32_t subw, uint64_t s0,
                                                   uint32_t shots) {
     const uint32_t obytes = (P.n_obs + 7) / 8;
-    for (uint32_t i = threadIdx.x; i < shots * obytes; i += M2D_NT) {
+    for (uint32_t i = threadIdx.x; i < shots * obytes; i += NT) {
         const uint32_t shot = i / obytes, j = i - shot * obytes;
         const uint32_t *const w = words + (shot / 32) * subw;
         uint32_t v = 0;
@@ -216,8 +217,10 @@ __device__ __forceinline__ void store_observables(const M2dParams &P, const uint
 // rather than rows on lanes (32x32 transposes across half-waves, output staged in LDS 64 blocks at a time) take
 // 0.96 instead of 1.53 ms per 2^20 shots at d=25 (4.3 TB/s); without its loads and stores the kernel takes 0.52.
 // Resident workgroups that prefetch the next tile's rows spill and wait for their stores: 2.1 ms.
-template <bool SLOW, bool ROWS>
-__global__ __launch_bounds__(M2D_NT, 4) void m2d_kernel(M2dParams P) {
+template <bool SLOW, int ROWS_NT>
+__global__ __launch_bounds__(ROWS_NT ? ROWS_NT : M2D_NT, 4) void m2d_kernel(M2dParams P) {
+    constexpr bool ROWS = ROWS_NT > 0;
+    constexpr int NT = ROWS ? ROWS_NT : M2D_NT;
     extern __shared__ __align__(16) uint32_t words[];
     const uint32_t tid = threadIdx.x, G = P.group;
     const uint64_t s0 = (uint64_t)xcd_tile(blockIdx.x, gridDim.x) * 32 * G;
@@ -226,16 +229,16 @@ __global__ __launch_bounds__(M2D_NT, 4) void m2d_kernel(M2dParams P) {
     const uint32_t subs = (shots + 31) / 32;
     const uint32_t subw = m2d_subtile_words(P.blocks, P.sweep_blocks, P.spill_slots);
     const uint32_t zero = m2d_padded(m2d_zero_word(P.blocks, P.sweep_blocks));
-    for (uint32_t i = tid; i < subs; i += M2D_NT) words[i * subw + zero] = 0;
-    for (uint32_t i = tid; i < subs * P.spill_slots; i += M2D_NT) {
+    for (uint32_t i = tid; i < subs; i += NT) words[i * subw + zero] = 0;
+    for (uint32_t i = tid; i < subs * P.spill_slots; i += NT) {
         const uint32_t t = i / P.spill_slots;
         words[t * subw + m2d_padded(m2d_zero_word(P.blocks, P.sweep_blocks) + 4 + (i - t * P.spill_slots))] = 0;
     }
 
     // Rows whose stride covers whole words are read past their last byte (never past the buffer's
     // shots * stride bytes); the bits there belong to no measurement.
-    if (ROWS) load_by_rows(words, subw, 0, P.in + s0 * P.in_stride, P.in_stride, P.in_row_bytes, P.blocks, !P.in_vec, shots);
-    for (uint32_t i = tid; !ROWS && i < subs * P.blocks; i += M2D_NT) {
+    if (ROWS) load_by_rows<NT>(words, subw, 0, P.in + s0 * P.in_stride, P.in_stride, P.in_row_bytes, P.blocks, !P.in_vec, shots);
+    for (uint32_t i = tid; !ROWS && i < subs * P.blocks; i += NT) {
         const uint32_t t = i / P.blocks, b = i - t * P.blocks;
         uint32_t x[32];
         load_rows(x, P.in + s0 * P.in_stride, P.in_stride, 32 * t * (uint32_t)P.in_stride, P.in_row_bytes, b, !P.in_vec,
@@ -249,9 +252,9 @@ __global__ __launch_bounds__(M2D_NT, 4) void m2d_kernel(M2dParams P) {
         const uint32_t sw0 = m2d_padded(m2d_sweep_word(P.blocks));
         const bool by_rows = ROWS && P.sweep;
         if (by_rows)
-            load_by_rows(words, subw, sw0, P.sweep + s0 * P.sweep_stride, P.sweep_stride, P.sweep_row_bytes,
+            load_by_rows<NT>(words, subw, sw0, P.sweep + s0 * P.sweep_stride, P.sweep_stride, P.sweep_row_bytes,
                          P.sweep_blocks, true, shots);
-        for (uint32_t i = tid; !by_rows && i < subs * P.sweep_blocks; i += M2D_NT) {
+        for (uint32_t i = tid; !by_rows && i < subs * P.sweep_blocks; i += NT) {
             const uint32_t t = i / P.sweep_blocks, b = i - t * P.sweep_blocks;
             uint32_t x[32];
 #pragma unroll
@@ -268,7 +271,7 @@ __global__ __launch_bounds__(M2D_NT, 4) void m2d_kernel(M2dParams P) {
     }
     __syncthreads();
     if (P.spill_chunks) {
-        for (uint32_t i = tid; i < subs * P.spill_chunks; i += M2D_NT) {
+        for (uint32_t i = tid; i < subs * P.spill_chunks; i += NT) {
             const uint32_t t = i / P.spill_chunks;
             const uint4 c = P.spill[i - t * P.spill_chunks];
             uint32_t *const w = words + t * subw;
@@ -279,7 +282,7 @@ __global__ __launch_bounds__(M2D_NT, 4) void m2d_kernel(M2dParams P) {
 
     const uint32_t nb = (P.n_out + 31) / 32, TB = P.total_blocks;
     const uint32_t lane = tid & 31;
-    for (uint32_t i = tid >> 5; ROWS && i < subs * nb; i += M2D_NT / 32) {
+    for (uint32_t i = tid >> 5; ROWS && i < subs * nb; i += NT / 32) {
         const uint32_t t = i / nb, b = i - t * nb;
         const uint32_t *const w = words + t * subw;
         const uint2 info = P.block_info[b];
@@ -293,7 +296,7 @@ __global__ __launch_bounds__(M2D_NT, 4) void m2d_kernel(M2dParams P) {
         if (live < 32) x &= (1u << live) - 1;
         if (32 * t + lane < shots) store_row(x, P.out + (s0 + 32 * t + lane) * P.out_stride, (P.n_out + 7) / 8, b);
     }
-    for (uint32_t i = tid; !ROWS && i < subs * nb; i += M2D_NT) {
+    for (uint32_t i = tid; !ROWS && i < subs * nb; i += NT) {
         const uint32_t t = i / nb, b = i - t * nb;
         const uint32_t *const w = words + t * subw;
         const uint2 info = P.block_info[b];
@@ -322,7 +325,7 @@ __global__ __launch_bounds__(M2D_NT, 4) void m2d_kernel(M2dParams P) {
         store_rows(x, P.out + s0 * P.out_stride, P.out_stride, 32 * t * (uint32_t)P.out_stride, b, (P.n_out + 7) / 8,
                    min(shots - 32 * t, 32u));
     }
-    store_observables<SLOW>(P, words, subw, s0, shots);
+    store_observables<SLOW, NT>(P, words, subw, s0, shots);
 }
 
 // Random words of the free results: Philox4x32-10 keyed by the sampler's expansion key, counter (group of
@@ -391,8 +394,10 @@ __device__ __forceinline__ void expand_record(uint32_t *words, uint4 r, uint4 q)
 // 1.32 ms (3.2 TB/s of y rows read and record rows written), of which the steps are about 0.45; with rows on
 // lanes, staged output and 1024-lane workgroups 1.76.
 // ONE: one subtile per workgroup (no divisions by the counts).
-template <bool ONE, bool ROWS>
-__global__ __launch_bounds__(M2D_NT, 4) void expand_kernel(ExpandDev E) {
+template <bool ONE, int ROWS_NT>
+__global__ __launch_bounds__(ROWS_NT ? ROWS_NT : M2D_NT, 4) void expand_kernel(ExpandDev E) {
+    constexpr bool ROWS = ROWS_NT > 0;
+    constexpr int NT = ROWS ? ROWS_NT : M2D_NT;
     extern __shared__ __align__(16) uint32_t words[];
     const M2dParams &P = E.out;
     const uint32_t tid = threadIdx.x, G = ONE ? 1 : P.group;
@@ -419,7 +424,7 @@ __global__ __launch_bounds__(M2D_NT, 4) void expand_kernel(ExpandDev E) {
     };
     if (!ROWS && tid < subs * E.y_blocks) load_block(tid);
     const uint32_t step0 = E.nsteps ? E.steps[1] : 0, staged = E.staged;
-    // Step 0's records of this lane: tid and tid + M2D_NT.
+    // Step 0's records of this lane: tid and tid + NT.
     uint4 ra, qa, rb, qb;
     uint32_t sub;
     if (tid < subs * step0) {
@@ -427,17 +432,17 @@ __global__ __launch_bounds__(M2D_NT, 4) void expand_kernel(ExpandDev E) {
         ra = E.items[2 * f];
         qa = E.items[2 * f + 1];
     }
-    if (tid + M2D_NT < subs * step0) {
-        const uint32_t f = split(tid + M2D_NT, step0, sub);
+    if (tid + NT < subs * step0) {
+        const uint32_t f = split(tid + NT, step0, sub);
         rb = E.items[2 * f];
         qb = E.items[2 * f + 1];
     }
-    for (uint32_t i = tid; i < 2 * staged; i += M2D_NT) stage[i] = E.items[2 * step0 + i];
-    for (uint32_t i = tid; i < (subs * subw + 3) / 4; i += M2D_NT) reinterpret_cast<uint4 *>(words)[i] = make_uint4(0, 0, 0, 0);
+    for (uint32_t i = tid; i < 2 * staged; i += NT) stage[i] = E.items[2 * step0 + i];
+    for (uint32_t i = tid; i < (subs * subw + 3) / 4; i += NT) reinterpret_cast<uint4 *>(words)[i] = make_uint4(0, 0, 0, 0);
     __syncthreads();
     // Free results (distinct from every y slot, so no ordering with the y words; slots padded, in fours).
     const uint32_t k0 = (uint32_t)E.seed, k1 = (uint32_t)(E.seed >> 32), fg = (E.nfree + 3) / 4;
-    for (uint32_t i = tid; i < subs * fg; i += M2D_NT) {
+    for (uint32_t i = tid; i < subs * fg; i += NT) {
         uint32_t t;
         const uint32_t g = split(i, fg, t);
         const uint64_t tile = E.tile0 + (uint64_t)block * G + t;
@@ -451,7 +456,7 @@ __global__ __launch_bounds__(M2D_NT, 4) void expand_kernel(ExpandDev E) {
     }
     // y words into their slots (two 16-bit padded indices per entry; columns past the last go to the spare word).
     const uint32_t lane = tid & 31;
-    for (uint32_t i = tid >> 5; ROWS && i < subs * E.y_blocks; i += M2D_NT / 32) {
+    for (uint32_t i = tid >> 5; ROWS && i < subs * E.y_blocks; i += NT / 32) {
         uint32_t t;
         const uint32_t b = split(i, E.y_blocks, t), y = 32 * b + lane;
         uint32_t v = load_row(E.in + (s0 + min(32 * t + lane, shots - 1)) * E.in_stride, 0, b, false);
@@ -461,7 +466,7 @@ __global__ __launch_bounds__(M2D_NT, 4) void expand_kernel(ExpandDev E) {
         for (uint32_t c = E.any_extra && y < E.Y ? E.extra_off[y] : 0; E.any_extra && y < E.Y && c < E.extra_off[y + 1]; c++)
             atomicXor(&w[m2d_padded(E.extra[c])], v);
     }
-    for (uint32_t i = tid; !ROWS && i < subs * E.y_blocks; i += M2D_NT) {
+    for (uint32_t i = tid; !ROWS && i < subs * E.y_blocks; i += NT) {
         if (i != tid) load_block(i);
         uint32_t t;
         const uint32_t b = split(i, E.y_blocks, t);
@@ -485,7 +490,7 @@ __global__ __launch_bounds__(M2D_NT, 4) void expand_kernel(ExpandDev E) {
     // Substitution: a step's records read results of earlier steps (a chain its own, in order).
     auto step = [&](uint32_t p, uint32_t i0) {
         const uint32_t at = E.steps[p], n = E.steps[p + 1] - at;
-        for (uint32_t i = i0; i < subs * n; i += M2D_NT) {
+        for (uint32_t i = i0; i < subs * n; i += NT) {
             uint32_t t;
             const uint32_t f = at + split(i, n, t);
             uint4 r, q;
@@ -508,11 +513,11 @@ __global__ __launch_bounds__(M2D_NT, 4) void expand_kernel(ExpandDev E) {
             (void)split(tid, step0, sub);
             expand_record(words + sub * subw, ra, qa);
         }
-        if (tid + M2D_NT < subs * step0) {
-            (void)split(tid + M2D_NT, step0, sub);
+        if (tid + NT < subs * step0) {
+            (void)split(tid + NT, step0, sub);
             expand_record(words + sub * subw, rb, qb);
         }
-        step(0, tid + 2 * M2D_NT);
+        step(0, tid + 2 * NT);
         __syncthreads();
     }
     const uint32_t wide = ONE ? max(E.wave_step, 1u) : E.nsteps;
@@ -533,13 +538,13 @@ __global__ __launch_bounds__(M2D_NT, 4) void expand_kernel(ExpandDev E) {
     }
     // Records: column m is measurement word m, inverted where the reference sample is 1 (words past the last
     // measurement are zero, as are their inversion bits).
-    for (uint32_t i = tid >> 5; ROWS && i < subs * P.blocks; i += M2D_NT / 32) {
+    for (uint32_t i = tid >> 5; ROWS && i < subs * P.blocks; i += NT / 32) {
         uint32_t t;
         const uint32_t b = split(i, P.blocks, t);
         const uint32_t v = transpose32(words[t * subw + 33 * b + lane], lane) ^ E.inv[b];
         if (32 * t + lane < shots) store_row(v, P.out + (s0 + 32 * t + lane) * P.out_stride, (P.n_out + 7) / 8, b);
     }
-    for (uint32_t i = tid; !ROWS && i < subs * P.blocks; i += M2D_NT) {
+    for (uint32_t i = tid; !ROWS && i < subs * P.blocks; i += NT) {
         uint32_t t;
         const uint32_t b = split(i, P.blocks, t);
         const uint32_t *const w = words + t * subw + 33 * b;
@@ -579,16 +584,6 @@ __device__ __forceinline__ uint32_t ring_column_word(const M2dParams &P, const u
         v = (c >= 1 ? w0 : 0u) ^ (c == 2 ? w1 : 0u);
     }
     return (r.x & M2D_INVERT) ? ~v : v;
-}
-
-// Writes staged blocks [0, nb) (bytes [0, nbytes) of each staged row) to bytes [off, off + nbytes) of
-// the tile's rows: thread t copies byte t of every row (coalesced across the workgroup per row).
-__device__ __forceinline__ void win_flush(const uint8_t *img, uint8_t *dst, uint64_t stride, uint32_t off,
-                                          uint32_t nbytes, uint64_t s0, uint32_t valid) {
-    const uint32_t c = threadIdx.x;
-    if (c >= nbytes) return;
-    uint8_t *base = dst + s0 * stride + off + c;
-    for (uint32_t r = 0; r < valid; r++) __builtin_nontemporal_store(img[r * WIN_PITCH + c], base + r * stride);
 }
 
 // Output blocks are staged a pass at a time: up to WIN_PASS blocks, block b + u * WIN_HALVES + half
@@ -745,19 +740,23 @@ static uint32_t subtiles(uint64_t tiles, uint32_t blocks, size_t subtile_bytes, 
 }
 
 // Small launches put rows on lanes, a half-wave per block: a lane per block takes a wave through two transposes of 500
-// instructions (5 us) while most SIMDs have no wave at all. With more than a block or two for each of a workgroup's 16
-// half-waves, or a wave for each SIMD, blocks on lanes win. Conversion, rows | blocks on lanes: 5 blocks per subtile, 4000
-// shots 6.2 | 9.0 us, 250,000 shots 12.6 | 13.6; 37 blocks, 1000 shots 8.8 | 9.6, 16,000 shots 11.7 | 10.5; 127 blocks, 250
-// shots 28.5 | 11.4. Expansion: 4 blocks, 4000 shots 7.9 | 15.6 us, 250,000 shots 15.1 | 25.5.
-static bool rows_on_lanes(uint64_t tiles, uint32_t blocks) {
-    return blocks <= 48 && tiles * blocks * ((blocks + 15) / 16) <= 48 * 1024;
+// instructions (5 us) while most SIMDs have no wave at all. Up to 256 subtiles, one workgroup per CU, of 1024 lanes: up to
+// four blocks for each of its 32 half-waves that is faster; beyond, with 512 lanes, as far as its 16 half-waves have a
+// block or two and the launch has less than a wave of blocks for each SIMD. Conversion, rows | blocks on lanes: 4 blocks
+// per subtile, 4000 shots 6.2 | 9.1 us, 120,000 shots 8.8 | 11.1; 26 blocks, 4000 shots 6.3 | 9.9, 16,000 shots 7.7 | 9.8,
+// 120,000 shots 24 | 16.5; 92 blocks, 4000 shots 8.4 | 9.2, 16,000 shots 12.5 | 10.8; 127 blocks, 250 shots 10.2 | 9.4; 508 blocks, 250 shots 25 | 11.6.
+// Expansion: 4 blocks, 4000 shots 7.9 | 15.7 us, 250,000 shots 15.1 (1024 lanes: 21.8) | 25.5.
+// 0: blocks on lanes.
+static int lanes_by_rows(uint64_t tiles, uint32_t blocks) {
+    if (tiles <= 256) return blocks <= 112 ? 1024 : 0;
+    return blocks <= 32 && tiles * blocks * ((blocks + 15) / 16) <= 48 * 1024 ? 512 : 0;
 }
 
 hipError_t launch_expand(ExpandDev E, hipStream_t stream) {
     const uint64_t tiles = (E.out.shots + 31) / 32;
     if (tiles == 0) return hipSuccess;
     const size_t sub = (size_t)expand_subtile_words(E.out.blocks) * 4;
-    const bool rows = rows_on_lanes(tiles, std::max(E.out.blocks, E.y_blocks));
+    const int rows = lanes_by_rows(tiles, std::max(E.out.blocks, E.y_blocks));
     E.out.group = subtiles(tiles, std::max(E.out.blocks, E.y_blocks), sub, std::max(E.in_stride, E.out.out_stride));
     // Records after phase 0 staged in LDS where two workgroups still fit a CU.
     size_t lds = (sub * E.out.group + 15) / 16 * 16;
@@ -770,11 +769,12 @@ hipError_t launch_expand(ExpandDev E, hipStream_t stream) {
         static size_t reserved = 0;                                                                              \
         const hipError_t e = reserve_lds(reinterpret_cast<const void *>(&expand_kernel<ONE, ROWS>), lds, reserved); \
         if (e != hipSuccess) return e;                                                                           \
-        hipLaunchKernelGGL((expand_kernel<ONE, ROWS>), dim3((uint32_t)grid), dim3(M2D_NT), lds, stream, E);       \
+        hipLaunchKernelGGL((expand_kernel<ONE, ROWS>), dim3((uint32_t)grid), dim3(ROWS ? ROWS : M2D_NT), lds, stream, E);       \
     }
-    if (rows) STIM_AMD_LAUNCH(false, true)
-    else if (E.out.group == 1) STIM_AMD_LAUNCH(true, false)
-    else STIM_AMD_LAUNCH(false, false)
+    if (rows == 1024) STIM_AMD_LAUNCH(false, 1024)
+    else if (rows) STIM_AMD_LAUNCH(false, 512)
+    else if (E.out.group == 1) STIM_AMD_LAUNCH(true, 0)
+    else STIM_AMD_LAUNCH(false, 0)
 #undef STIM_AMD_LAUNCH
     return hipGetLastError();
 }
@@ -797,13 +797,15 @@ hipError_t launch_m2d(M2dParams P, hipStream_t stream) {
         static size_t reserved = 0;                                                                              \
         const hipError_t e = reserve_lds(reinterpret_cast<const void *>(&m2d_kernel<SLOW, ROWS>), lds, reserved); \
         if (e != hipSuccess) return e;                                                                           \
-        hipLaunchKernelGGL((m2d_kernel<SLOW, ROWS>), dim3((uint32_t)grid), dim3(M2D_NT), lds, stream, P);         \
+        hipLaunchKernelGGL((m2d_kernel<SLOW, ROWS>), dim3((uint32_t)grid), dim3(ROWS ? ROWS : M2D_NT), lds, stream, P);         \
     }
-    const bool rows = rows_on_lanes(tiles, nb);
-    if (P.slow && rows) STIM_AMD_LAUNCH(true, true)
-    else if (P.slow) STIM_AMD_LAUNCH(true, false)
-    else if (rows) STIM_AMD_LAUNCH(false, true)
-    else STIM_AMD_LAUNCH(false, false)
+    const int rows = lanes_by_rows(tiles, nb);
+    if (rows == 1024 && P.slow) STIM_AMD_LAUNCH(true, 1024)
+    else if (rows == 1024) STIM_AMD_LAUNCH(false, 1024)
+    else if (rows && P.slow) STIM_AMD_LAUNCH(true, 512)
+    else if (rows) STIM_AMD_LAUNCH(false, 512)
+    else if (P.slow) STIM_AMD_LAUNCH(true, 0)
+    else STIM_AMD_LAUNCH(false, 0)
 #undef STIM_AMD_LAUNCH
     return hipGetLastError();
 }

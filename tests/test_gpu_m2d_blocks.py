@@ -40,8 +40,10 @@ def _expected(meas, cols):
     (1, 1, 0, 1, 1), (3, 2, 1, 2, 33), (24, 31, 2, 3, 64), (31, 32, 9, 5, 95), (33, 33, 1, 12, 31),
     (145, 120, 1, 4, 40001), (2049, 2057, 3, 2, 65), (4160, 4095, 1, 6, 70), (16400, 16417, 1, 3, 33),
     (30000, 12000, 2, 8, 40),   # too many long columns for slots next to the record: listed
-    # Both sides of the line between rows on lanes and blocks on lanes: 48 and 49 blocks, many shots of few blocks.
-    (1536, 1535, 1, 6, 100), (1500, 1537, 2, 6, 100), (3, 2, 1, 2, 1600001), (33, 33, 1, 12, 800001),
+    # Both sides of the lines between rows on lanes and blocks on lanes: 112 and 113 blocks, 256 and 257 subtiles with 32 and
+    # 33 blocks, many shots of few blocks.
+    (3584, 3583, 1, 6, 100), (3500, 3585, 2, 6, 100), (1024, 1023, 1, 5, 8192), (1000, 1024, 1, 5, 8193),
+    (1000, 1025, 1, 5, 8193), (3, 2, 1, 2, 1600001), (33, 33, 1, 12, 800001),
 ])
 def test_whole_record_kernel_layout_edges(M, D, O, terms, shots):
     import torch
