@@ -89,9 +89,8 @@ int mfs_m2d_stats(const mfs_m2d *c, uint64_t out[4]);
  * MFS_SEPARATE_OBSERVABLES, observable rows; MFS_BIT_PACKED selects packed outputs (else one byte per
  * entry); MFS_DEVICE_OUTPUT means every pointer is device memory. Each detector (observable) is the
  * XOR of its measurements, inverted when the XOR of their reference bits is 1. Packed device
- * measurement rows with 16-byte-aligned address and stride >= 16 * ceil(M / 128) are read in place,
- * 16 bytes at a time, so that buffer must span shots * meas_stride bytes. Output strides must be
- * below 2^30 bytes.
+ * measurement rows with 16-byte-aligned address and stride >= 16 * ceil(M / 128) are read past their last
+ * byte, so that buffer must span shots * meas_stride bytes. Output strides must be below 2^30 bytes.
  * Reference: CompiledMeasurementsToDetectionEventsConverter.convert
  * (measurements_to_detection_events.pybind.cc:78-157) and measurements_to_detection_events_helper
  * (src/stim/simulators/measurements_to_detection_events.inl:29-131). */
@@ -119,7 +118,7 @@ int mfs_m2d_bench(mfs_m2d *c, uint64_t shots, int warmup, int iters, double out_
 int mfs_m2d_set_kernel(mfs_m2d *c, int kernel);
 /* out[0..3] = ring words of the windowed kernel per output layout (0: not applicable): observables
  * appended, observables separate, detectors only, observables appended and separate; out[4] = LDS
- * bytes per tile of the whole-record kernel, out[5] = of the windowed kernel (appended layout; 0 when
+ * bytes a tile's record counts for (its words plus 8 KB: what must fit for the whole-record kernel), out[5] = of the windowed kernel (appended layout; 0 when
  * not applicable). */
 int mfs_m2d_kernel_info(const mfs_m2d *c, uint64_t out[6]);
 
@@ -306,7 +305,7 @@ int mfs_get_info(const mfs_sampler *s, uint64_t out[8]); /* tile_words, lds_byte
 /* Symptom-engine scan kernel: 0 (default) = the specialised kernel with one precomputed outcome record
  * per (noise site, outcome) where the model allows it (plain groups with uniform outcomes, as in the
  * QEC memory circuits), else the generic kernel; 1 = always the generic kernel, which applies a hit's
- * basis-column records one by one. Both draw the same hits, so rows are bit-identical. No reference
+ * basis-column records one by one (a detector error model's: the kernel that reads full records). Both draw the same hits, so rows are bit-identical. No reference
  * counterpart. */
 int mfs_set_scan_variant(mfs_sampler *s, int variant);
 

@@ -57,7 +57,8 @@ struct ExpandPlan {
     // chain (a check repeated round after round);
     // 2 <= n <= 7: result k ^= the XOR of results words 1 .. n (the terms inline);
     // n >= 8: result k ^= the XOR of results terms[word 1 .. word 1 + n).
-    // Unused words are 0. Thread t runs records [sched_off[p * threads + t], sched_off[p * threads + t +
+    // Unused words are 0. The kernel runs them as steps, a lane per record (upload_expand_steps in sampler_impl.h: the
+    // threads' first records of a phase, then their second ones, ...). Thread t owns records [sched_off[p * threads + t], sched_off[p * threads + t +
     // 1]) in phase p.
     uint32_t threads = 0, phases = 0;
     std::vector<uint32_t> sched_off, items, terms;

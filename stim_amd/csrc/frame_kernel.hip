@@ -443,8 +443,8 @@ __device__ __forceinline__ DevOp scalar_op(const uint4 &lo, const uint4 &hi) {
 // tiles takes 0.83 of the time of one of 512. So ops are staged a page at a time and not from one barrier to the next
 // (5000 qubits, 20 layers: 388 page turns before, 58 with the large pages, and 97 barriers, where ops share rows), and
 // steer scalar branches; a lane handles several items of an op at once; and noise keeps its loads in flight while it
-// draws. 16384 shots of that circuit 0.548 -> 0.313 ms, of which noise takes 0.10 and the Clifford ops 0.21 (LDS
-// transfers alone: 0.07); 1000 shots of the surface code of d = 5 0.110 -> 0.072 ms; 2^18 shots of d = 25 5.06 -> 3.42 ms.
+// draws. 16384 shots of that circuit 0.548 -> 0.306 ms, of which noise takes 0.10 and the Clifford ops 0.21 (LDS
+// transfers alone: 0.07); 1000 shots of the surface code of d = 5 0.110 -> 0.073 ms; 2^18 shots of d = 25 5.06 -> 3.36 ms.
 template <int T, int NT>
 __global__ __launch_bounds__(NT) void frame_sim_kernel(const uint32_t *__restrict__ blob,
                                                        const uint32_t *__restrict__ ntgt,
