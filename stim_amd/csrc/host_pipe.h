@@ -9,7 +9,8 @@
 // at the link's 57 GB/s) into new numpy arrays, whose pages are touched for the first time here: 1.17 ms, and 1.1
 // to 1.5 ms with one transfer and then one copy of the whole batch; 20,001 rows of 1,798 entries as bytes 1.4 instead of
 // 1.8 ms. Inputs in host memory (m2d) take the same way in: 50,001 records of 181 bytes converted in 0.72 ms, where
-// a pitched copy from pageable memory took 9 us for each row, 460 ms.
+// a pitched copy from pageable memory took 9 us for each row, 460 ms; 600,001 of them, seven batches, in 3.9 ms (5.8 where
+// an input's helpers wait behind those of the output before it).
 // Per slot, three orderings keep the buffers consistent:
 //   - the DMA of batch i waits for batch i's kernels (event `produced`, a wait on the copy stream);
 //   - batch i + 2's kernels wait for batch i's DMA out of the slot (the last event `arrived`, a wait on the
@@ -32,11 +33,12 @@
 #include <cstring>
 #include <deque>
 #include <functional>
+#include <memory>
 #include <mutex>
 #include <stdexcept>
 #include <string>
-#include <system_error>
 #include <thread>
+#include <utility>
 #include <vector>
 
 namespace sa {
@@ -83,52 +85,233 @@ inline void pack_bytes(const uint8_t *src, uint8_t *dst, size_t n) {
     }
 }
 
-// Host threads of all pipelines in the process: at most as many as a batch uses (HostPipe::host_threads), started when
-// work waits and no thread is idle, and ended after a second without work. Starting threads anew for
-// each batch took about 15 us each, as much as a 1 MB transfer.
-class CopyPool {
+// Idle host threads of the process, lent to one pipeline's call at a time and given back when it ends; a thread without
+// work for a second ends. Starting threads anew for each batch took about 15 us each, as much as a 1 MB transfer.
+class HostThreads {
    public:
-    static CopyPool &get() {
-        static CopyPool *pool = new CopyPool;   // never destroyed: a thread may still be idle at exit
-        return *pool;
+    static HostThreads &get() {
+        static HostThreads *threads = new HostThreads;   // never destroyed: a thread may still be idle at exit
+        return *threads;
     }
-    // Queues f to run on some thread; false when none could be started and none will take it.
-    bool run(std::function<void()> f, int most) {
+    // Runs f on up to n threads, each its own (none waits for a thread that runs something else); returns how many.
+    int run(const std::function<void()> &f, int n) {
+        int got = 0, wake = 0;
         std::unique_lock<std::mutex> lock(mu_);
-        if (idle_ <= (int)queue_.size() && alive_ < most) {
-            try {
-                std::thread([this] { serve(); }).detach();
-                alive_++;
-            } catch (const std::system_error &) {
-                if (alive_ == 0) return false;
+        try {
+            for (; got < n; got++) {
+                if (idle_ > (int)queue_.size()) {
+                    queue_.push_back(f);
+                    wake++;
+                } else if (alive_ < MOST) {
+                    std::thread([this, f] { serve(f); }).detach();
+                    alive_++;
+                } else {
+                    break;
+                }
             }
+        } catch (const std::exception &) {
+            // No further thread or no memory: those that run are enough.
         }
-        queue_.push_back(std::move(f));
         lock.unlock();
-        cv_.notify_one();
-        return true;
+        for (int k = 0; k < wake; k++) cv_.notify_one();
+        return got;
     }
 
    private:
-    void serve() {
+    static constexpr int MOST = 256;   // 32 calls' worth at once; further calls copy on their own threads
+    void serve(std::function<void()> f) {
+        f();
+        f = nullptr;
         std::unique_lock<std::mutex> lock(mu_);
         for (;;) {
             idle_++;
             cv_.wait_for(lock, std::chrono::seconds(1), [&] { return !queue_.empty(); });
             idle_--;
             if (queue_.empty()) break;
-            std::function<void()> f = std::move(queue_.front());
+            f = std::move(queue_.front());
             queue_.pop_front();
             lock.unlock();
             f();
+            f = nullptr;
             lock.lock();
         }
         alive_--;
     }
     std::mutex mu_;
     std::condition_variable cv_;
-    std::deque<std::function<void()>> queue_;
+    std::deque<std::function<void()>> queue_;   // at most one entry per idle thread
     int alive_ = 0, idle_ = 0;
+};
+
+// The threads that copy for one pipeline during a call, and their work: up to three jobs, each a number of shares that are
+// taken one after another. The shares of an output become available a piece at a time, as the transfer's chunks arrive: one
+// thread at a time waits for the next chunk, of the older output first. The call's own thread takes part while it waits
+// for a job. A call has threads of its own, so that none waits behind another call's kernel, and an input is
+// copied by all of them while an output is still on its way.
+class Crew : public std::enable_shared_from_this<Crew> {
+   public:
+    enum { INPUT = 0, OUTPUT = 1, JOBS = 3 };   // INPUT, and one output per slot
+
+    // Posts job `j` (which is done) for at least `helpers` threads beside the caller: shares 0 .. total - 1, available
+    // at once, or `piece` more each time arrive(number of the piece) returns.
+    void post(int j, int helpers, int total, std::function<void(int)> share, int piece = 0,
+              std::function<hipError_t(int)> arrive = nullptr) {
+        const std::function<void()> member = [self = shared_from_this()] { self->serve(); };
+        int need;
+        {
+            std::lock_guard<Spin> lock(mu_);
+            Job &job = jobs_[j];
+            job.share = std::move(share);
+            job.arrive = std::move(arrive);
+            job.total = total;
+            job.piece = piece;
+            job.available = piece ? 0 : total;
+            job.next = 0;
+            job.order = orders_++;
+            job.error = hipSuccess;
+            in_call_ = true;
+            need = std::max(0, helpers - members_);
+            members_ += need;
+            version_++;
+        }
+        cv_.notify_all();
+        if (!need) return;
+        const int got = HostThreads::get().run(member, need);
+        if (got < need) {
+            std::lock_guard<Spin> lock(mu_);
+            members_ -= need - got;
+        }
+    }
+
+    // Takes part in job j until it is done.
+    hipError_t finish(int j) {
+        std::unique_lock<Spin> lock(mu_);
+        while (active(jobs_[j])) {
+            if (!step(lock, j)) wait(lock);
+        }
+        return std::exchange(jobs_[j].error, hipSuccess);
+    }
+
+    // Withdraws what nobody has started and waits for the rest.
+    void cancel() {
+        std::unique_lock<Spin> lock(mu_);
+        for (Job &job : jobs_) job.total = job.available = job.next;
+        for (Job &job : jobs_) {
+            while (active(job)) wait(lock);
+            job.error = hipSuccess;
+        }
+    }
+
+    // The call has ended (every job is done): the threads go as soon as they notice, and nothing waits for that.
+    void end_call() {
+        {
+            std::lock_guard<Spin> lock(mu_);
+            in_call_ = false;
+            version_++;
+        }
+        cv_.notify_all();
+    }
+
+   private:
+    // Held for a few instructions at a time, by up to nine threads that a chunk's arrival sets going at once: a mutex puts
+    // most of them to sleep there (36 MB of rows in 1.30 instead of 1.16 ms).
+    struct Spin {
+        std::atomic_flag held = ATOMIC_FLAG_INIT;
+        void lock() {
+            for (int tries = 0; held.test_and_set(std::memory_order_acquire); tries++) {
+                if (tries % 64 == 63) std::this_thread::yield();
+                else _mm_pause();
+            }
+        }
+        void unlock() { held.clear(std::memory_order_release); }
+    };
+
+    struct Job {
+        std::function<void(int)> share;
+        std::function<hipError_t(int)> arrive;
+        int total = 0, piece = 0, available = 0, next = 0;
+        int running = 0;         // threads in a share
+        bool waiting = false;    // a thread waits for its next piece
+        uint64_t order = 0;
+        hipError_t error = hipSuccess;
+    };
+
+    static bool active(const Job &job) { return job.next < job.total || job.running || job.waiting; }
+
+    // Takes one share, the input's first, then the older output's, or waits for one piece. The call's own thread names the
+    // job that it needs next (a member: -1): it takes no other share while it needs an input, which kernels wait for, and
+    // waits for no newer output's piece (36 MB of rows in 1.30 instead of 1.17 ms if it takes no other output's share).
+    bool step(std::unique_lock<Spin> &lock, int needed) {
+        int by_age[JOBS] = {INPUT, OUTPUT, OUTPUT + 1};
+        if (jobs_[OUTPUT + 1].order < jobs_[OUTPUT].order) std::swap(by_age[1], by_age[2]);
+        for (int j : by_age) {
+            Job &job = jobs_[j];
+            if ((needed == INPUT && j != INPUT) || job.next >= job.available) continue;
+            const int i = job.next++;
+            job.running++;
+            lock.unlock();
+            job.share(i);
+            lock.lock();
+            job.running--;
+            if (!active(job)) version_++;
+            return true;
+        }
+        bool waiting = false;
+        for (const Job &job : jobs_) waiting = waiting || job.waiting;
+        for (int j : by_age) {
+            Job &job = jobs_[j];
+            if (waiting || needed == INPUT || job.available >= job.total) continue;
+            if (needed >= 0 && job.order > jobs_[needed].order) continue;
+            job.waiting = true;
+            lock.unlock();
+            const hipError_t e = job.arrive(job.available / job.piece);
+            lock.lock();
+            job.waiting = false;
+            if (e == hipSuccess) {
+                job.available = std::min(job.total, job.available + job.piece);
+            } else {
+                job.error = e;
+                job.total = job.available = job.next;
+            }
+            version_++;
+            return true;
+        }
+        return false;
+    }
+
+    // Waits until something changes: polling while some job is under way (a chunk, or another thread's share, is
+    // about to end; waking eight sleepers for each chunk costs more), asleep while there is none.
+    void wait(std::unique_lock<Spin> &lock) {
+        const uint64_t seen = version_;
+        bool soon = false;
+        for (const Job &job : jobs_) soon = soon || active(job);
+        if (!soon) {
+            cv_.wait(lock, [&] { return version_ != seen; });
+            return;
+        }
+        lock.unlock();
+        for (int polls = 0; version_ == seen; polls++) {
+            if (polls < 1000) std::this_thread::yield();
+            else std::this_thread::sleep_for(std::chrono::microseconds(20));   // a long kernel
+        }
+        lock.lock();
+    }
+
+    void serve() {
+        std::unique_lock<Spin> lock(mu_);
+        while (in_call_) {
+            if (!step(lock, -1)) wait(lock);
+        }
+        members_--;
+    }
+
+    Spin mu_;
+    std::condition_variable_any cv_;
+    std::atomic<uint64_t> version_{0};
+    Job jobs_[JOBS];
+    uint64_t orders_ = 0;
+    int members_ = 0;
+    bool in_call_ = false;
 };
 
 class HostPipe {
@@ -238,9 +421,12 @@ class HostPipe {
         };
         const size_t total = std::max(row, bytes) * rows;
         const int k = (int)std::max<uint64_t>(1, std::min<uint64_t>(nthreads_, total >> 20));
-        Team team;
-        team.start(k - 1, nthreads_, [&, k](int t) { copy(rows * t / k, rows * (t + 1) / k); }, k);
-        team.finish();
+        if (k > 1) {
+            crew_->post(Crew::INPUT, k - 1, k, [&, k](int t) { copy(rows * t / k, rows * (t + 1) / k); });
+            (void)crew_->finish(Crew::INPUT);
+        } else {
+            copy(0, rows);
+        }
         chk(hipMemcpyAsync(dev, pin, pitch * rows, hipMemcpyHostToDevice, compute_), "copy from pinned buffer");
         if (several_) {
             chk(hipEventRecord(consumed_[s], compute_), "record");
@@ -314,13 +500,14 @@ class HostPipe {
         join(1);
         if (in_flight_) chk(hipStreamSynchronize(compute_), "copies on the compute stream");
         in_flight_ = false;
+        crew_->end_call();
     }
 
     // Ends whatever is in flight without reporting errors (used when a call is unwinding).
     void drain_noexcept() {
+        crew_->cancel();
+        crew_->end_call();
         for (int s = 0; s < 2; s++) {
-            if (batches_[s].team.total) batches_[s].team.finish();
-            batches_[s].error = hipSuccess;
             if (in_used_[s]) (void)hipEventSynchronize(consumed_[s]);
         }
         if (copy_) (void)hipStreamSynchronize(copy_);
@@ -334,51 +521,11 @@ class HostPipe {
     static constexpr int MAX_CHUNKS = 16;
     static constexpr size_t CHUNK_BYTES = (size_t)2 << 20;   // host bytes per chunk, at least
 
-    // Shares 0 .. total - 1 of some work, taken by up to `helpers` pool threads and by the thread that finishes it.
-    struct Team {
-        std::function<void(int)> share;
-        int total = 0;
-        std::atomic<int> next{0};
-        int helping = 0;
-        std::mutex mu;
-        std::condition_variable cv;
-
-        void work() {
-            for (int i = next++; i < total; i = next++) share(i);
-        }
-        void start(int helpers, int most, std::function<void(int)> f, int n) {
-            share = std::move(f);
-            next = 0;
-            total = n;
-            for (int h = 0; h < helpers; h++) {
-                {
-                    std::lock_guard<std::mutex> lock(mu);
-                    helping++;
-                }
-                auto leave = [this] {
-                    std::lock_guard<std::mutex> lock(mu);
-                    if (--helping == 0) cv.notify_all();
-                };
-                if (!CopyPool::get().run([this, leave] { work(); leave(); }, most)) leave();
-            }
-        }
-        void finish() {
-            work();
-            std::unique_lock<std::mutex> lock(mu);
-            cv.wait(lock, [&] { return helping == 0; });
-            total = 0;
-        }
-    };
-
     struct Batch {
         std::vector<Part> parts;   // dev = pinned source rows, at the device rows' stride
         uint64_t rows = 0;
         int chunks = 1, nthreads = 1;
         bool direct = false;           // transferred on the compute stream
-        std::atomic<int> ready{0};     // chunks that have arrived; -1: an error ended the wait
-        std::atomic_flag waiting = ATOMIC_FLAG_INIT;   // some thread waits for the next chunk
-        hipError_t error = hipSuccess;
-        Team team;
     };
 
     static void chk(hipError_t e, const char *what) {
@@ -423,45 +570,22 @@ class HostPipe {
         copy_rows(b, 0, b.rows);
     }
 
-    // Has pool threads take the batch's shares (chunk * nthreads + part of the chunk) as the chunks arrive: of the threads
-    // that need a chunk, one waits for its event and the others for that one.
+    // Has the crew take the batch's shares (chunk * nthreads + part of the chunk) as the chunks arrive.
     void start(int s) {
         Batch &b = batches_[s];
-        b.ready = 0;
-        b.error = hipSuccess;
-        auto share = [&b, s, this](int i) {
+        auto share = [&b](int i) {
             const int c = i / b.nthreads, part = i % b.nthreads;
-            int ready, polls = 0;
-            while ((ready = b.ready.load(std::memory_order_acquire)) >= 0 && ready <= c) {
-                if (!b.waiting.test_and_set(std::memory_order_acquire)) {
-                    ready = b.ready.load(std::memory_order_acquire);
-                    if (ready >= 0 && ready <= c) {
-                        hipError_t e = hipSetDevice(device_);
-                        if (e == hipSuccess) e = hipEventSynchronize(arrived_[s][ready]);
-                        if (e != hipSuccess) b.error = e;
-                        b.ready.store(e == hipSuccess ? ready + 1 : -1, std::memory_order_release);
-                    }
-                    b.waiting.clear(std::memory_order_release);
-                } else if (++polls < 1000) {
-                    std::this_thread::yield();
-                } else {
-                    std::this_thread::sleep_for(std::chrono::microseconds(20));   // a long kernel
-                }
-            }
-            if (ready < 0) return;
             const uint64_t a = b.rows * c / b.chunks, n = b.rows * (c + 1) / b.chunks - a;
             copy_rows(b, a + n * part / b.nthreads, a + n * (part + 1) / b.nthreads);
         };
-        b.team.start(b.nthreads, nthreads_, share, b.chunks * b.nthreads);
+        auto arrive = [this, s](int c) {
+            const hipError_t e = hipSetDevice(device_);
+            return e == hipSuccess ? hipEventSynchronize(arrived_[s][c]) : e;
+        };
+        crew_->post(Crew::OUTPUT + s, b.nthreads, b.chunks * b.nthreads, share, b.nthreads, arrive);
     }
 
-    void join(int s) {
-        Batch &b = batches_[s];
-        if (b.team.total) b.team.finish();
-        const hipError_t e = b.error;
-        b.error = hipSuccess;
-        chk(e, "copy to pinned buffer");
-    }
+    void join(int s) { chk(crew_->finish(Crew::OUTPUT + s), "copy to pinned buffer"); }
 
     hipStream_t compute_ = nullptr, copy_ = nullptr;
     int device_ = 0;
@@ -474,6 +598,7 @@ class HostPipe {
     bool used_[2] = {false, false}, in_used_[2] = {false, false};
     size_t in_at_ = 0;   // bytes of the next batch's pinned input buffer in use
     Batch batches_[2];
+    std::shared_ptr<Crew> crew_ = std::make_shared<Crew>();   // its threads may leave after the pipeline is gone
     uint64_t batch_ = 0;
     int pending_ = -1;
     int nthreads_ = 1;
