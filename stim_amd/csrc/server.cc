@@ -408,6 +408,8 @@ int mfs_server_copy_result(mfs_server *v, uint64_t id, uint8_t *dets, size_t det
         // Through pinned buffers, a batch of rows at a time.
         const size_t row = r.det_row + r.obs_row;
         if (!row || !r.shots) return;
+        if ((dets && dets_stride < r.det_row) || (obs && obs_stride < r.obs_row))
+            throw std::runtime_error("copy result: rows are longer than their stride");
         const uint64_t batch = std::min<uint64_t>(r.shots, std::max<uint64_t>(1, PIPE_BATCH_BYTES / row));
         struct Drain {
             HostPipe &p;
