@@ -14,6 +14,7 @@
 #include <chrono>
 #include <deque>
 #include <map>
+#include <mutex>
 #include <thread>
 #include <unordered_map>
 
@@ -117,7 +118,9 @@ struct mfs_server {
     std::vector<uint64_t> active, finished;
     Arena arena;
     hipStream_t stream = nullptr;
-    HostPipe pipe;   // results on their way to host rows
+    // Results on their way to host rows: one caller's at a time, since finished requests may be copied from several threads.
+    HostPipe pipe;
+    std::mutex copying;
     DevBuf d_jobs, d_prefix, d_counter;
     SymDevParams *h_jobs = nullptr;   // pinned staging for the work list
     uint64_t *h_prefix = nullptr;
@@ -411,6 +414,7 @@ int mfs_server_copy_result(mfs_server *v, uint64_t id, uint8_t *dets, size_t det
         if ((dets && dets_stride < r.det_row) || (obs && obs_stride < r.obs_row))
             throw std::runtime_error("copy result: rows are longer than their stride");
         const uint64_t batch = std::min<uint64_t>(r.shots, std::max<uint64_t>(1, PIPE_BATCH_BYTES / row));
+        std::lock_guard<std::mutex> lock(v->copying);
         struct Drain {
             HostPipe &p;
             ~Drain() { p.drain_noexcept(); }

@@ -1,4 +1,7 @@
-"""Copying served results to the host: strides that a row does not fit in are refused."""
+"""Copying served results to the host: strides that a row does not fit in are refused, and several threads may copy finished
+requests of one server at once."""
+
+import threading
 
 import numpy as np
 import pytest
@@ -41,3 +44,24 @@ def test_rows_longer_than_their_stride_are_refused(shots):
     assert np.array_equal(d, dets) and (o == 0xA5).all()
     N.check(copy(srv._h, r, None, 0, o.ctypes.data, 1))
     assert np.array_equal(o, obs)
+
+
+def test_results_copied_by_several_threads_at_once():
+    """Requests of one batch and of several, small ones on the compute stream and large ones on the copy stream."""
+    srv, ids = _served([(11, 160_001), (3, 501), (9, 60_000), (13, 90_001), (5, 1), (7, 30_003)])
+    want = [srv.result(r) for r in ids]
+    got = {}
+    start = threading.Barrier(len(ids))
+
+    def copy(k):
+        start.wait()
+        got[k] = [srv.result(ids[k]) for _ in range(3)]
+
+    threads = [threading.Thread(target=copy, args=(k,)) for k in range(len(ids))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(timeout=60)
+    for k, w in enumerate(want):
+        for g in got[k]:
+            assert np.array_equal(g[0], w[0]) and np.array_equal(g[1], w[1]), k
