@@ -341,10 +341,11 @@ static void convert_host(mfs_m2d &c, uint64_t shots, const uint8_t *meas, size_t
     const bool tight = c.whole_fits() && c.kernel_mode != 2;
     const size_t in_pitch = tight ? c.in_row() : std::max<size_t>(c.in_vec_stride(), 16);
     const size_t srow = sweep ? c.sweep_row() : 0, out_row = (n_out + 7) / 8, obs_row = (n_obs + 7) / 8;
-    // Batches of about HOST_CONVERT_BYTES of host rows each way, so that the host's copies of one overlap the transfers
-    // and the kernel of another.
+    // Batches of about HOST_CONVERT_BYTES each way, so that the host's copies of one overlap the transfers and the kernel of
+    // another: of all that a shot brings in (its sweep bits too), on the host or in the pitched buffers, and of what it gets.
     constexpr size_t HOST_CONVERT_BYTES = (size_t)16 << 20;
-    const size_t host_row = std::max<size_t>({bytes ? c.M : c.in_row(), (packed ? out_row : n_out) + (packed ? obs_row : n_obs), 1});
+    const size_t host_row = std::max<size_t>({(bytes ? c.M : c.in_row()) + srow, in_pitch + srow,
+                                              packed ? out_row + obs_row : (size_t)n_out + n_obs, 1});
     const uint64_t batch = std::min<uint64_t>(shots, std::max<uint64_t>(32, HOST_CONVERT_BYTES / host_row / 32 * 32));
     struct Drain {
         HostPipe &p;
