@@ -19,9 +19,10 @@ struct mfs_batch {
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     DevBuf d_jobs, d_prefix, d_counter, d_advance;
-    // Occupancy levels: jobs grouped by the workgroups per CU their own LDS allows, one persistent
-    // kernel per level (each at the occupancy a plain launch of its jobs would get).
+    // Levels: jobs grouped by their scan (SYM_BATCH_*) and by the workgroups per CU their own LDS allows, one
+    // persistent kernel per level (each at the occupancy a plain launch of its jobs would get).
     struct Level {
+        uint32_t kind;
         size_t lds;
         uint32_t grid;
         uint32_t first, count;   // jobs [first, first + count) of the uploaded list
@@ -80,6 +81,7 @@ struct mfs_batch {
             double cost;
             uint32_t job;
             size_t lds;
+            uint32_t kind;
             int per_cu;
             mfs_sampler *s;
         };
@@ -109,8 +111,9 @@ struct mfs_batch {
             const double S = r.P.shots_per_tile;
             // Per-tile cost estimate: hits applied plus output bytes written, plus a fixed overhead.
             const double cost = S * (hits * 16.0 + r.P.det_row_bytes + r.P.obs_row_bytes) + 4096.0;
-            items.push_back({r.P, r.tiles, cost, j, std::max<size_t>(r.lds_scan, 64),
-                             sym_batch_blocks_per_cu(std::max<size_t>(r.lds_scan, 64)), s});
+            const uint32_t kind = sym_batch_kind(r.P);
+            items.push_back({r.P, r.tiles, cost, j, std::max<size_t>(r.lds_scan, 64), kind,
+                             sym_batch_blocks_per_cu(kind, std::max<size_t>(r.lds_scan, 64)), s});
         }
         for (auto &kv : next_tile) {
             uint64_t start = 0;
@@ -118,9 +121,10 @@ struct mfs_batch {
                 if (e.first == kv.first) start = e.second;
             advance.push_back({kv.first, kv.second - start});
         }
-        // Levels by occupancy (highest first); inside a level, heaviest tiles first so the tail of the
+        // Levels by scan and occupancy (highest first); inside a level, heaviest tiles first so the tail of the
         // run is made of light tiles.
         std::stable_sort(items.begin(), items.end(), [](const Item &a, const Item &b) {
+            if (a.kind != b.kind) return a.kind > b.kind;
             return a.per_cu != b.per_cu ? a.per_cu > b.per_cu : a.cost > b.cost;
         });
         std::vector<SymDevParams> params;
@@ -130,9 +134,9 @@ struct mfs_batch {
         lds = 64;
         for (size_t i = 0; i < items.size();) {
             size_t e = i;
-            Level lv{0, 0, (uint32_t)i, 0, 0};
+            Level lv{items[i].kind, 0, 0, (uint32_t)i, 0, 0};
             std::vector<uint64_t> pre{0};
-            while (e < items.size() && items[e].per_cu == items[i].per_cu) {
+            while (e < items.size() && items[e].kind == items[i].kind && items[e].per_cu == items[i].per_cu) {
                 params.push_back(items[e].P);
                 pre.push_back(pre.back() + items[e].tiles);
                 uint64_t a = 0;
@@ -174,7 +178,7 @@ struct mfs_batch {
             check(hipGetDevice(&dev), "device");
             check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "device");
             for (Level &lv : levels) {
-                const uint64_t resident = (uint64_t)std::max(cus, 1) * (uint64_t)sym_batch_blocks_per_cu(lv.lds);
+                const uint64_t resident = (uint64_t)std::max(cus, 1) * (uint64_t)sym_batch_blocks_per_cu(lv.kind, lv.lds);
                 lv.grid = persistent ? (uint32_t)std::min<uint64_t>(resident, lv.tiles) : (uint32_t)lv.tiles;
                 grid += lv.grid;
             }
@@ -200,7 +204,7 @@ struct mfs_batch {
         // Level l's jobs start at levels[l].first; its prefix array (count + 1 entries) at first + l.
         for (size_t l = 0; l < levels.size(); l++) {
             const Level &lv = levels[l];
-            check(launch_sym_batch(d_jobs.as<SymDevParams>() + lv.first, d_prefix.as<uint64_t>() + lv.first + l,
+            check(launch_sym_batch(lv.kind, d_jobs.as<SymDevParams>() + lv.first, d_prefix.as<uint64_t>() + lv.first + l,
                                    d_advance.as<uint64_t>() + lv.first, lv.count, d_counter.as<uint32_t>() + l,
                                    lv.grid, lv.lds, stream),
                   "batch launch");

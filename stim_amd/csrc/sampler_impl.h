@@ -41,9 +41,9 @@ hipError_t launch_sym_sample(const SymDevParams &P, uint32_t tiles, size_t lds, 
 hipError_t launch_sym_fixed(const SymDevParams &P, const uint64_t *off, const uint32_t *cols, uint32_t tiles,
                             size_t lds, hipStream_t stream);
 hipError_t launch_sym_scan(const SymDevParams &P, uint32_t tiles, size_t lds, hipStream_t stream, bool fast);
-hipError_t launch_sym_batch(SymDevParams *jobs, const uint64_t *prefix, const uint64_t *advance, uint32_t njobs,
+hipError_t launch_sym_batch(uint32_t kind, SymDevParams *jobs, const uint64_t *prefix, const uint64_t *advance, uint32_t njobs,
                             uint32_t *counter, uint32_t grid, size_t lds, hipStream_t stream);
-int sym_batch_blocks_per_cu(size_t lds);
+int sym_batch_blocks_per_cu(uint32_t kind, size_t lds);
 hipError_t launch_sym_count(const uint8_t *det, uint32_t det_row, const uint8_t *obs, uint32_t obs_row, uint64_t rows,
                             uint32_t *counts, hipStream_t stream);
 hipError_t launch_sym_fill(const uint8_t *det, uint32_t det_row, const uint8_t *obs, uint32_t obs_row, uint64_t rows,

@@ -125,7 +125,7 @@ struct mfs_server {
     SymDevParams *h_jobs = nullptr;   // pinned staging for the work list
     uint64_t *h_prefix = nullptr;
     size_t h_cap = 0;
-    std::map<size_t, uint32_t> grid_for_lds;
+    std::map<std::pair<uint32_t, size_t>, uint32_t> grid_for_lds;   // by scan and LDS bytes
     // Device time of the serving launches (HIP events around each) and the row bytes they wrote.
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     double kernel_ms = 0;
@@ -220,13 +220,14 @@ struct mfs_server {
         }
     }
 
-    uint32_t grid(size_t lds, uint64_t tiles) {
-        auto it = grid_for_lds.find(lds);
+    uint32_t grid(uint32_t kind, size_t lds, uint64_t tiles) {
+        auto it = grid_for_lds.find({kind, lds});
         if (it == grid_for_lds.end()) {
             int dev = 0, cus = 0;
             check(hipGetDevice(&dev), "device");
             check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "device");
-            it = grid_for_lds.emplace(lds, (uint32_t)std::max(cus, 1) * (uint32_t)sym_batch_blocks_per_cu(lds)).first;
+            const uint32_t all = (uint32_t)std::max(cus, 1) * (uint32_t)sym_batch_blocks_per_cu(kind, lds);
+            it = grid_for_lds.emplace(std::make_pair(kind, lds), all).first;
         }
         return (uint32_t)std::min<uint64_t>(it->second, tiles);
     }
@@ -270,21 +271,32 @@ struct mfs_server {
             if (left <= 0) break;
             left -= give(id, left);
         }
-        // Work list: one job per request chunk.
+        // Work list: one job per request chunk, one launch per scan that they need (mostly a single one).
+        std::stable_sort(take.begin(), take.end(), [&](const auto &a, const auto &b) {
+            return sym_batch_kind(reqs.at(a.first).P) < sym_batch_kind(reqs.at(b.first).P);
+        });
         if (take.size() > h_cap) {
             if (h_jobs) (void)hipHostFree(h_jobs);
             if (h_prefix) (void)hipHostFree(h_prefix);
             h_cap = std::max<size_t>(take.size(), 2 * h_cap);
             check(hipHostMalloc((void **)&h_jobs, h_cap * sizeof(SymDevParams), hipHostMallocDefault), "pinned");
-            check(hipHostMalloc((void **)&h_prefix, (h_cap + 1) * sizeof(uint64_t), hipHostMallocDefault), "pinned");
+            check(hipHostMalloc((void **)&h_prefix, (h_cap + SYM_BATCH_KINDS) * sizeof(uint64_t), hipHostMallocDefault), "pinned");
             d_jobs.ensure(h_cap * sizeof(SymDevParams));
-            d_prefix.ensure((h_cap + 1) * sizeof(uint64_t));
+            d_prefix.ensure((h_cap + SYM_BATCH_KINDS) * sizeof(uint64_t));
         }
-        size_t lds = 64;
-        h_prefix[0] = 0;
+        struct Launch {
+            uint32_t kind;
+            size_t first, lds;   // its first job; its prefix sums start at first + its number in the list
+        };
+        std::vector<Launch> launches;
         for (size_t k = 0; k < take.size(); k++) {
             Req &r = reqs.at(take[k].first);
             SymDevParams P = r.P;
+            const uint32_t kind = sym_batch_kind(P);
+            if (launches.empty() || launches.back().kind != kind) {
+                launches.push_back({kind, k, 64});
+                h_prefix[k + launches.size() - 1] = 0;
+            }
             const uint64_t a = r.next_tile;
             const uint64_t s0 = a * P.shots_per_tile;
             P.tile0 = a;
@@ -292,20 +304,24 @@ struct mfs_server {
             P.dets.ptr = r.dets + s0 * r.det_row;
             P.obs.ptr = r.obs + s0 * r.obs_row;
             h_jobs[k] = P;
-            h_prefix[k + 1] = h_prefix[k] + take[k].second;
+            uint64_t *const sum = h_prefix + k + launches.size() - 1;
+            sum[1] = sum[0] + take[k].second;
             bytes_written += std::min<uint64_t>(take[k].second * P.shots_per_tile, P.shots) * (r.det_row + r.obs_row);
-            lds = std::max(lds, r.lds);
+            launches.back().lds = std::max(launches.back().lds, r.lds);
             r.next_tile += take[k].second;
         }
-        const uint64_t tiles = h_prefix[take.size()];
         check(hipMemcpyAsync(d_jobs.p, h_jobs, take.size() * sizeof(SymDevParams), hipMemcpyHostToDevice, stream),
               "upload work list");
-        check(hipMemcpyAsync(d_prefix.p, h_prefix, (take.size() + 1) * sizeof(uint64_t), hipMemcpyHostToDevice, stream),
-              "upload work list");
-        const uint32_t g = grid(lds, tiles);
+        check(hipMemcpyAsync(d_prefix.p, h_prefix, (take.size() + launches.size()) * sizeof(uint64_t), hipMemcpyHostToDevice,
+                             stream), "upload work list");
         check(hipEventRecord(ev0, stream), "event");
-        check(launch_sym_batch(d_jobs.as<SymDevParams>(), d_prefix.as<uint64_t>(), nullptr, (uint32_t)take.size(),
-                               d_counter.as<uint32_t>(), g, lds, stream), "serving step");
+        for (size_t l = 0; l < launches.size(); l++) {
+            const Launch &x = launches[l];
+            const size_t end = l + 1 < launches.size() ? launches[l + 1].first : take.size();
+            check(launch_sym_batch(x.kind, d_jobs.as<SymDevParams>() + x.first, d_prefix.as<uint64_t>() + x.first + l, nullptr,
+                                   (uint32_t)(end - x.first), d_counter.as<uint32_t>(),
+                                   grid(x.kind, x.lds, h_prefix[end + l]), x.lds, stream), "serving step");
+        }
         check(hipEventRecord(ev1, stream), "event");
         check(hipStreamSynchronize(stream), "serving step");
         float ms = 0;

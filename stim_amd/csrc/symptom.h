@@ -161,6 +161,11 @@ struct SymDevParams {
     uint32_t mech_null, mech_runs;
     uint32_t direct_null;          // first of 64 null entries (no flips; their fields name words spread over a row)
 };
+// The scan that a batch job's tiles run, the one of a plain launch; a launch of the batch kernel takes jobs of one kind.
+enum : uint32_t { SYM_BATCH_DIRECT, SYM_BATCH_RECORDS, SYM_BATCH_MECHS, SYM_BATCH_GENERIC, SYM_BATCH_KINDS };
+inline uint32_t sym_batch_kind(const SymDevParams &P) {
+    return P.direct ? SYM_BATCH_DIRECT : P.orecs ? SYM_BATCH_RECORDS : P.mechs ? SYM_BATCH_MECHS : SYM_BATCH_GENERIC;
+}
 // Direct site entry (16 bytes): x = d0 | d1 << 14 | nout << 28, y = d2 | d3 << 14, z = d4 | d5 << 14 with the
 // detectors that the site's basis columns reach (unused fields repeat d0, or are 0), w = byte j: bit e < 6
 // set when basis column j flips detector d_e, bits 6 and 7 when it flips observable 0 and 1.

@@ -1151,33 +1151,34 @@ __global__ __launch_bounds__(NT, 5) void sym_scan_fast_kernel(SymDevParams P) {
     scan_tile_fast<OBS, DIRECT>(P, blockIdx.x, lds);
 }
 
-// A batch job's tile: the specialised scan for jobs whose sampler has outcome records (the job's
-// plain launch runs that kernel too; rows are identical either way), the generic scan otherwise.
+// A batch job's tile, on the scan that the job's plain launch runs. A launch's jobs are all of one KIND (symptom.h): a kernel
+// with the bodies of every scan keeps 5 VGPRs and 24 bytes a lane of scratch that no scan needs by itself.
+template <uint32_t KIND>
 __device__ __forceinline__ void batch_tile(const SymDevParams &P, uint32_t btile, uint32_t *lds) {
-    if (P.direct) {
-        if (P.obs_mode != 0) scan_tile_fast<true, true>(P, btile, lds);
-        else scan_tile_fast<false, true>(P, btile, lds);
-    } else if (P.orecs) {
-        if (P.obs_mode != 0) scan_tile_fast<true, false>(P, btile, lds);
-        else scan_tile_fast<false, false>(P, btile, lds);
-    } else if (P.mechs) {
+    if (KIND == SYM_BATCH_MECHS) {
         if (P.obs_mode != 0) scan_tile_mechs<true>(P, btile, lds);
         else scan_tile_mechs<false>(P, btile, lds);
-    } else if (P.wave_split) {
-        scan_tile_waves(P, btile, lds);
+    } else if (KIND == SYM_BATCH_GENERIC) {
+        if (P.wave_split) scan_tile_waves(P, btile, lds);
+        else scan_tile(P, btile, lds);
     } else {
-        scan_tile(P, btile, lds);
+        if (P.obs_mode != 0) scan_tile_fast<true, KIND == SYM_BATCH_DIRECT>(P, btile, lds);
+        else scan_tile_fast<false, KIND == SYM_BATCH_DIRECT>(P, btile, lds);
     }
 }
 
 // Batched form: many launches (jobs, possibly of different circuits) in one kernel; job j owns global
 // tiles [prefix[j], prefix[j+1]). Persistent schedule (grid smaller than the tile count): workgroups
-// claim chunks of BATCH_CHUNK consecutive tiles from a counter, caching the current job so the search
+// claim chunks of up to BATCH_CHUNK consecutive tiles from a counter, caching the current job so the search
 // only runs when a chunk crosses into another job, and leave once the counter passes the last tile.
 // With a grid of one workgroup per tile, each workgroup samples its own tile.
+// A chunk is half of what a workgroup gets on average, so that a launch of few tiles does not end with one workgroup's
+// eight in a row (400,000, 200,000 and 300,000 shots of 80, 420 and 16 bytes, 4981 tiles: 0.163 ms with chunks of 8, 0.090
+// with this rule).
 constexpr uint32_t BATCH_CHUNK = 8;
 
-__global__ __launch_bounds__(NT, 6) void sym_batch_kernel(const SymDevParams *__restrict__ jobs,
+template <uint32_t KIND>
+__global__ __launch_bounds__(NT, KIND == SYM_BATCH_DIRECT ? 5 : 6) void sym_batch_kernel(const SymDevParams *__restrict__ jobs,
                                                        const uint64_t *__restrict__ prefix, uint32_t njobs,
                                                        uint32_t *counter) {
     extern __shared__ __align__(16) uint32_t lds[];
@@ -1195,19 +1196,20 @@ __global__ __launch_bounds__(NT, 6) void sym_batch_kernel(const SymDevParams *__
         const uint32_t j = __builtin_amdgcn_readfirstlane(a);
         if (t < total) {
             const SymDevParams P = jobs[j];
-            batch_tile(P, (uint32_t)(t - prefix[j]), lds);
+            batch_tile<KIND>(P, (uint32_t)(t - prefix[j]), lds);
         }
         return;
     }
+    const uint32_t chunk = (uint32_t)max<uint64_t>(1, min<uint64_t>(BATCH_CHUNK, total / (2 * gridDim.x)));
     uint32_t j = 0;
     uint64_t lo = 0, hi = 0;   // tile range of job j (empty until the first search)
     for (;;) {
         __syncthreads();
-        if (threadIdx.x == 0) next = atomicAdd(counter, BATCH_CHUNK);
+        if (threadIdx.x == 0) next = atomicAdd(counter, chunk);
         __syncthreads();
         const uint64_t t0 = next;
         if (t0 >= total) break;
-        const uint64_t t1 = t0 + BATCH_CHUNK < total ? t0 + BATCH_CHUNK : total;
+        const uint64_t t1 = t0 + chunk < total ? t0 + chunk : total;
         for (uint64_t t = t0; t < t1; t++) {
             if (t < lo || t >= hi) {
                 uint32_t a = 0, b = njobs;
@@ -1222,7 +1224,7 @@ __global__ __launch_bounds__(NT, 6) void sym_batch_kernel(const SymDevParams *__
             }
             if (t != t0) __syncthreads();   // the previous tile's rows are written before the image is reused
             const SymDevParams P = jobs[j];
-            batch_tile(P, (uint32_t)(t - lo), lds);
+            batch_tile<KIND>(P, (uint32_t)(t - lo), lds);
         }
     }
 }
@@ -1414,12 +1416,19 @@ hipError_t launch_sym_scan(const SymDevParams &P, uint32_t tiles, size_t lds, hi
     return hipGetLastError();
 }
 
+using BatchKernel = void (*)(const SymDevParams *, const uint64_t *, uint32_t, uint32_t *);
+static BatchKernel batch_kernel(uint32_t kind) {
+    constexpr BatchKernel kernels[SYM_BATCH_KINDS] = {sym_batch_kernel<SYM_BATCH_DIRECT>, sym_batch_kernel<SYM_BATCH_RECORDS>,
+                                                      sym_batch_kernel<SYM_BATCH_MECHS>, sym_batch_kernel<SYM_BATCH_GENERIC>};
+    return kernels[kind];
+}
+
 // The dynamic LDS attribute is set by sym_batch_blocks_per_cu (before any graph capture).
 // advance == null: no tile-base update (callers that set the bases themselves).
-hipError_t launch_sym_batch(SymDevParams *jobs, const uint64_t *prefix, const uint64_t *advance, uint32_t njobs,
+hipError_t launch_sym_batch(uint32_t kind, SymDevParams *jobs, const uint64_t *prefix, const uint64_t *advance, uint32_t njobs,
                             uint32_t *counter, uint32_t grid, size_t lds, hipStream_t stream) {
     hipLaunchKernelGGL(sym_batch_reset_kernel, dim3(1), dim3(64), 0, stream, counter);
-    hipLaunchKernelGGL(sym_batch_kernel, dim3(grid), dim3(NT), lds, stream, jobs, prefix, njobs, counter);
+    hipLaunchKernelGGL(batch_kernel(kind), dim3(grid), dim3(NT), lds, stream, jobs, prefix, njobs, counter);
     if (advance)
         hipLaunchKernelGGL(sym_batch_advance_kernel, dim3((njobs + 255) / 256), dim3(256), 0, stream, jobs, advance,
                            njobs);
@@ -1428,11 +1437,12 @@ hipError_t launch_sym_batch(SymDevParams *jobs, const uint64_t *prefix, const ui
 
 // Raises (never lowers) the batch kernel's dynamic-LDS limit to lds, then returns how many of its
 // workgroups with that much LDS fit on one CU. Every launch size is announced through here first.
-int sym_batch_blocks_per_cu(size_t lds) {
-    static size_t reserved = 0;
-    (void)reserve_lds((const void *)sym_batch_kernel, lds, reserved);
+int sym_batch_blocks_per_cu(uint32_t kind, size_t lds) {
+    static size_t reserved[SYM_BATCH_KINDS] = {};
+    const BatchKernel kernel = batch_kernel(kind);
+    (void)reserve_lds((const void *)kernel, lds, reserved[kind]);
     int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, sym_batch_kernel, NT, lds) != hipSuccess) return 1;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, NT, lds) != hipSuccess) return 1;
     return n > 0 ? n : 1;
 }
 
