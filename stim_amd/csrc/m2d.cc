@@ -188,10 +188,10 @@ struct mfs_m2d {
     std::vector<uint32_t> ovf;
     // Tables of the whole-record kernel (m2d.h).
     std::vector<uint32_t> terms;
-    std::vector<uint2> block_info;
+    std::vector<uint2> entries, block_info;
     std::vector<uint4> spill;
     uint32_t spill_slots = 0, slow = 0;
-    DevBuf d_terms, d_block_info, d_spill;
+    DevBuf d_terms, d_entries, d_block_info, d_spill;
     DevBuf d_cols, d_ovf, d_in, d_out, d_obs, d_sweep;
     // Windowed kernel (no sweep bits), one plan per output layout: 0 = observables appended, 1 =
     // observables separate, 2 = detectors only, 3 = observables appended and separate. kernel_mode:
@@ -240,6 +240,7 @@ struct mfs_m2d {
         P.sweep_row_bytes = (uint32_t)sweep_row();
         P.sweep_blocks = sweep_blocks();
         P.terms = const_cast<DevBuf &>(d_terms).as<uint32_t>();
+        P.entries = const_cast<DevBuf &>(d_entries).as<uint2>();
         P.block_info = const_cast<DevBuf &>(d_block_info).as<uint2>();
         P.spill = const_cast<DevBuf &>(d_spill).as<uint4>();
         P.spill_chunks = (uint32_t)spill.size();
@@ -263,6 +264,7 @@ struct mfs_m2d {
         }
         const uint32_t z = m2d_padded(zero), none = z | (z << 16);
         terms.assign((size_t)64 * std::max(tb, 1u), none);
+        entries.assign((size_t)32 * std::max(tb, 1u), make_uint2(none, none));
         block_info.assign(std::max(tb, 1u), make_uint2(0, 0));
         uint32_t slot = 0;
         for (uint32_t j = 0; j < cols; j++) {
@@ -288,6 +290,7 @@ struct mfs_m2d {
             }
             terms[(size_t)(j % 32) * tb + b] = listed ? 0xFFFFFFFFu : w[0] | (w[1] << 16);
             terms[(size_t)(32 + j % 32) * tb + b] = w[2] | (w[3] << 16);
+            entries[j] = make_uint2(terms[(size_t)(j % 32) * tb + b], w[2] | (w[3] << 16));
             if (invert[j]) block_info[b].x |= 1u << (j % 32);
         }
     }
@@ -477,6 +480,7 @@ int mfs_m2d_compile(const char *stim_text, size_t len, int skip_reference_sample
         mfs_sampler::upload(c->d_cols, c->cols, "m2d columns");
         mfs_sampler::upload(c->d_ovf, c->ovf, "m2d overflow terms");
         mfs_sampler::upload(c->d_terms, c->terms, "m2d terms");
+        mfs_sampler::upload(c->d_entries, c->entries, "m2d entries");
         mfs_sampler::upload(c->d_block_info, c->block_info, "m2d blocks");
         mfs_sampler::upload(c->d_spill, c->spill, "m2d spilled columns");
         for (int l = 0; l < 4; l++) {

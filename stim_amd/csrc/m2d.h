@@ -38,6 +38,7 @@ struct M2dParams {
     uint32_t sweep_blocks;      // ceil(K / 32): LDS word m2d_sweep_word(blocks) + k holds sweep bit k
     // Whole-record kernel (m2d_kernel): blocks of 32 columns (tables below).
     const uint32_t *terms;      // column 32 b + k of block b at [k * total_blocks + b]: up to four LDS words
+    const uint2 *entries;       // the same by column: x = its first plane's entry, y = its second's
     const uint2 *block_info;    // per block: its columns' inversion bits, whether one has more than two words
     const uint4 *spill;         // columns of more than four terms: their words are summed into slots
     uint32_t spill_chunks, spill_slots;

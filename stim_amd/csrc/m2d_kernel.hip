@@ -128,7 +128,7 @@ __device__ __forceinline__ void store_rows(uint32_t (&x)[32], uint8_t *base, uin
 }
 
 // Rows on lanes: a half-wave's lane loads, or stores, the word of its own row (row < valid) of one block. For launches so
-// small that a lane per block leaves most of the chip idle (lanes_by_rows).
+// small that a lane per block leaves most of the chip idle (convert_lanes_by_rows, expand_lanes_by_rows).
 __device__ __forceinline__ uint32_t load_row(const uint8_t *r, uint32_t row_bytes, uint32_t b, bool exact) {
     if (exact && row_bytes < 4) {
         uint32_t v = 0;
@@ -149,16 +149,46 @@ __device__ __forceinline__ void store_row(uint32_t v, uint8_t *r, uint32_t row_b
         if (left > 2) r[2] = (uint8_t)(v >> 16);
     }
 }
-// Loads row blocks [0, blocks) of each subtile into its words from word `at` on.
+// Four consecutive blocks of a lane's row at once, from block b on (those past `blocks` are not used): a half-wave's 32
+// loads, or stores, each touch a line of their own whatever their width.
+typedef uint32_t __attribute__((ext_vector_type(4), aligned(1))) unaligned_u32x4;
+__device__ __forceinline__ void load_row4(uint32_t (&x)[4], const uint8_t *r, uint32_t row_bytes, uint32_t b, uint32_t blocks,
+                                          bool exact) {
+    if (!exact || 4 * b + 16 <= row_bytes) {
+        const u32x4 v = *reinterpret_cast<const unaligned_u32x4 *>(r + 4 * b);
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++) x[k] = v[k];
+    } else {
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++) x[k] = b + k < blocks ? load_row(r, row_bytes, b + k, exact) : 0u;
+    }
+}
+// Loads row blocks [0, blocks) of each subtile into its words from word `at` on: a block a half-wave where all fit at once,
+// else four.
 template <int NT>
 __device__ __forceinline__ void load_by_rows(uint32_t *words, uint32_t subw, uint32_t at, const uint8_t *in,
                                              uint64_t stride, uint32_t row_bytes, uint32_t blocks, bool exact,
                                              uint32_t shots) {
     const uint32_t lane = threadIdx.x & 31, subs = (shots + 31) / 32;
-    for (uint32_t i = threadIdx.x >> 5; i < subs * blocks; i += NT / 32) {
-        const uint32_t t = i / blocks, b = i - t * blocks;
-        const uint32_t x = load_row(in + min(32 * t + lane, shots - 1) * stride, row_bytes, b, exact);
-        words[t * subw + at + 33 * b + lane] = transpose32(x, lane);
+    if (subs * blocks <= NT / 32) {
+        const uint32_t i = threadIdx.x >> 5;
+        if (i < subs * blocks) {
+            const uint32_t t = i / blocks, b = i - t * blocks;
+            const uint32_t x = load_row(in + min(32 * t + lane, shots - 1) * stride, row_bytes, b, exact);
+            words[t * subw + at + 33 * b + lane] = transpose32(x, lane);
+        }
+        return;
+    }
+    const uint32_t groups = (blocks + 3) / 4;
+    for (uint32_t i = threadIdx.x >> 5; i < subs * groups; i += NT / 32) {
+        const uint32_t t = i / groups, b = 4 * (i - t * groups);
+        uint32_t x[4];
+        load_row4(x, in + min(32 * t + lane, shots - 1) * stride, row_bytes, b, blocks, exact);
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++) {
+            const uint32_t v = transpose32(x[k], lane);
+            if (b + k < blocks) words[t * subw + at + 33 * (b + k) + lane] = v;
+        }
     }
 }
 
@@ -182,6 +212,56 @@ __device__ __forceinline__ uint32_t listed_word(const M2dParams &P, const uint32
         v ^= w[m2d_padded(a.x)] ^ w[m2d_padded(a.y)] ^ w[m2d_padded(a.z)] ^ w[m2d_padded(a.w)];
     }
     return v;
+}
+
+// Rows on lanes: each half-wave makes B consecutive blocks of 32 output columns of a subtile (a lane a column, its entry
+// from the table by columns), transposes them and stores each row's words. The first blocks' entries are loaded
+// before the workgroup's rows are.
+template <uint32_t B>
+struct ColumnEntries {
+    uint2 e[B];
+    uint32_t invert[B];
+    __device__ __forceinline__ void load(const M2dParams &P, uint32_t nb, uint32_t b) {
+#pragma unroll
+        for (uint32_t k = 0; k < B; k++) {
+            const uint32_t c = min(b + k, nb - 1);
+            e[k] = P.entries[32 * c + (threadIdx.x & 31)];
+            invert[k] = P.block_info[c].x;
+        }
+    }
+};
+template <bool SLOW, int NT, uint32_t B>
+__device__ __forceinline__ void store_by_rows(const M2dParams &P, const uint32_t *words, uint32_t subw, uint64_t s0,
+                                              uint32_t shots, ColumnEntries<B> &c) {
+    const uint32_t lane = threadIdx.x & 31, subs = (shots + 31) / 32;
+    const uint32_t nb = (P.n_out + 31) / 32, groups = (nb + B - 1) / B, row_bytes = (P.n_out + 7) / 8;
+    for (uint32_t i = threadIdx.x >> 5; i < subs * groups; i += NT / 32) {
+        const uint32_t t = i / groups, b = B * (i - t * groups);
+        const uint32_t *const w = words + t * subw;
+        if (i >= NT / 32) c.load(P, nb, b);
+        uint32_t x[B];
+#pragma unroll
+        for (uint32_t k = 0; k < B; k++) {
+            if (SLOW && c.e[k].x == 0xFFFFFFFFu) x[k] = b + k < nb ? listed_word(P, w, 32 * (b + k) + lane) : 0u;
+            else x[k] = terms_word(w, c.e[k].x) ^ terms_word(w, c.e[k].y);
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < B; k++) {
+            x[k] = transpose32(x[k], lane) ^ c.invert[k];
+            const uint32_t live = P.n_out - min(32 * (b + k), P.n_out);
+            if (live < 32) x[k] &= (1u << live) - 1;
+        }
+        if (32 * t + lane >= shots) continue;
+        uint8_t *const r = P.out + (s0 + 32 * t + lane) * P.out_stride;
+        if (B == 4 && 4 * b + 16 <= row_bytes) {
+            const u32x4 v = {x[0], x[B > 1 ? 1 : 0], x[B > 2 ? 2 : 0], x[B > 3 ? 3 : 0]};
+            *reinterpret_cast<unaligned_u32x4 *>(r + 4 * b) = v;
+        } else {
+#pragma unroll
+            for (uint32_t k = 0; k < B; k++)
+                if (b + k < nb) store_row(x[k], r, row_bytes, b + k);
+        }
+    }
 }
 
 // Separate observable rows (a few columns) of a workgroup's shots: one lane per shot and byte.
@@ -235,6 +315,17 @@ __global__ __launch_bounds__(ROWS_NT ? ROWS_NT : M2D_NT, 4) void m2d_kernel(M2dP
         words[t * subw + m2d_padded(m2d_zero_word(P.blocks, P.sweep_blocks) + 4 + (i - t * P.spill_slots))] = 0;
     }
 
+    // Rows on lanes: this half-wave's first entries, of four blocks where one a half-wave does not do.
+    const uint32_t nb = (P.n_out + 31) / 32;
+    const bool wide = subs * nb > NT / 32;
+    ColumnEntries<4> four;
+    ColumnEntries<1> one;
+    if (ROWS && nb) {
+        const uint32_t i = tid >> 5, groups = (nb + 3) / 4;
+        if (wide) four.load(P, nb, 4 * (i % groups));
+        else one.load(P, nb, i % nb);
+    }
+
     // Rows whose stride covers whole words are read past their last byte (never past the buffer's
     // shots * stride bytes); the bits there belong to no measurement.
     if (ROWS) load_by_rows<NT>(words, subw, 0, P.in + s0 * P.in_stride, P.in_stride, P.in_row_bytes, P.blocks, !P.in_vec, shots);
@@ -280,21 +371,10 @@ __global__ __launch_bounds__(ROWS_NT ? ROWS_NT : M2D_NT, 4) void m2d_kernel(M2dP
         __syncthreads();
     }
 
-    const uint32_t nb = (P.n_out + 31) / 32, TB = P.total_blocks;
-    const uint32_t lane = tid & 31;
-    for (uint32_t i = tid >> 5; ROWS && i < subs * nb; i += NT / 32) {
-        const uint32_t t = i / nb, b = i - t * nb;
-        const uint32_t *const w = words + t * subw;
-        const uint2 info = P.block_info[b];
-        const uint32_t a = (P.terms + (size_t)lane * TB)[b];
-        uint32_t x;
-        if (SLOW && a == 0xFFFFFFFFu) x = listed_word(P, w, 32 * b + lane);
-        else x = terms_word(w, a);
-        if (info.y) x ^= terms_word(w, (P.terms + (size_t)(32 + lane) * TB)[b]);
-        x = transpose32(x, lane) ^ info.x;
-        const uint32_t live = P.n_out - 32 * b;
-        if (live < 32) x &= (1u << live) - 1;
-        if (32 * t + lane < shots) store_row(x, P.out + (s0 + 32 * t + lane) * P.out_stride, (P.n_out + 7) / 8, b);
+    const uint32_t TB = P.total_blocks;
+    if (ROWS) {
+        if (wide) store_by_rows<SLOW, NT, 4>(P, words, subw, s0, shots, four);
+        else store_by_rows<SLOW, NT, 1>(P, words, subw, s0, shots, one);
     }
     for (uint32_t i = tid; !ROWS && i < subs * nb; i += NT) {
         const uint32_t t = i / nb, b = i - t * nb;
@@ -739,24 +819,32 @@ static uint32_t subtiles(uint64_t tiles, uint32_t blocks, size_t subtile_bytes, 
     return (uint32_t)std::max<uint64_t>(g, 1);
 }
 
-// Small launches put rows on lanes, a half-wave per block: a lane per block takes a wave through two transposes of 500
-// instructions (5 us) while most SIMDs have no wave at all. Up to 256 subtiles, one workgroup per CU, of 1024 lanes: up to
-// four blocks for each of its 32 half-waves that is faster; beyond, with 512 lanes, as far as its 16 half-waves have a
-// block or two and the launch has less than a wave of blocks for each SIMD. Conversion, rows | blocks on lanes: 4 blocks
-// per subtile, 4000 shots 6.2 | 9.1 us, 120,000 shots 8.8 | 11.1; 26 blocks, 4000 shots 6.3 | 9.9, 16,000 shots 7.7 | 9.8,
-// 120,000 shots 24 | 16.5; 92 blocks, 4000 shots 8.4 | 9.2, 16,000 shots 12.5 | 10.8; 127 blocks, 250 shots 10.2 | 9.4; 508 blocks, 250 shots 25 | 11.6.
-// Expansion: 4 blocks, 4000 shots 7.9 | 15.7 us, 250,000 shots 15.1 (1024 lanes: 21.8) | 25.5.
-// 0: blocks on lanes.
-static int lanes_by_rows(uint64_t tiles, uint32_t blocks) {
+// Small launches put rows on lanes (0: blocks on lanes): a lane per block takes a wave through two transposes of 500
+// instructions (5 us) while most SIMDs have no wave at all. Rows on lanes pay for a line per row and group of blocks.
+// Expansion, a block a half-wave. Up to 256 subtiles, one workgroup per CU, of 1024 lanes: up to four blocks for each of its
+// 32 half-waves that is faster; beyond, with 512 lanes, as far as its 16 half-waves have a block or two and the launch has
+// less than a wave of blocks for each SIMD. Rows | blocks on lanes: 4 blocks per subtile, 4000 shots 7.9 | 15.7 us,
+// 250,000 shots 15.1 (1024 lanes: 21.8) | 25.5.
+static int expand_lanes_by_rows(uint64_t tiles, uint32_t blocks) {
     if (tiles <= 256) return blocks <= 112 ? 1024 : 0;
     return blocks <= 32 && tiles * blocks * ((blocks + 15) / 16) <= 48 * 1024 ? 512 : 0;
+}
+// Conversion, four blocks a half-wave. One subtile a CU: 1024 lanes, while those are no more than two rounds (rows | blocks on
+// lanes, 4000 shots: 69 blocks 7.5 | 9.3 us, 138 blocks 7.9 | 9.2, 193 blocks 9.1 | 9.3, 313 blocks 11.9 | 11.7). Up to four a
+// CU: 512 lanes (69 blocks, 11,000 shots 9.0 | 10.7, 23,000 shots 10.9 | 14.2; 136 blocks, 11,000 shots 11.3 | 11.5, 16,000
+// shots 11.9 | 11.1, 20,000 shots 14.0 | 14.7). More: by the blocks in all (31 blocks, 65,000 shots 11.7 | 14.0, 131,000
+// shots 18.3 | 16.7; 69 blocks, 33,000 shots 14.3 | 13.9).
+static int convert_lanes_by_rows(uint64_t tiles, uint32_t blocks) {
+    if (tiles <= 256) return blocks <= 176 ? 1024 : 0;
+    if (tiles <= 1024) return blocks <= (tiles <= 512 ? 120 : 144) ? 512 : 0;
+    return tiles * blocks <= 68 * 1024 ? 512 : 0;
 }
 
 hipError_t launch_expand(ExpandDev E, hipStream_t stream) {
     const uint64_t tiles = (E.out.shots + 31) / 32;
     if (tiles == 0) return hipSuccess;
     const size_t sub = (size_t)expand_subtile_words(E.out.blocks) * 4;
-    const int rows = lanes_by_rows(tiles, std::max(E.out.blocks, E.y_blocks));
+    const int rows = expand_lanes_by_rows(tiles, std::max(E.out.blocks, E.y_blocks));
     E.out.group = subtiles(tiles, std::max(E.out.blocks, E.y_blocks), sub, std::max(E.in_stride, E.out.out_stride));
     // Records after phase 0 staged in LDS where two workgroups still fit a CU.
     size_t lds = (sub * E.out.group + 15) / 16 * 16;
@@ -799,7 +887,7 @@ hipError_t launch_m2d(M2dParams P, hipStream_t stream) {
         if (e != hipSuccess) return e;                                                                           \
         hipLaunchKernelGGL((m2d_kernel<SLOW, ROWS>), dim3((uint32_t)grid), dim3(ROWS ? ROWS : M2D_NT), lds, stream, P);         \
     }
-    const int rows = lanes_by_rows(tiles, nb);
+    const int rows = convert_lanes_by_rows(tiles, nb);
     if (rows == 1024 && P.slow) STIM_AMD_LAUNCH(true, 1024)
     else if (rows == 1024) STIM_AMD_LAUNCH(false, 1024)
     else if (rows && P.slow) STIM_AMD_LAUNCH(true, 512)
