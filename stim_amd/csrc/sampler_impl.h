@@ -964,8 +964,14 @@ struct mfs_sampler {
         }
         if (nsites >= (1ull << 30)) return;
         std::vector<uint2> sites(std::max<uint64_t>(nsites, 1), make_uint2(0, 0));
-        std::vector<uint4> direct(sites.size(), make_uint4(0, 0, 0, 0));
+        std::vector<uint4> direct;
         bool all_direct = nsites < (1ull << 27);   // 32-bit byte offsets of 16-byte entries
+        for (const SymClass &cl : plan.classes) {
+            for (uint64_t st = 0; st < cl.nsites && all_direct; st++) {
+                direct.push_back(make_uint4(0, 0, 0, 0));
+                all_direct = direct_entry(cl, st, offs, ents, direct.back());
+            }
+        }
         std::vector<uint2> orec;
         std::vector<uint32_t> oovf;
         std::vector<uint32_t> acc;
@@ -978,7 +984,6 @@ struct mfs_sampler {
             const uint32_t nout = cl.nout & 0xFFFFu;
             site_syms.resize(nout);
             for (uint64_t st = 0; st < cl.nsites; st++) {
-                if (all_direct) all_direct = direct_entry(cl, st, offs, ents, direct[site0[c] + st]);
                 uint32_t lo = D;
                 for (uint32_t code = 1; code <= nout; code++) {
                     acc.clear();
@@ -1055,19 +1060,21 @@ struct mfs_sampler {
                 if (base[4 * gi + k] != base[4 * gi]) return;
             }
         }
-        if (orec.empty()) orec.push_back(make_uint2(0, 0));
-        upload(d_orecs, orec, "outcome records");
         upload(d_orec_base, base, "outcome record site bases");
-        upload(d_orec_sites, sites, "outcome record sites");
-        upload(d_orec_ovf, oovf, "outcome record overflow lists");
         sym_direct = all_direct;
         if (sym_direct) {
+            // A hit reads its direct entry alone.
             direct_null = (uint32_t)direct.size();
             for (uint32_t l = 0; l < 64; l++) {
                 const uint32_t d = D ? 32 * l % D : 0;
                 direct.push_back(make_uint4(d | (d << 14) | (1u << 28), d | (d << 14), d | (d << 14), 0));
             }
             upload(d_direct, direct, "direct site entries");
+        } else {
+            if (orec.empty()) orec.push_back(make_uint2(0, 0));
+            upload(d_orecs, orec, "outcome records");
+            upload(d_orec_sites, sites, "outcome record sites");
+            upload(d_orec_ovf, oovf, "outcome record overflow lists");
         }
         orec_blocks = blocks.size();
         orec_records = orec.size();

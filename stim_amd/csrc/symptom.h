@@ -138,7 +138,8 @@ struct SymDevParams {
     uint32_t *err_words;
     uint64_t err_stride_words;
     const uint32_t *site_mech;
-    // Outcome records of the specialised scan kernel (null when it does not apply). A site's outcomes
+    // Outcome records of the specialised scan kernel (null when it does not apply, and where direct entries are read
+    // instead). A site's outcomes
     // (code 1..nout) have symptoms: the XOR of the basis columns each code selects, with entries that
     // cancel removed. Written relative to the site's lowest detector b, these symptoms repeat from
     // site to site (every round of a memory circuit repeats the one before, shifted), so each distinct
