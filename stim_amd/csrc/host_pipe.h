@@ -85,7 +85,7 @@ inline void pack_bytes(const uint8_t *src, uint8_t *dst, size_t n) {
     }
 }
 
-// Idle host threads of the process, lent to one pipeline's call at a time and given back when it ends; a thread without
+// Idle host threads of the process, lent to one pipeline at a time and given back when its calls end; a thread without
 // work for a second ends. Starting threads anew for each batch took about 15 us each, as much as a 1 MB transfer.
 class HostThreads {
    public:
@@ -149,7 +149,7 @@ class HostThreads {
 // The threads that copy for one pipeline during a call, and their work: up to three jobs, each a number of shares that are
 // taken one after another. The shares of an output become available a piece at a time, as the transfer's chunks arrive: one
 // thread at a time waits for the next chunk, of the older output first. The call's own thread takes part while it waits
-// for a job. A call has threads of its own, so that none waits behind another call's kernel, and an input is
+// for a job. A pipeline has threads of its own, so that no call waits behind another call's kernel, and an input is
 // copied by all of them while an output is still on its way.
 class Crew : public std::enable_shared_from_this<Crew> {
    public:
@@ -199,23 +199,24 @@ class Crew : public std::enable_shared_from_this<Crew> {
     void cancel() {
         std::unique_lock<Spin> lock(mu_);
         for (Job &job : jobs_) job.total = job.available = job.next;
+        version_++;
         for (Job &job : jobs_) {
             while (active(job)) wait(lock);
             job.error = hipSuccess;
         }
     }
 
-    // The call has ended (every job is done): the threads go as soon as they notice, and nothing waits for that.
+    // The call has ended (every job is done): its threads go unless another call of the pipeline follows within LINGER, and
+    // nothing waits for that.
     void end_call() {
-        {
-            std::lock_guard<Spin> lock(mu_);
-            in_call_ = false;
-            version_++;
-        }
-        cv_.notify_all();
+        std::lock_guard<Spin> lock(mu_);
+        in_call_ = false;
     }
 
    private:
+    // A program's calls follow each other: giving the threads back at once and borrowing them anew costs each call 15 us.
+    static constexpr std::chrono::milliseconds LINGER{2};
+
     // Held for a few instructions at a time, by up to nine threads that a chunk's arrival sets going at once: a mutex puts
     // most of them to sleep there (36 MB of rows in 1.30 instead of 1.16 ms).
     struct Spin {
@@ -284,36 +285,33 @@ class Crew : public std::enable_shared_from_this<Crew> {
         return false;
     }
 
-    // Waits until something changes: polling while some job is under way (a chunk, or another thread's share, is
-    // about to end; waking eight sleepers for each chunk costs more), asleep while there is none.
-    void wait(std::unique_lock<Spin> &lock) {
+    // Waits until something changes (true): polling while some job is under way (a chunk, or another thread's share, is
+    // about to end; waking eight sleepers for each chunk costs more), and asleep, for LINGER at most, while there is none.
+    bool wait(std::unique_lock<Spin> &lock) {
         const uint64_t seen = version_;
         bool soon = false;
         for (const Job &job : jobs_) soon = soon || active(job);
-        if (!soon) {
-            cv_.wait(lock, [&] { return version_ != seen; });
-            return;
-        }
+        if (!soon) return cv_.wait_for(lock, LINGER, [&] { return version_ != seen; });
         lock.unlock();
         for (int polls = 0; version_ == seen; polls++) {
             if (polls < 1000) std::this_thread::yield();
             else std::this_thread::sleep_for(std::chrono::microseconds(20));   // a long kernel
         }
         lock.lock();
+        return true;
     }
 
     void serve() {
         std::unique_lock<Spin> lock(mu_);
-        while (in_call_) {
-            if (!step(lock, -1)) wait(lock);
-        }
+        while (step(lock, -1) || wait(lock) || in_call_) {}
         members_--;
     }
 
-    Spin mu_;
-    std::condition_variable_any cv_;
-    std::atomic<uint64_t> version_{0};
+    // What waiting threads poll lies apart from what the others write.
+    alignas(64) std::atomic<uint64_t> version_{0};
+    alignas(64) Spin mu_;
     Job jobs_[JOBS];
+    std::condition_variable_any cv_;
     uint64_t orders_ = 0;
     int members_ = 0;
     bool in_call_ = false;
