@@ -72,7 +72,6 @@ struct DevOp {
 };
 static_assert(sizeof(DevOp) == 32, "DevOp layout");
 
-// A run of ops with no barrier inside (host bookkeeping).
 // Entries of a noise op's outcome table, at least: it is filled up with thresholds that no draw exceeds, so that the
 // kernel compares with all of them at once.
 #ifdef __HIPCC__

@@ -788,7 +788,7 @@ __device__ __forceinline__ void apply_outcomes(const SymDevParams &P, const Sink
 // their width (64 128-byte lines at 56 B per cycle), and a d=25 tile applies 1,745 hits, so the second dependent
 // load per hit that outcome blocks need (site entry, then record) costs more than the XORs into two more words:
 // 2^20 shots at d=25 take 0.547 ms with direct entries, 0.593 ms with outcome blocks (1.11e8 128-byte lines from L2
-// for 1.14e8 hits; 839 VALU instructions per wave; with its row stores the L1 is busy about nine tenths of the time).
+// for 1.14e8 hits, which is 79% of the L1s' time at that rate; 839 VALU instructions per wave, 68% of the issue slots).
 template <bool OBS, uint32_t K>
 __device__ __forceinline__ void apply_direct(const SymDevParams &P, const Sink &sink, const uint32_t *at,
                                              const uint32_t *oc, const uint32_t *shot) {
@@ -1047,7 +1047,9 @@ __device__ __forceinline__ uint32_t mech_round(const SymDevParams &P, const Sink
 // take about 145 cycles of its CU's L1 from L2 and 326 from beyond it. A range's first round takes up to 8 gaps
 // a lane; what the first 512 draws leave is mostly under 100 hits, drawn 128 at a time (two a lane, the same
 // draws in the same order) instead of another 512. 2^20 shots of the d=25 model: 0.683 ms, 1.25 ms with
-// scan_tile_waves (now 1.21). It stays for models of more runs and for launches that record errors.
+// scan_tile_waves (now 1.21). What bounds it now is VALU issue (90% of the slots, 1,426 instructions per wave); the lines
+// that its gathers fetch take about half of the L1s' time. scan_tile_waves stays for models of more runs and for launches
+// that record errors.
 template <bool OBS>
 __device__ __forceinline__ void scan_tile_mechs(const SymDevParams &P, uint32_t btile, uint32_t *lds) {
     const uint32_t S = P.shots_per_tile;
