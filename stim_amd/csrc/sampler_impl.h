@@ -1363,6 +1363,7 @@ struct mfs_sampler {
         P.orec_sites = nullptr;
         P.orec_ovf = nullptr;
         P.direct = nullptr;
+        P.by_xcd = 0;
         P.mechs = nullptr;
         P.err_words = err_words_cur;
         P.err_stride_words = err_stride_cur;
@@ -1441,6 +1442,15 @@ struct mfs_sampler {
             P.orec_ovf = d_orec_ovf.as<uint32_t>();
             P.direct = sym_direct ? d_direct.as<uint4>() : nullptr;
             P.direct_null = direct_null;
+            // A launch that writes more than the Infinity Cache holds and applies few hits is bound by its stores, whose
+            // speed then goes by how tiles lie on the chip: neighbours on one XCD (xcd_tile). Tiles in turn | by XCD at
+            // p = 1e-4, 10^6 shots: d=17 122 | 104 us, d=21 216 | 185, d=25 381 | 279, repetition d=51 58 | 55; at 2e-4 107 | 102,
+            // 233 | 185, 316 | 297, 57 | 52. With more hits either may be faster (d=21 at 3e-4 214 | 234), and below 256 MB
+            // they are alike (200,000 shots of d=17 23.5 | 23.6).
+            double hits = 0;   // of a shot
+            for (const SymClass &cl : plan.classes) hits += (double)cl.nsites * cl.p;
+            const double row = (double)(det_bytes + obs_bytes);
+            P.by_xcd = (double)n * row > 256.0 * (1 << 20) && hits < 0.0115 * row ? 1u : 0u;
         }
         return r;
     }

@@ -160,6 +160,7 @@ struct SymDevParams {
     const uint32_t *mech_ovf;
     const uint2 *mech_run_table;
     uint32_t mech_null, mech_runs;
+    uint32_t by_xcd;               // specialised scan, plain launches: neighbouring tiles on one XCD
     uint32_t direct_null;          // first of 64 null entries (no flips; their fields name words spread over a row)
 };
 // The scan that a batch job's tiles run, the one of a plain launch; a launch of the batch kernel takes jobs of one kind.

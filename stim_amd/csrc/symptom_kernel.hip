@@ -1150,7 +1150,7 @@ __global__ __launch_bounds__(NT, 5) void sym_scan_mechs_kernel(SymDevParams P) {
 template <bool OBS, bool DIRECT>
 __global__ __launch_bounds__(NT, 5) void sym_scan_fast_kernel(SymDevParams P) {
     extern __shared__ __align__(16) uint32_t lds[];
-    scan_tile_fast<OBS, DIRECT>(P, blockIdx.x, lds);
+    scan_tile_fast<OBS, DIRECT>(P, P.by_xcd ? xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x, lds);
 }
 
 // A batch job's tile, on the scan that the job's plain launch runs. A launch's jobs are all of one KIND (symptom.h): a kernel
