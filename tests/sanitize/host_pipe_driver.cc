@@ -260,8 +260,36 @@ static void errors() {
     (void)hipStreamDestroy(stream);
 }
 
+// Rows of bits that become bytes: every remainder, tight and strided rows, with a newline, in one batch and on threads.
+static void bits() {
+    HostPipe pipe;
+    hipStream_t stream;
+    (void)hipStreamCreateWithFlags(&stream, 0);
+    for (size_t n = 1; n < 80; n++) {
+        for (int form = 0; form < 4; form++) {
+            const size_t row = (n + 7) / 8, pitch = row + (form & 1), stride = n + (form < 2 ? 0 : 3);
+            const uint64_t rows = n % 13 == 5 ? (3 << 20) / n : 1 + n % 7;
+            const long newline = form == 3 ? (long)n : -1L;
+            const uint8_t base = form == 1 ? 0 : '0';
+            pipe.begin(stream, false, rows * pitch, rows * pitch);
+            size_t cap;
+            uint8_t *const dev = pipe.next_slot(&cap);
+            for (uint64_t i = 0; i < rows * pitch; i++) dev[i] = (uint8_t)((i * 2654435761u + n) >> 11);
+            std::vector<uint8_t> out(rows * stride - (stride - n) + (newline >= 0 ? 1 : 0), 0x5A);
+            pipe.submit({{dev, pitch, row, out.data(), stride, newline, n, base}}, rows);
+            pipe.finish();
+            for (uint64_t r = 0; r < rows; r++) {
+                for (size_t k = 0; k < n; k++) EXPECT(out[r * stride + k] == base + ((dev[r * pitch + k / 8] >> (k % 8)) & 1));
+                for (size_t k = n; k < stride && r * stride + k < out.size(); k++)
+                    EXPECT(out[r * stride + k] == (k == n && newline >= 0 ? '\n' : 0x5A));
+            }
+        }
+    }
+    (void)hipStreamDestroy(stream);
+}
+
 int main(int argc, char **argv) {
-    const std::map<std::string, void (*)()> all = {{"rows", rows}, {"callers", callers}, {"overlap", overlap}, {"errors", errors}};
+    const std::map<std::string, void (*)()> all = {{"rows", rows}, {"callers", callers}, {"overlap", overlap}, {"errors", errors}, {"bits", bits}};
     if (argc != 2 || !all.count(argv[1])) return 2;
     all.at(argv[1])();
     std::printf("ok\n");

@@ -1,7 +1,7 @@
 """The host pipeline (stim_amd/csrc/host_pipe.h) on streams that are host threads, under ThreadSanitizer and
 AddressSanitizer (no GPU needed): rows of calls of several batches through reused slots and pinned input buffers, a call
-that ends while another call's kernel is held, an input that is copied while the kernel before it is held, and
-errors in the middle of a call. A scenario that waits for what is held does not end, and fails by its time limit."""
+that ends while another call's kernel is held, an input that is copied while the kernel before it is held, errors
+in the middle of a call, and rows of bits that become bytes. A scenario that waits for what is held does not end, and fails by its time limit."""
 
 import os
 import subprocess
@@ -25,7 +25,7 @@ def driver(request, tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize('scenario', ['rows', 'callers', 'overlap', 'errors'])
+@pytest.mark.parametrize('scenario', ['rows', 'callers', 'overlap', 'errors', 'bits'])
 def test_host_pipeline(driver, scenario):
     r = subprocess.run([driver, scenario], capture_output=True, text=True, timeout=60,
                        env=dict(os.environ, TSAN_OPTIONS='halt_on_error=1:exitcode=25', ASAN_OPTIONS='detect_leaks=1'))
