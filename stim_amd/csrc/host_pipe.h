@@ -6,11 +6,11 @@
 // any row stride), or expand its bits to one byte per entry (a transfer of an eighth of the bytes). So the
 // host copy of a chunk runs while the next one crosses PCIe, also in a call of one batch, and while
 // batch i's rows travel, batch i + 1's kernels run into the other slot. 131,071 rows of 274 bytes (36 MB, 0.63 ms
-// at the link's 57 GB/s) into new numpy arrays, whose pages are touched for the first time here: 1.17 ms, and 1.1
-// to 1.5 ms with one transfer and then one copy of the whole batch; 20,001 rows of 1,798 entries as bytes 1.4 instead of
-// 1.8 ms. Inputs in host memory (m2d) take the same way in: 50,001 records of 181 bytes converted in 0.72 ms, where
-// a pitched copy from pageable memory took 9 us for each row, 460 ms; 600,001 of them, seven batches, in 3.9 ms (5.8 where
-// an input's helpers wait behind those of the output before it).
+// at the link's 57 GB/s) into new numpy arrays, whose pages are touched for the first time here: 1.16 ms (1.35 in processes
+// whose new arrays find no large pages), and 1.1 to 1.6 ms with one transfer and then one copy of the whole batch; 20,001 rows
+// of 1,798 entries as bytes 1.3 to 1.5 instead of 1.8 ms. Inputs in host memory (m2d) take the same way in: 50,001 records of
+// 181 bytes converted in 0.70 ms, where a pitched copy from pageable memory took 9 us for each row, 460 ms; 600,001 of them,
+// seven batches, in 3.9 ms (5.8 where an input's helpers wait behind those of the output before it).
 // Per slot, three orderings keep the buffers consistent:
 //   - the DMA of batch i waits for batch i's kernels (event `produced`, a wait on the copy stream);
 //   - batch i + 2's kernels wait for batch i's DMA out of the slot (the last event `arrived`, a wait on the
